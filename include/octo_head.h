@@ -104,7 +104,8 @@ int octo_timing_read(const char *kernel, int *launches, double *total_ms);
  * 2 GiB or more (h_rows * ldh * element bytes >= 2^31) is first gathered into the workspace (the GEMMs address
  * mapped rows with 32-bit offsets): add OCTO_WS_GATHER for those calls.
  * Backward: the size of its plan at a 2 GiB staging budget (see octo_head_bwd); a smaller workspace is accepted
- * down to the plan at a 1 MiB budget, a larger one may run fewer chunks. OCTO_WS_STEP [| OCTO_WS_NO_GRADW |
+ * down to the plan at a 1 MiB budget, a larger one may run fewer chunks. Both gradient sizes hold room for fp32
+ * partial tiles of grad_h where few rows make it worth splitting its contraction over V (it runs unsplit without). OCTO_WS_STEP [| OCTO_WS_NO_GRADW |
  * OCTO_WS_NO_GRADH]: for octo_head_step_grpo and octo_head_step_grpo_pairs (n_max = the pair rows), whose plan has
  * row passes only, each pass's [rows, V] exponentials within the 2 GiB staging budget (a larger workspace runs larger
  * passes); for fp32 operands the larger of the forward's and the backward's. */
@@ -322,7 +323,8 @@ int octo_head_step_grpo(const void *h, int64_t h_rows, int64_t ldh, int h_dtype,
  * ld_out] receives each flat token's (logprob, entropy), 0 for a token with no pair (a masked one adds its loss term
  * at logprob 0, as the objective over the expanded columns does); lse and grpo->g are per pair row
  * (grpo->g complete, also past the count: 0); grad_h [n_pairs, ld_gh] per pair row (rows of one tree position are
- * summed by the caller's scatter). g and the loss are sums of float atomics: their last bits may vary run to run.
+ * summed by the caller's scatter). g is summed in 64 bits (float atomics) and rounded once; the loss is a sum of fp32
+ * atomics: its last bits may vary run to run.
  * flags: OCTO_LSE_PAIR only (labels are per pair row). 16-bit operands; workspace as octo_head_step_grpo. */
 int octo_head_step_grpo_pairs(const void *h, int64_t h_rows, int64_t ldh, int h_dtype,
                               const void *w, int64_t ldw, int w_dtype, const float *w_scale,

@@ -70,7 +70,10 @@ __device__ __forceinline__ void bounded_tiles(const GemmShape &s, int64_t &mtile
 // XCD x's k-th tile; false past its tiles.
 __device__ __forceinline__ bool tile_at(const GemmShape &s, int x, int64_t k, int64_t mtiles, int64_t ntiles, int &mt,
                                         int &nt) {
-  return octo_tiles::tile_at(s.group_m, x, k, mtiles, ntiles, mt, nt);
+  if (!octo_tiles::tile_at(s.group_m, x, k, mtiles, ntiles, mt, nt)) return false;
+  mt = __builtin_amdgcn_readfirstlane(mt);  // the same in every lane (the divisions leave them in vector registers)
+  nt = __builtin_amdgcn_readfirstlane(nt);
+  return true;
 }
 // The one-shot grid's block -> (mt, nt): block b is XCD b % 8's (b / 8)-th tile.
 __device__ __forceinline__ bool tile_of(const GemmShape &s, int &mt, int &nt) {

@@ -434,7 +434,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     StepLayout Lmin;
     size_t least = 0;
     for (int q = kBudgetQMin; q <= kBudgetQMax && !least; ++q)
-      if (step_plan(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, staging_candidate(q), Lmin, false))
+      if (step_plan(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, staging_candidate(q), Lmin, false, false))
         least = Lmin.total;
     return octo_fail(OCTO_EWORKSPACE, "head_step_grpo: workspace %zu bytes, below the smallest plan's %zu%s",
                      ws ? ws_bytes : (size_t)0, least,
@@ -566,7 +566,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     }
     if (pm) {
       m.zero_g = 1;
-      m.g_zero = gt->g;
+      m.g_zero = (double *)(wsb + L.g64);
     }
     rc = launch_merge(m, st);
     if (rc) return rc;
@@ -588,6 +588,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
       pa.eps_hi = gt->eps_hi;
       pa.reject_upper = gt->reject_upper;
       pa.z = z;
+      pa.g64 = (double *)(wsb + L.g64);
       pa.g = gt->g;
       pa.loss = gt->loss;
       pa.out2 = pm->out_flat;
@@ -664,6 +665,11 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     o2.ldc = ld_gh;
     o2.dtype = gh_dtype;
     o2.row_scale = rowoff ? rscale : nullptr;
+    if (L.split_items) {  // few, long tiles: their K in runs (tile_order.h)
+      o2.split = (float *)(wsb + L.split);
+      o2.split_cap = (int)L.split_items;
+      o2.split_alone = !need_gw;
+    }
     // grad_W (+)= dz^T . h   (K = this pass's rows)
     const Operand A3 = plain_operand(dz, L.V_pad * esz, L.P, nullptr, 0);
     const Operand B3 = plain_operand(ht, L.P * esz, d, nullptr, 0);
@@ -686,6 +692,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
       rc = grad_w_pass(cm.dt, A3, KM_A, B3, V, d, r0, rows, p, L.passes, L.gacc_on, gacc, grad_w, gw_dtype, flags,
                        count, st, true);
     }
+    if (!rc && need_gh) rc = launch_split_sum(s2, o2, st);
     if (rc) return rc;
   }
   return OCTO_OK;
@@ -908,7 +915,7 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
     BwdLayout Lmin;
     size_t least = 0;
     for (int q = kBudgetQMin; q <= kBudgetQMax; ++q)
-      if (bwd_plan(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, staging_candidate(q), Lmin) &&
+      if (bwd_plan(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, staging_candidate(q), Lmin, false) &&
           (!least || Lmin.total < least))
         least = Lmin.total;
     return octo_fail(OCTO_EWORKSPACE, "head_bwd: workspace %zu bytes, below the smallest plan's %zu%s",
@@ -1030,10 +1037,16 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
           o.dtype = gh_dtype;
           o.accumulate = 0;
         }
+        if (L.split_items) {
+          o.split = (float *)(wsb + L.split);
+          o.split_cap = (int)L.split_items;
+          o.split_alone = 1;
+        }
         {
           TimedLaunch t("gemm_store_grad_h", st);
           rc = launch_gemm_store(cm.dt, A2, B2, s2, o, st, wk ? KM_B : KM_NONE);
         }
+        if (!rc) rc = launch_split_sum(s2, o, st);
         if (rc) return rc;
       }
       if (need_gw) {  // grad_W[v0 .. v0 + vc) (+)= dz^T . h   (K = this pass's rows)

@@ -177,11 +177,11 @@ __global__ __launch_bounds__(64 * kMergeRows) void merge_kernel(MergeArgs a) {
           }
         }
       }
-      if (a.zero_g) a.g_zero[r] = 0.f;
+      if (a.zero_g) a.g_zero[rl] = 0.0;
     }
   } else if (lane == 0 && rl < rows) {
     if (a.hit) a.hit[rl] = 0.f;
-    if (a.zero_g && a.row_off + rl < a.n_max) a.g_zero[a.row_off + rl] = 0.f;
+    if (a.zero_g) a.g_zero[rl] = 0.0;
   }
   if (!a.loss) return;  // uniform across the workgroup: no barrier below is skipped by part of it
   if (lane == 0) loss_part[wave] = lt;
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256) void pairs_grpo_kernel(PairsGrpoArgs a) {
         float gt = 0.f;
         grpo_token(lp, a.prox ? a.prox + t : nullptr, a.old ? a.old + t : nullptr, a.adv[t], a.eps_lo, a.eps_hi,
                    a.reject_upper, 1.f / a.z[0], gt, lt);
-        if (gt != 0.f) atomicAdd(a.g + p, gt);
+        if (gt != 0.f) atomicAdd(a.g64 + (p - a.r0), (double)gt);
       }
     } else if (!paired && a.first_pass) {  // columns 0; a masked token adds its loss term at logprob 0 (no row)
       a.out2[t * a.ld_out2] = 0.f;
@@ -498,9 +498,17 @@ __global__ __launch_bounds__(256) void pairs_grpo_kernel(PairsGrpoArgs a) {
   if (threadIdx.x == 0 && part[0] != 0.f) atomicAdd(a.loss, part[0]);
 }
 
+// g of the pass's pair rows from their 64-bit sums.
+__global__ __launch_bounds__(256) void pairs_g_kernel(const double *g64, float *g, int64_t rows) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < rows) g[i] = (float)g64[i];
+}
+
 int launch_pairs_grpo(const PairsGrpoArgs &a, hipStream_t st) {
-  if (a.n_flat == 0) return OCTO_OK;
-  hipLaunchKernelGGL(pairs_grpo_kernel, dim3((unsigned)cdiv(a.n_flat, 256)), dim3(256), 0, st, a);
+  if (a.n_flat > 0)
+    hipLaunchKernelGGL(pairs_grpo_kernel, dim3((unsigned)cdiv(a.n_flat, 256)), dim3(256), 0, st, a);
+  if (a.rows > 0)
+    hipLaunchKernelGGL(pairs_g_kernel, dim3((unsigned)cdiv(a.rows, 256)), dim3(256), 0, st, a.g64, a.g + a.r0, a.rows);
   OCTO_CHECK_LAUNCH("pairs_grpo");
   return OCTO_OK;
 }

@@ -567,6 +567,19 @@ __device__ __forceinline__ void store_blocked(const typename L::V (&acc)[L::NI][
       }
 }
 
+// A split-K run's partial tile (StoreArgs::split): the accumulators in their own order, 256 contiguous bytes per store.
+template <class L>
+__device__ __forceinline__ void store_split(const typename L::V (&acc)[L::NI][L::NJ], float *tile) {
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  float *b = tile + w * (L::NI * L::NJ * L::NV * 64) + lane;
+#pragma unroll
+  for (int i = 0; i < L::NI; ++i)
+#pragma unroll
+    for (int j = 0; j < L::NJ; ++j)
+#pragma unroll
+      for (int v = 0; v < L::NV; ++v) b[((i * L::NJ + j) * L::NV + v) * 64] = acc[i][j][v];
+}
+
 // acc += the blocked partials of the earlier passes (the pass that stores C).
 template <class L>
 __device__ __forceinline__ void add_blocked(typename L::V (&acc)[L::NI][L::NJ], const float *addend, int64_t ldc,
@@ -660,9 +673,10 @@ __global__ __launch_bounds__(NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 
 // rows, d 2560, V 151,936: grad_W 13.6 against 14.1 ms and grad_h 13.9 against 14.4 ms for the 4-wave form; grad_h
 // reading W K-major without SPLIT 15.0 against 14.15 ms.
 // One tile (mt, nt) of the 8-wave gradient GEMM; OT < 0: the output type is e.dtype, chosen after the mainloop.
+// part != NULL: a split-K run, s.K its length, whose sum goes to that partial tile.
 template <int DT, int OT, int KM>
 __device__ __forceinline__ void store8_tile(const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e,
-                                            int mt, int nt, int which, lds_char *smem) {
+                                            int mt, int nt, int which, lds_char *smem, float *part = nullptr) {
   const int64_t m0 = (int64_t)mt * TM, n0 = (int64_t)nt * TN;
   int64_t mvalid = s.M - m0, nvalid = s.N - n0, K_eff = s.K;
   if (s.count_on == 1) mvalid = dev_count(s.count, s.count_off + m0, mvalid);
@@ -672,6 +686,10 @@ __device__ __forceinline__ void store8_tile(const Operand &A, const Operand &B, 
   if constexpr (KM == KM_A) mainloop_ring5<DT, OpColsN<8, 128>, OpRowsN<8, 64>>(A, B, m0, n0, K_eff, smem, acc);
   else if constexpr (KM == KM_B) mainloop_ring5<DT, OpRowsN<8, 128>, OpColsN<8, 64>, true>(A, B, m0, n0, K_eff, smem, acc);
   else mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true>(A, B, m0, n0, K_eff, smem, acc);
+  if (KM != KM_A && part) {
+    store_split<Acc16N<4>>(acc, part);
+    return;
+  }
   StoreArgs eb = e;
   if (e.part_blocked && which == 1 && e.addend) {  // the blocked partials added here, C stored as usual
     add_blocked<Acc16N<4>>(acc, e.addend, e.ldc, m0, n0);
@@ -688,20 +706,56 @@ __device__ __forceinline__ void store8_tile(const Operand &A, const Operand &B, 
   }
 }
 
+// grad_h's tile, or run of a tile (StoreArgs::split), of block b: A = dz (K-contiguous), B = W K-major (KM_B) or W^T.
+template <int DT, int OT, int KM>
+__device__ __forceinline__ void gradh8_block(Operand A, Operand B, GemmShape s, const StoreArgs &e, unsigned b,
+                                             lds_char *smem) {
+  int64_t mtiles, ntiles;
+  int mt, nt;
+  bounded_tiles(s, mtiles, ntiles);
+  const int nk = (int)cdiv(s.K, (int64_t)64), tiles = (int)(mtiles * ntiles);
+  // the same in every lane, and told so: a loop count that may differ between lanes costs the mainloop its scalar loop
+  const int S = __builtin_amdgcn_readfirstlane(
+      e.split ? octo_tiles::k_splits(tiles, nk, e.split_alone != 0, e.split_cap) : 1);
+  float *part = nullptr;
+  if (S > 1) {
+    int run;
+    const bool in = octo_tiles::split_item_at((int)(b & 7), (int)(b >> 3), S, (int)mtiles, (int)ntiles, run, mt, nt);
+    if (!__builtin_amdgcn_readfirstlane(in)) return;
+    run = __builtin_amdgcn_readfirstlane(run);
+    mt = __builtin_amdgcn_readfirstlane(mt);
+    nt = __builtin_amdgcn_readfirstlane(nt);
+    part = e.split + ((int64_t)__builtin_amdgcn_readfirstlane(run * tiles + nt * (int)mtiles + mt) << 16);
+    const int k0 = 64 * __builtin_amdgcn_readfirstlane(octo_tiles::split_stage(run, S, nk));
+    const int k1 = 64 * __builtin_amdgcn_readfirstlane(octo_tiles::split_stage(run + 1, S, nk));
+    A.base += (int64_t)k0 * 2;
+    B.base += KM == KM_B ? k0 * B.ld : (int64_t)k0 * 2;
+    s.K = __builtin_amdgcn_readfirstlane(min(k1, (int)s.K) - k0);
+  } else if (!tile_at(s, (int)(b & 7), (int64_t)(b >> 3), mtiles, ntiles, mt, nt)) {
+    return;
+  }
+  store8_tile<DT, OT, KM>(A, B, s, e, mt, nt, 1, smem, part);
+}
+
 template <int DT, int OT, int KM>
 __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_store8_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
   static_assert(ring5_ok(DT), "16-bit operands");
   __shared__ __attribute__((aligned(16))) char smem_[SMEM_RING5];
   lds_char *smem = (lds_char *)smem_;
-  int mt, nt;
-  if (!tile_of(s, mt, nt)) return;
-  const int which = pass_store(e);
-  if (which == 0) return;
-  store8_tile<DT, OT, KM>(A, B, s, e, mt, nt, which, smem);
+  if constexpr (KM != KM_A) {
+    gradh8_block<DT, OT, KM>(A, B, s, e, blockIdx.x, smem);
+  } else {
+    int mt, nt;
+    if (!tile_of(s, mt, nt)) return;
+    const int which = pass_store(e);
+    if (which == 0) return;
+    store8_tile<DT, OT, KM>(A, B, s, e, mt, nt, which, smem);
+  }
 }
 
 // Both gradient GEMMs of one row pass in one launch (the fused step): blocks [0, nh) run grad_h = dz . W (nh = its
-// tile grid, a multiple of 8, so block b still runs on XCD b % 8 in either part), the rest grad_W = dz^T . h. The
+// tile grid, or that of its split-K runs, a multiple of 8, so block b still runs on XCD b % 8 in either part), the
+// rest grad_W = dz^T . h. The
 // grad_h tiles, K = V long, are dispatched first; grad_W's, K = the pass's rows, fill the CUs its grid leaves idle
 // and the rest of its last round (a pass of 6,656 rows at d 2560 has 260 grad_h tiles: alone, a second round for 4
 // of them). KMH: grad_h reads W K-major as stored (KM_B) or a staged W^T (KM_NONE); grad_W reads dz K-major.
@@ -711,13 +765,11 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
   __shared__ __attribute__((aligned(16))) char smem_[SMEM_RING5];
   lds_char *smem = (lds_char *)smem_;
   const unsigned b = blockIdx.x;
-  int64_t mtiles, ntiles;
-  int mt, nt;
   if (b < nh) {
-    bounded_tiles(sh, mtiles, ntiles);
-    if (!tile_at(sh, (int)(b & 7), (int64_t)(b >> 3), mtiles, ntiles, mt, nt)) return;
-    store8_tile<DT, -1, KMH>(Ah, Bh, sh, eh, mt, nt, 1, smem);
+    gradh8_block<DT, -1, KMH>(Ah, Bh, sh, eh, b, smem);
   } else {
+    int64_t mtiles, ntiles;
+    int mt, nt;
     const unsigned c = b - nh;
     bounded_tiles(sw, mtiles, ntiles);
     if (!tile_at(sw, (int)(c & 7), (int64_t)(c >> 3), mtiles, ntiles, mt, nt)) return;
@@ -814,6 +866,11 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
 // ---- host launchers ----------------------------------------------------------------------------
 
 static inline dim3 grid_of(const GemmShape &s) { return dim3((unsigned)tile_grid(s.mtiles, s.ntiles)); }
+// Blocks of grad_h's tiles or, where it may split, of the most runs any device count makes of them.
+static inline int64_t split_grid(const GemmShape &s, const StoreArgs &e) {
+  const int64_t tiles = tile_grid(s.mtiles, s.ntiles);
+  return e.split ? (tiles > round_up(e.split_cap, 8) ? tiles : round_up(e.split_cap, 8)) : tiles;
+}
 
 template <int DT, bool F8, bool TH>
 static int go_stats(const Operand &A, const Operand &B, const GemmShape &s, const StatsArgs &e, hipStream_t st) {
@@ -877,10 +934,11 @@ int launch_gemm_dz(int dt, bool a_fp8, bool tanh, const Operand &A, const Operan
 template <int DT, int KM>
 static int go_store(const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e, hipStream_t st) {
   if constexpr (ring5_ok(DT)) {
+    const dim3 grid((unsigned)split_grid(s, e));
     switch (e.dtype) {
-      case OCTO_BF16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_BF16, KM>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F16, KM>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F32: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F32, KM>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+      case OCTO_BF16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_BF16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+      case OCTO_F16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+      case OCTO_F32: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F32, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
       default: return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: output dtype %d", e.dtype);
     }
   } else {
@@ -898,7 +956,7 @@ static int go_store(const Operand &A, const Operand &B, const GemmShape &s, cons
 template <int DT>
 static int go_grads(const Operand &Ah, const Operand &Bh, const GemmShape &sh, const StoreArgs &eh, bool wh_kmajor,
                     const Operand &Aw, const Operand &Bw, const GemmShape &sw, const StoreArgs &ew, hipStream_t st) {
-  const int64_t nh = tile_grid(sh.mtiles, sh.ntiles), nw = tile_grid(sw.mtiles, sw.ntiles);
+  const int64_t nh = split_grid(sh, eh), nw = tile_grid(sw.mtiles, sw.ntiles);
   if (nh + nw > 0x7fffffffLL) return octo_fail(OCTO_EINVAL, "gemm_grads: %lld tiles", (long long)(nh + nw));
   const dim3 grid((unsigned)(nh + nw));
   if (wh_kmajor)
@@ -922,6 +980,7 @@ int launch_gemm_grads(int dt, const Operand &Ah, const Operand &Bh, const GemmSh
                       hipStream_t st) {
   if (!eh.C || !ew.C || !Ah.base || !Bh.base || !Aw.base || !Bw.base)
     return octo_fail(OCTO_EINVAL, "gemm_grads: null operand or output");
+  if (ew.split) return octo_fail(OCTO_EUNSUPPORTED, "gemm_grads: grad_W is not split");
   if (wh_kmajor && !kmajor_layout_ok(Bh)) return octo_fail(OCTO_EINVAL, "gemm_grads: K-major W layout");
   if (!kmajor_layout_ok(Aw)) return octo_fail(OCTO_EINVAL, "gemm_grads: K-major dz layout");
   for (int t : {eh.dtype, ew.dtype})
@@ -938,6 +997,8 @@ int launch_gemm_store(int dt, const Operand &A, const Operand &B, const GemmShap
   if (!e.C || !A.base || !B.base) return octo_fail(OCTO_EINVAL, "gemm_store: null operand or output");
   if (dt == OCTO_F32 && (e.part || e.part_blocked))
     return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: fp32 operands store no partials");
+  if (e.split && (dt == OCTO_F32 || kmajor == KM_A || e.pass_count))
+    return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: split K of this product");
   if (kmajor != KM_NONE) {
     if (!kmajor_layout_ok(kmajor == KM_A ? A : B)) return octo_fail(OCTO_EINVAL, "gemm_store: K-major operand layout");
     switch (dt) {

@@ -130,6 +130,13 @@ struct StoreArgs {
   int part_blocked = 0;
   // row_scale: C's row m takes row_scale[m] x acc (before any addend); the final store only (not the partials)
   const float *row_scale = nullptr;
+  // split K (grad_h; tile_order.h k_splits): with room for split_cap partial tiles of 256 x 256 fp32 at split, the
+  // kernels cut each tile's K into the runs k_splits gives for the tiles the device count leaves, run s of tile (mt,
+  // nt) stores its sum at split + ((s tiles + nt mtiles + mt) << 16) in the accumulator's own order, and
+  // launch_split_sum makes C of them (all of the above). One run: C is stored by the GEMM and launch_split_sum ends.
+  float *split = nullptr;
+  int split_cap = 0;
+  int split_alone = 0;  // no other tiles in the launch
 };
 
 int launch_gemm_stats(int dt, bool a_fp8, bool tanh, const Operand &A, const Operand &B, const GemmShape &s,
@@ -140,6 +147,8 @@ int launch_gemm_dz(int dt, bool a_fp8, bool tanh, const Operand &A, const Operan
 enum { KM_NONE = 0, KM_A = 1, KM_B = 2 };
 int launch_gemm_store(int dt, const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e,
                       hipStream_t st, int kmajor = KM_NONE);
+// C of a split-K product from its partial tiles (StoreArgs::split), with the shape and store its GEMM had.
+int launch_split_sum(const GemmShape &s, const StoreArgs &e, hipStream_t st);
 // grad_h (Ah = dz K-contiguous, Bh = W K-major as stored when wh_kmajor, else W^T K-contiguous) and grad_W (Aw = dz
 // K-major, Bw = h^T) of one row pass in one launch, each with its own shape and store (16-bit operands).
 int launch_gemm_grads(int dt, const Operand &Ah, const Operand &Bh, const GemmShape &sh, const StoreArgs &eh,
@@ -177,13 +186,13 @@ struct MergeArgs {
   float *g, *loss;
   // Rows row_off .. row_off + rows of the compact order (rows < 0: all n_max), part indexed from row_off. With hit
   // != NULL, hit[r - row_off] = the row's dz at its label per unit of g gmul, (1 - p_y) post'(z_y) x (fp8 row scale)
-  // (launch_hit's formula without g gmul); 0 past the count or for a label outside [0, V). zero_g: g_zero[r] = 0 for
-  // the launch's rows (rows whose g a later kernel accumulates).
+  // (launch_hit's formula without g gmul); 0 past the count or for a label outside [0, V). zero_g: g_zero[r -
+  // row_off] = 0 for the launch's rows (rows whose g a later kernel accumulates).
   int64_t row_off = 0, rows = -1;
   float c = 0.f;
   float *hit = nullptr;
   int zero_g = 0;
-  float *g_zero = nullptr;
+  double *g_zero = nullptr;
   // tdot: the rows' raw target dot products h . W_y from launch_row_offsets (compact rows), used in place of the
   // merge's own (the same computation). exs (the row-offset exponentials, StatsArgs::xoff; needs hit): a row whose
   // maximum m2 lies at most kExClamp above its offset xoff[r] gets its label entry written into exs[r - row_off][y],
@@ -278,8 +287,10 @@ int launch_dz_scale(const DzScaleArgs &a, hipStream_t st);
 
 // The GRPO tail of the fused step over prefix-tree pair rows: flat token t reads its pair row p = flat_pair[t]; for
 // the pass's rows (r0 <= p < r0 + rows, below the row count) it takes the row's (logprob, entropy) from rowout (2
-// floats per compact row) into out2[t] and, when mask[t] != 0, adds its GRPO weight to g[p] and its loss term to the
-// loss (atomics: the last bits of both sums may vary). Tokens with no pair (p < 0 or past the count) get out2 = 0
+// floats per compact row) into out2[t] and, when mask[t] != 0, adds its GRPO weight to its pair's sum and its loss term
+// to the loss (atomics: the last bits of the loss may vary). The pairs' sums are kept in 64 bits, g64[p - r0], zeroed by
+// the pass's merge, and rounded once to g[p]: in 32 bits the order of the additions showed in g's last bit, and where
+// a gradient lies near a tie of its 16-bit rounding, in the gradient. Tokens with no pair (p < 0 or past the count) get out2 = 0
 // in the first pass and, when masked, their loss term at logprob 0 (as the objective over the expanded columns).
 struct PairsGrpoArgs {
   const int64_t *flat_pair;
@@ -291,6 +302,7 @@ struct PairsGrpoArgs {
   int64_t n_tokens;
   float eps_lo, eps_hi, reject_upper;
   const float *z;
+  double *g64;
   float *g, *loss, *out2;
   int64_t ld_out2;
   int first_pass;

@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include "../../include/octo_head.h"
+#include "tile_order.h"
 
 namespace octo_plan {
 
@@ -118,18 +119,26 @@ inline FwdLayout fwd_layout(int64_t n_max, int d, int V, int w_dtype, bool gathe
 inline bool gh_reads_w(int d, int V, int w_dtype) {
   return elem_bytes(staged_dtype(w_dtype)) == 2 && V % 64 == 0 && d % 256 == 0;
 }
+// Bytes of one fp32 partial tile of a split-K grad_h (StoreArgs::split).
+constexpr size_t kSplitTile = (size_t)kTile * kTile * sizeof(float);
+// Partial tiles a pass of P rows may make, K elements long (0: no split at any row count of the pass).
+inline int64_t gradh_split(int64_t P, int d, int64_t K, bool alone) {
+  return octo_tiles::split_items(ceil_div(P, kTile), ceil_div(d, kTile), ceil_div(K, 64), alone);
+}
 struct BwdLayout {
   int64_t P, passes, Vc, chunks, V_pad;
+  int64_t split_items;
   int esz;
   bool hacc_on, gacc_on;
-  size_t wt, ht, dza, dzb, hit, wide, hacc, gacc, rows, total;
+  size_t wt, ht, dza, dzb, hit, wide, hacc, gacc, split, rows, total;
 };
 
 // The plan for a staging budget (0: unbounded, one chunk). Rows per pass start at kPassRowsMax (balanced over the
 // passes); the chunk width is the widest multiple of 256 whose staging fits the budget, and rows per pass halve
-// while not even 256 columns fit. Returns false when no plan fits (a budget below one 256 x 256 chunk).
+// while not even 256 columns fit. Returns false when no plan fits (a budget below one 256 x 256 chunk). split: with
+// room for grad_h's split-K partial tiles (16-bit operands), where a row count of the pass asks for them.
 inline bool bwd_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bool need_gw, bool gather,
-                     size_t budget, BwdLayout &L) {
+                     size_t budget, BwdLayout &L, bool split = true) {
   L.esz = elem_bytes(staged_dtype(w_dtype));
   L.V_pad = round_to(V, kTile);
   const bool dz_a = need_gh || (need_gw && L.esz == 2), dz_b = need_gw && L.esz == 4;
@@ -185,6 +194,15 @@ inline bool bwd_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, boo
   if (L.hacc_on) off += align_up((size_t)L.P * d * sizeof(float));
   L.gacc = off;  // fp32 grad_W partial sums across passes, for a 16-bit grad_W
   if (L.gacc_on) off += align_up((size_t)V * d * sizeof(float));
+  // grad_h's split-K partial tiles, part of the staging: with one chunk, where the budget has room for them (more chunks
+  // mean rows in plenty; the default budget bounds them where the staging itself is unbounded)
+  L.split = off;
+  L.split_items = split && need_gh && L.esz == 2 && L.chunks == 1 ? gradh_split(L.P, d, L.Vc, true) : 0;
+  if (L.split_items) {
+    const size_t staged = (size_t)L.P * L.Vc * L.esz + (wt ? (size_t)d * L.Vc * L.esz : 0) + (wide ? (size_t)L.Vc * d * 2 : 0);
+    if (staged + L.split_items * kSplitTile > (budget ? budget : kStagingBudget)) L.split_items = 0;
+  }
+  off += L.split_items * kSplitTile;
   L.rows = off;  // the gathered hidden rows (OCTO_WS_GATHER), last
   if (gather) off += gather_bytes(n_max, d, w_dtype == OCTO_FP8E4M3 ? OCTO_BF16 : w_dtype);
   L.total = off;
@@ -201,13 +219,16 @@ constexpr int kBudgetQMax = 160, kBudgetQMin = 80;
 
 // The plan the backward runs in ws_bytes of workspace: unbounded if it fits, else the largest candidate staging
 // budget whose plan fits. With the queried size (the plan at kStagingBudget = 2^31, a candidate) this is that plan or
-// one with fewer chunks in no more bytes. Returns false when none fits.
+// one with fewer chunks in no more bytes. At each budget the plan with room for grad_h's partial tiles first, then
+// without (a workspace short of them keeps its chunks). Returns false when none fits.
 inline bool bwd_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bool need_gw, bool gather,
                          size_t ws_bytes, BwdLayout &L) {
-  if (bwd_plan(n_max, d, V, w_dtype, need_gh, need_gw, gather, 0, L) && L.total <= ws_bytes) return true;
-  for (int q = kBudgetQMax; q >= kBudgetQMin; --q)
-    if (bwd_plan(n_max, d, V, w_dtype, need_gh, need_gw, gather, staging_candidate(q), L) && L.total <= ws_bytes)
-      return true;
+  for (int q = kBudgetQMax + 1; q >= kBudgetQMin; --q) {
+    const size_t budget = q > kBudgetQMax ? 0 : staging_candidate(q);
+    for (int split = 1; split >= 0; --split)
+      if (bwd_plan(n_max, d, V, w_dtype, need_gh, need_gw, gather, budget, L, split != 0) && L.total <= ws_bytes)
+        return true;
+  }
   return false;
 }
 
@@ -223,9 +244,10 @@ inline bool bwd_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh,
 // bf16 (fp8 weights) or staged as W^T (16-bit weights that grad_h cannot read K-major as stored).
 struct StepLayout {
   int64_t P, passes, mtiles, V_pad;
+  int64_t split_items;
   int esz;
   bool gacc_on, wide_on, wt_on;
-  size_t part, z, hit, rowout, xoff, tdot, xuse, scale, flags, ht, dz, wide, wt, gacc, rows, total;
+  size_t part, z, hit, rowout, g64, xoff, tdot, xuse, scale, flags, ht, dz, wide, wt, gacc, split, rows, total;
 };
 
 // Rows per pass when grad_h is asked for: each pass's grad_h is one tile per CU per round of long tiles (K = V), so
@@ -258,9 +280,9 @@ constexpr int64_t kWtRows = 16384;
 
 // False when the budget holds fewer than 256 rows, or for fp32 operands (the step then runs the forward and the
 // backward: step_fallback). opt_wt: stage W^T where it pays (kWtRows); it is staged regardless where grad_h cannot
-// read W as stored.
+// read W as stored. split: with room for grad_h's split-K partial tiles where a row count of the pass asks for them.
 inline bool step_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bool need_gw, bool gather,
-                      size_t budget, StepLayout &L, bool opt_wt = true) {
+                      size_t budget, StepLayout &L, bool opt_wt = true, bool split = true) {
   L.esz = elem_bytes(staged_dtype(w_dtype));
   if (L.esz != 2) return false;
   L.mtiles = ceil_div(V, kTile);
@@ -280,13 +302,22 @@ inline bool step_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bo
   L.wt_on = need_gh && (!gh_reads_w(d, V, w_dtype) || (opt_wt && !need_gw && n_max >= kWtRows));
   size_t off = 0;
   L.part = off;  // (m, S, U) per (row of the pass, vocabulary tile)
-  off += align_up((size_t)L.P * L.mtiles * kStat4);
+  const size_t part = align_up((size_t)L.P * L.mtiles * kStat4);
+  // grad_h's split-K partial tiles, in the same place: the pass's statistics are read for the last time before its
+  // gradient GEMMs. One pass makes room for all of them; several (61 MB, 232 tiles, at 6,400 rows and V 151,936) have
+  // their ragged last pass to split and take what there is.
+  L.split = L.part;
+  L.split_items = split && need_gh ? gradh_split(L.P, d, V, !need_gw) : 0;
+  if (L.passes > 1 && L.split_items > (int64_t)(part / kSplitTile)) L.split_items = part / kSplitTile;
+  off += part > L.split_items * kSplitTile ? part : L.split_items * kSplitTile;
   L.z = off;  // the GRPO tail's token count
   off += kAlign;
   L.hit = off;  // dz at each row's label per unit of g gmul [P] fp32
   off += align_up((size_t)L.P * sizeof(float));
   L.rowout = off;  // (logprob, entropy) per compact row [n_max, 2] fp32, for the pair-row GRPO tail
   off += align_up((size_t)n_max * 2 * sizeof(float));
+  L.g64 = off;  // the pass's pair rows' GRPO weights as they are summed [P] fp64
+  off += align_up((size_t)L.P * sizeof(double));
   // bf16 operands, the row-offset exponentials: each compact row's offset and target dot [n_max] fp32; per pass row
   // the offset in use and the dz scale [P] fp32, the flagged rows [P] int32; a flag count per pass
   L.xoff = off;
@@ -316,13 +347,15 @@ inline bool step_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bo
 }
 
 // The plan the step runs in ws_bytes: unbounded if it fits, else the largest candidate staging budget that fits; at
-// each budget the optional W^T first, then without it (a workspace short of the W^T keeps the larger passes).
+// each budget the optional W^T and grad_h's partial tiles first, then without the tiles, then without the W^T, then
+// without both (a workspace short of them keeps the larger passes).
 inline bool step_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh, bool need_gw, bool gather,
                           size_t ws_bytes, StepLayout &L) {
   for (int q = kBudgetQMax + 1; q >= kBudgetQMin; --q) {
     const size_t budget = q > kBudgetQMax ? 0 : staging_candidate(q);
-    for (int opt = 1; opt >= 0; --opt)
-      if (step_plan(n_max, d, V, w_dtype, need_gh, need_gw, gather, budget, L, opt != 0) && L.total <= ws_bytes)
+    for (int opt = 3; opt >= 0; --opt)
+      if (step_plan(n_max, d, V, w_dtype, need_gh, need_gw, gather, budget, L, (opt & 2) != 0, (opt & 1) != 0) &&
+          L.total <= ws_bytes)
         return true;
   }
   return false;

@@ -51,4 +51,70 @@ constexpr bool tile_at(int group_m, int x, int64_t k, int64_t mtiles, int64_t nt
   return true;
 }
 
+// ---- split K (grad_h) ----------------------------------------------------------------------------------------
+//
+// grad_h = dz . W contracts over the vocabulary: few tiles (rows / 256 x d / 256), each long (V / 64 stages). With fewer
+// tiles than CUs the long tiles set the time: 225 scored rows at d 2560, V 151,936 are 10 tiles of 2,374 stages, 3.0 ms
+// on 10 CUs while grad_W's 5,940 tiles of 4 stages keep the others busy for 0.3. So a tile's K is cut into S runs of
+// whole stages, each a workgroup of its own that leaves an fp32 partial tile, which a small kernel sums in run order.
+//
+// k_splits: S for `tiles` tiles of nk stages. A run keeps at least kSplitStages stages (a partial tile costs about
+// kSplitCost stages of time to write and sum: 256 KB each way at 5 TB/s over 256 CUs, against 1.25 us a stage), and
+// tiles x S stays within cap, the partial tiles the workspace holds.
+//   beside grad_W (alone = false): the short tiles fill any CU the long ones leave, so a run need only be no longer
+//     than a CU's share of both products, tiles x nk / 128 stages: S = ceil(144 / tiles), none from 112 tiles on (at
+//     120 tiles three runs per tile took 0.13 ms of 5.7 longer: their partial tiles' traffic, nothing evened out).
+//   alone: whole rounds of the 256 CUs count, r of them with S = floor(256 r / tiles) runs, each run nk / S stages and
+//     its partial tile: the cheapest of r = 1 .. 4 and of no split (120 tiles: r = 1, S = 2, half of the time; 200
+//     tiles: r = 4, S = 5, 0.83 of it; 250 tiles: none).
+// 32-bit integers: every block of a launch works these out.
+constexpr int kSplitStages = 16, kSplitCost = 21, kCus = 256;
+constexpr int kSplitItemsMax = 4 * kCus;
+constexpr int k_splits(int tiles, int nk, bool alone, int cap) {
+  if (tiles <= 0 || cap <= tiles) return 1;
+  int most = nk / kSplitStages;
+  if (most > cap / tiles) most = cap / tiles;
+  if (most < 2) return 1;
+  if (!alone) {
+    const int s = tiles >= 112 ? 1 : (144 + tiles - 1) / tiles;
+    return s < most ? s : most;
+  }
+  int best = 1, cost = ((tiles + kCus - 1) / kCus) * nk;
+  for (int r = 1; r <= 4; ++r) {
+    int s = kCus * r / tiles;
+    if (s > most) s = most;
+    if (s < 2) continue;
+    const int c = ((tiles * s + kCus - 1) / kCus) * ((nk + s - 1) / s + kSplitCost);
+    if (c < cost) {
+      cost = c;
+      best = s;
+    }
+  }
+  return best;
+}
+
+// XCD x's k-th of the S x mtiles x ntiles runs: run-major (the tiles of one run of K read the same rows of both
+// operands), M fastest within a run, cut into 8 contiguous segments; false past its segment.
+constexpr bool split_item_at(int x, int k, int S, int mtiles, int ntiles, int &s, int &mt, int &nt) {
+  const int t = mtiles * ntiles, T = S * t, L = x * T / 8 + k;
+  if (L >= (x + 1) * T / 8) return false;
+  s = L / t;
+  const int p = L - s * t;
+  nt = p / mtiles;
+  mt = p - nt * mtiles;
+  return true;
+}
+// First stage of run s of S over nk stages (run s ends where s + 1 begins).
+constexpr int split_stage(int s, int S, int nk) { return (int)((int64_t)s * nk / S); }
+
+// The most runs any row count up to mtiles M-tiles makes (0: none of them splits), over K of nk stages.
+constexpr int split_items(int64_t mtiles, int64_t ntiles, int64_t nk, bool alone) {
+  int most = 0;
+  for (int64_t m = 1; m <= mtiles && m * ntiles < kSplitItemsMax; ++m) {
+    const int t = (int)(m * ntiles), s = k_splits(t, (int)nk, alone, kSplitItemsMax);
+    if (s > 1 && t * s > most) most = t * s;
+  }
+  return most;
+}
+
 }  // namespace octo_tiles

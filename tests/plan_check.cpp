@@ -57,10 +57,11 @@ static void check_step(const StepLayout &L, int64_t n_max, int d, int V, int w_d
                        bool gather) {
   const size_t esz = L.esz, hesz = w_dtype == OCTO_FP8E4M3 ? 2 : elem_bytes(w_dtype);
   std::vector<Region> r = {
-      {"part", L.part, (size_t)L.P * L.mtiles * kStat4},
+      {"part", L.part, std::max((size_t)L.P * L.mtiles * kStat4, (size_t)L.split_items << 18)},  // then partial tiles
       {"z", L.z, 4},
       {"hit", L.hit, (size_t)L.P * 4},
       {"rowout", L.rowout, (size_t)n_max * 8},
+      {"g64", L.g64, (size_t)L.P * 8},
       {"xoff", L.xoff, (size_t)n_max * 4},
       {"tdot", L.tdot, (size_t)n_max * 4},
       {"xuse", L.xuse, (size_t)L.P * 4},
@@ -74,6 +75,7 @@ static void check_step(const StepLayout &L, int64_t n_max, int d, int V, int w_d
       {"rows", L.rows, gather ? (size_t)n_max * d * hesz : 0},
   };
   check_regions(r, L.total, "step", n_max, d, V);
+  CHECK(L.split == L.part && L.split_items >= 0, "step partial tiles");
   CHECK(L.P % kTile == 0 && L.P * L.passes >= n_max && (L.passes == 0 || L.P * (L.passes - 1) < n_max),
         "step passes: P %lld passes %lld n %lld", (long long)L.P, (long long)L.passes, (long long)n_max);
   CHECK(L.V_pad % kTile == 0 && L.V_pad >= V && L.V_pad - V < kTile, "step V_pad %lld V %d", (long long)L.V_pad, V);
@@ -100,6 +102,7 @@ static void check_bwd(const BwdLayout &L, int64_t n_max, int d, int V, int w_dty
       {"wide", L.wide, w_dtype == OCTO_FP8E4M3 ? (size_t)L.Vc * d * 2 : 0},
       {"hacc", L.hacc, need_gh && L.chunks > 1 ? (size_t)L.P * d * 4 : 0},
       {"gacc", L.gacc, need_gw && L.passes > 1 && esz == 2 ? (size_t)V * d * 4 : 0},
+      {"split", L.split, (size_t)L.split_items << 18},
       {"rows", L.rows, gather ? (size_t)n_max * d * hesz : 0},
   };
   check_regions(r, L.total, "bwd", n_max, d, V);
@@ -165,6 +168,34 @@ static void check_tiles(int64_t mtiles, int64_t ntiles, int group_m) {
         (long long)octo_tiles::tile_grid(mtiles, ntiles), (long long)most);
 }
 
+// grad_h's split K as its GEMM and the sum of its partial tiles work it out, for every row count of a pass of P rows:
+// the runs cover each tile's stages once and none is empty, every (run, tile) is some block's and lands in a partial
+// tile of its own inside the room the plan gave, and no tile count below the room is left out of the sum's grid.
+static void check_split(int64_t P, int d, int64_t K, bool alone, int room) {
+  using namespace octo_tiles;
+  const int nt = (int)ceil_div(d, kTile), nk = (int)ceil_div(K, 64);
+  for (int m = 1; m <= (int)ceil_div(P, kTile); ++m) {
+    const int tiles = m * nt, S = k_splits(tiles, nk, alone, room);
+    CHECK(S >= 1 && (S == 1 || (tiles * S <= room && tiles < room && nk / S >= kSplitStages)),
+          "split %d of %d tiles, %d stages, room %d", S, tiles, nk, room);
+    if (S == 1) continue;
+    for (int r = 0; r < S; ++r)
+      CHECK(split_stage(r, S, nk) < split_stage(r + 1, S, nk), "run %d of %d over %d stages", r, S, nk);
+    CHECK(split_stage(0, S, nk) == 0 && split_stage(S, S, nk) == nk, "runs over %d stages", nk);
+    std::vector<unsigned char> seen((size_t)(S * tiles), 0);
+    const int blocks = (int)round_to(room, 8);  // at least the grid: 8 XCDs of blocks / 8
+    int found = 0;
+    for (int b = 0; b < blocks; ++b) {
+      int r = -1, mt = -1, t = -1;
+      if (!split_item_at(b & 7, b >> 3, S, m, nt, r, mt, t)) continue;
+      const bool in = r >= 0 && r < S && mt >= 0 && mt < m && t >= 0 && t < nt;
+      CHECK(in, "block %d: run %d tile (%d, %d)", b, r, mt, t);
+      if (in && !seen[(size_t)(r * tiles + t * m + mt)]++) ++found;
+    }
+    CHECK(found == S * tiles, "%d of %d runs found (%d x %d tiles, S %d)", found, S * tiles, m, nt, S);
+  }
+}
+
 int main() {
   const int64_t ns[] = {0, 1, 255, 256, 257, 1000, 3000, 6400, 24576, 32768, 32769, 65536, 131072};
   const int ds[] = {8, 64, 136, 256, 2560, 4096};
@@ -212,6 +243,18 @@ int main() {
                 }
               }
             }
+          }
+        }
+  for (int64_t P : {256, 512, 1536, 3072, 6400, 8192, 32768})
+    for (int d : {64, 256, 1000, 2560, 4096})
+      for (int64_t K : {100, 1024, 2100, 32000, 151936})
+        for (int alone = 0; alone < 2; ++alone) {
+          const int room = (int)gradh_split(P, d, K, alone != 0);
+          CHECK(room >= 0 && room <= octo_tiles::kSplitItemsMax, "room %d", room);
+          if (room) {
+            check_split(P, d, K, alone != 0, room);
+            check_split(P, d, K > 5000 ? K / 3 : K, alone != 0, room);  // a last, shorter vocabulary chunk
+            check_split(P, d, K, alone != 0, room / 2);
           }
         }
   for (int64_t m = 1; m <= 40; ++m)
