@@ -230,6 +230,11 @@ int octo_rows_scatter(const void *src, int64_t ld_src, int src_dtype, const int6
 int octo_scale_add(void *y, const void *x, int dtype, int64_t n, const float *c, const int32_t *skip_x,
                    void *stream);
 
+/* y[i] = c x[i] for i < n, c = *c read on the device, the product in fp32 rounded once to dtype. y and x 16-byte
+ * aligned, apart or the same vector. No counterpart in the reference: the fused GRPO step's backward scales the
+ * gradients its forward computed by the incoming gradient of the loss. */
+int octo_scale(void *y, const void *x, int dtype, int64_t n, const float *c, void *stream);
+
 /* The bound GRPO step's fit of the incoming dL/dlogprob, on the device: a[r] = src[idx[r] * ld_src] (src[r * ld_src]
  * without idx) for r < *count (all n without count), 0 past it; c = <a, g_head> / <g_head, g_head> (0 when g_head is
  * 0); rest[r] = a[r] - c g_head[r] for r < n; and when ||rest|| <= tol ||a||, *count_rest = 0 and *skip = 1 (the

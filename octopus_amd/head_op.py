@@ -341,6 +341,35 @@ def _(rows, weight, w_scale, pair_label, pair_pos, pair_count, flat_pair, inv_T,
             _empty(weight) if need_weight else weight.new_empty(0))
 
 
+@torch.library.custom_op("octohead::scaled", mutates_args=(), device_types="cuda")
+def scaled(x: Tensor, c: Tensor) -> Tensor:
+    """c x for a one-element c on x's device, the product formed in fp32 and rounded once to x's dtype."""
+    x = x.contiguous()
+    out = torch.empty_like(x)
+    c = c.float().contiguous()
+    _lib.call("octo_scale", _p(out), _p(x), _dtype_code(x), x.numel(), _p(c), _stream(x))
+    return out
+
+
+@scaled.register_fake
+def _(x, c):
+    return torch.empty_like(x, memory_format=torch.contiguous_format)
+
+
+def _scaled_setup(ctx, inputs, output):
+    ctx.save_for_backward(*inputs)
+
+
+def _scaled_backward(ctx, gout):
+    x, c = ctx.saved_tensors
+    gx = scaled(gout, c) if ctx.needs_input_grad[0] else None
+    gc = (gout.float() * x.float()).sum().reshape(c.shape).to(c.dtype) if ctx.needs_input_grad[1] else None
+    return gx, gc
+
+
+torch.library.register_autograd("octohead::scaled", _scaled_backward, setup_context=_scaled_setup)
+
+
 def _step_setup(ctx, inputs, output):
     _out, _lse, _g, _loss, grad_rows, grad_w = output
     # Held on ctx as detached aliases, not saved: an activation-offload pack hook (saved_tensors_hooks) would otherwise
@@ -348,18 +377,21 @@ def _step_setup(ctx, inputs, output):
     ctx.grads = (grad_rows.detach(), grad_w.detach())
     ctx.need = (inputs[-2], inputs[-1])  # need_rows, need_weight: the ops' last two arguments
     ctx.n_inputs = len(inputs)
+    # an output no loss reads has no gradient to look at: no [V, d] of zeros stands in for the held gradient's
+    ctx.set_materialize_grads(False)
 
 
 def _step_backward(ctx, _gout, _glse, _gg, gloss, _ggr, _ggw):
     """The loss is the only differentiable output: its gradients were computed by the forward call, scaled here by
     the incoming gradient of the loss (1 for loss.backward())."""
     grad_rows, grad_w = ctx.grads
-    need_rows, need_weight = ctx.need
-    # the product in fp32, rounded once to the gradient's dtype (a scale such as 1/3 is not exact in bf16)
-    scale = gloss.float()
-    gr = (grad_rows.float() * scale).to(grad_rows.dtype) if need_rows and ctx.needs_input_grad[0] else None
-    gw = (grad_w.float() * scale).to(grad_w.dtype) if need_weight and ctx.needs_input_grad[1] else None
-    return (gr, gw) + (None,) * (ctx.n_inputs - 2)
+    need_rows = ctx.need[0] and ctx.needs_input_grad[0]
+    need_weight = ctx.need[1] and ctx.needs_input_grad[1]
+    # the product in fp32, rounded once to the gradient's dtype (a scale such as 1/3 is not exact in bf16), into a
+    # tensor of its own: the held one answers a second backward through a retained graph
+    scale = (lambda t: torch.zeros_like(t)) if gloss is None else (lambda t: scaled(t, gloss))  # noqa: E731
+    return (scale(grad_rows) if need_rows else None, scale(grad_w) if need_weight else None) + \
+        (None,) * (ctx.n_inputs - 2)
 
 
 torch.library.register_autograd("octohead::head_step_grpo", _step_backward, setup_context=_step_setup)
