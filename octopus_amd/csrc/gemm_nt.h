@@ -82,48 +82,12 @@ __device__ __forceinline__ bool tile_of(const GemmShape &s, int &mt, int &nt) {
   return tile_at(s, (int)(blockIdx.x & 7), (int64_t)(blockIdx.x >> 3), mtiles, ntiles, mt, nt);
 }
 
-template <int DT> struct Mfma;
-template <> struct Mfma<OCTO_F32> {
-  // a 16-byte fragment holds 4 fp32 K values: four 32x32x2 steps, lane half h supplies k = 4h + e
-  static __device__ __forceinline__ void run(const i32x4 a, const i32x4 b, f32x16 &c) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      c = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(a[e]), __int_as_float(b[e]), c, 0, 0, 0);
-  }
-};
-
 __device__ __forceinline__ const char *uniform_ptr(const char *p) {
   const uint64_t v = (uint64_t)p;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
   return (const char *)(((uint64_t)hi << 32) | lo);
 }
-
-// ---- 4-stage mainloop (fp32 operands) ----------------------------------------------------------------
-//
-// K advances 64 bytes per stage (16 fp32). Each operand's stage slice (16 KB)
-// is written straight into LDS by buffer_load_dwordx4 ... lds: a wave instruction moves 1 KB, lane i's 16 bytes
-// landing at the instruction's LDS base + 16 i, so the LDS layout is chosen by which global chunk each lane
-// fetches. DNSTAGE stages form a ring (A slice, then B slice, per stage). One bare s_barrier per stage (no
-// memory fence: the waits are explicit) separates "stage k + 1 landed in every wave" and "every wave has read
-// stage k" from the DMA that overwrites stage k's slot.
-//
-// The operand (OpRows, K-contiguous rows): a slice is 256 rows x 64 bytes. Chunk c of row r sits at
-//     physical chunk c ^ ((r >> 2) & 3), so a 16-lane pass of fragment reads (rows r0..r0+15 of one logical
-//     chunk) covers all 64 banks once. A fragment is one ds_read_b128: lane l holds row l & 31 of a 32-row
-//     block, K chunk 2 sub + (l >> 5).
-constexpr int DKB = 64;                    // K bytes per stage
-constexpr int DSLICE = 256 * DKB;          // one operand's stage slice (16 KB)
-constexpr int DSTAGE = 2 * DSLICE;         // A + B bytes per stage
-#ifndef OCTO_NSTAGE
-#define OCTO_NSTAGE 4
-#endif
-constexpr int DNSTAGE = OCTO_NSTAGE;       // ring depth
-constexpr int DIPW = 4;                    // DMA instructions per wave per operand and stage
-constexpr int DNSUB = 2;                   // 16-byte-fragment sub-steps per stage
-// LDS of one GEMM workgroup: the DMA ring.
-constexpr int SMEM_BYTES = DNSTAGE * DSTAGE;
-static_assert(SMEM_BYTES <= 160 * 1024, "LDS budget");
 
 // s_waitcnt immediates (gfx9 encoding: vmcnt[3:0] + vmcnt[5:4] at bits 15:14, expcnt 6:4, lgkmcnt 11:8)
 constexpr int waitcnt_vm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
@@ -133,151 +97,10 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, uint32_t vo
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, voff, 0, 0, 0);
 }
 
-// K-contiguous operand: instruction q of wave w fills slice rows (4 q + w) * 16 .. + 16; lane i takes row
-// + (i >> 2) and physical chunk i & 3.
-struct OpRows {
-  static constexpr int NI = DIPW;     // DMA instructions per wave and stage
-  __amdgpu_buffer_rsrc_t rs;
-  uint32_t off[DIPW], coff[DIPW];
-  int fo[DNSUB];  // fragment byte offsets in the slice (block 0)
-
-  __device__ __forceinline__ void init(const Operand &op, int64_t row0, int wsub, uint32_t /*krows*/) {
-    const int w = threadIdx.x >> 6, i = threadIdx.x & 63, lane = i;
-    const int64_t valid = dev_count(op.count, op.count_off + row0, op.rows - row0);
-#pragma unroll
-    for (int q = 0; q < DIPW; ++q) {
-      const int r = (4 * q + w) * 16 + (i >> 2);
-      coff[q] = (uint32_t)(((i & 3) ^ ((r >> 2) & 3)) << 4);
-      uint32_t rowoff;
-      if (r < valid) rowoff = op.map ? (uint32_t)(op.map[row0 + r] * op.ld) : (uint32_t)(r * op.ld);
-      else rowoff = 0x80000000u;
-      off[q] = rowoff + coff[q];
-    }
-    if (op.map) rs = make_rsrc(uniform_ptr(op.base), op.extent);
-    else rs = make_rsrc(uniform_ptr(op.base + row0 * op.ld), (uint32_t)(256 * op.ld));
-#pragma unroll
-    for (int ks = 0; ks < DNSUB; ++ks) {
-      const int c = 2 * ks + (lane >> 5);
-      fo[ks] = (wsub * 128 + (lane & 31)) * DKB + ((c ^ ((lane >> 2) & 3)) << 4);
-    }
-  }
-  // K chunks at or past kbytes (bytes per row) read zero
-  __device__ __forceinline__ void dma(int k, int q, uint32_t kbytes, lds_char *slice) const {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t kb = (uint32_t)k * DKB;
-    lds_dma16(rs, (kb + coff[q] < kbytes) ? off[q] + kb : 0x80000000u, slice + (4 * q + w) * 1024);
-  }
-  __device__ __forceinline__ i32x4 frag(const lds_char *slice, int sub, int blk) const {
-    return *(const lds_i32x4 *)(slice + fo[sub] + blk * 32 * DKB);
-  }
-};
-
 // Instruction order is fixed in the source: a scheduling fence after every MFMA / load keeps the fragment
 // reads of the next sub-step early (so register allocation cannot fold them onto fragments still in use)
 // and spreads the DMA issues evenly between MFMAs.
 #define OCTO_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-// smem: DNSTAGE * DSTAGE bytes; stage s at s * DSTAGE, A slice first then B slice. `krows` bounds the K-rows
-// of MN-contiguous operands.
-//
-// Stage j's A slice is issued right after the barrier that frees its slot (in iteration j - DNSTAGE), its B slice
-// under the first sub-step of the next iteration (into the slot stage j - DNSTAGE left), so the DMA instructions
-// of a stage are spread over two sub-steps.
-template <int DT, typename OA, typename OB>
-__device__ __forceinline__ void mainloop_dma(const Operand &A, const Operand &B, int64_t m0, int64_t n0, int64_t K_eff,
-                                             lds_char *smem, f32x16 (&acc)[4][4]) {
-  static_assert(DNSTAGE >= 3, "ring depth");
-  constexpr int NA = OA::NI, NB = OB::NI, NPS = NA + NB;  // DMA instructions per wave and stage
-  constexpr int SPA = 8 / NA, SPB = 8 / NB;                // MFMAs between two DMA issues
-  static_assert(NPS * DNSTAGE <= 63, "vmcnt range");
-  const int w = threadIdx.x >> 6;
-  const int wm = w >> 1, wn = w & 1;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-  constexpr int ebytes = (DT == OCTO_F32) ? 4 : 2;
-  const uint32_t kbytes = (uint32_t)(K_eff * ebytes);
-  const int nk = (int)((kbytes + DKB - 1) / DKB);
-  if (nk == 0) return;
-
-  OA opa;
-  OB opb;
-  opa.init(A, m0, wm, (uint32_t)K_eff);
-  opb.init(B, n0, wn, (uint32_t)K_eff);
-
-#pragma unroll
-  for (int st = 0; st < DNSTAGE; ++st) {
-#pragma unroll
-    for (int q = 0; q < NA; ++q) opa.dma(st, q, kbytes, smem + st * DSTAGE);
-    if (st < DNSTAGE - 1) {
-#pragma unroll
-      for (int q = 0; q < NB; ++q) opb.dma(st, q, kbytes, smem + st * DSTAGE + DSLICE);
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(NPS * (DNSTAGE - 2) + NA));  // stage 0 landed
-  __builtin_amdgcn_s_barrier();
-
-  i32x4 fa[2][4], fb[2][4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    fa[0][b] = opa.frag(smem, 0, b);
-    fb[0][b] = opb.frag(smem + DSLICE, 0, b);
-  }
-  int slot = 0;                 // k % DNSTAGE
-  int prev_slot = DNSTAGE - 1;  // (k - 1) % DNSTAGE
-  for (int k = 0; k < nk; ++k) {
-    const int next_slot = (slot + 1 == DNSTAGE) ? 0 : slot + 1;
-    const lds_char *cur = smem + slot * DSTAGE;
-    __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);  // this sub-step's fragments (read under the previous one) are in
-    OCTO_FENCE();
-    // sub-step 0: read sub-step 1's fragments under the first 8 MFMAs; the B slice of stage k + DNSTAGE - 1 (into
-    // the slot stage k - 1 left) under the last 8
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      Mfma<DT>::run(fa[0][q >> 2], fb[0][q & 3], acc[q >> 2][q & 3]);
-      OCTO_FENCE();
-      if (q < 8) {
-        if (q < 4) fa[1][q] = opa.frag(cur, 1, q);
-        else fb[1][q - 4] = opb.frag(cur + DSLICE, 1, q - 4);
-        OCTO_FENCE();
-      }
-      if (q >= 8 && (q - 8) % SPB == SPB - 1) {
-        opb.dma(k + DNSTAGE - 1, (q - 8) / SPB, kbytes, smem + prev_slot * DSTAGE + DSLICE);
-        OCTO_FENCE();
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);                           // this wave's reads of stage k are done
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(NPS * (DNSTAGE - 2)));     // stage k + 1 landed (this wave's part)
-    __builtin_amdgcn_s_barrier();                                     // ... in every wave; stage k is free
-    OCTO_FENCE();
-    // sub-step 1: read the next stage's first fragments under the first 8 MFMAs, refill stage k's slot with
-    // stage k + DNSTAGE's A slice under the last 8
-    const lds_char *nxt = smem + next_slot * DSTAGE;
-    lds_char *refill = smem + slot * DSTAGE;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      Mfma<DT>::run(fa[1][q >> 2], fb[1][q & 3], acc[q >> 2][q & 3]);
-      OCTO_FENCE();
-      if (q < 8) {
-        if (q < 4) fa[0][q] = opa.frag(nxt, 0, q);
-        else fb[0][q - 4] = opb.frag(nxt + DSLICE, 0, q - 4);
-        OCTO_FENCE();
-      }
-      if (q >= 8 && (q - 8) % SPA == SPA - 1) {
-        opa.dma(k + DNSTAGE, (q - 8) / SPA, kbytes, refill);
-        OCTO_FENCE();
-      }
-    }
-    prev_slot = slot;
-    slot = next_slot;
-  }
-  __builtin_amdgcn_s_waitcnt(waitcnt_vm(0) & WAIT_LGKM0);
-  __builtin_amdgcn_s_barrier();
-}
 
 // ---- full-line mainloop: K = 64 per stage, a 5-slot ring ------------------------------------------
 //
@@ -599,19 +422,6 @@ __device__ __forceinline__ void mainloop_ring5(const Operand &A, const Operand &
 // Row (M) and column (N), relative to the tile origin, of element v of block (i, j) of wave (wm, wn). In both
 // layouts elements 4 g .. 4 g + 3 of a block are 4 consecutive rows of one column, and the lanes holding one column
 // (the rows of a column reduction) differ in the lane bits above the column bits.
-struct Acc32 {  // 4 x 4 blocks of v_mfma_f32_32x32x*: column l & 31, rows 8 (v >> 2) + 4 (l >> 5) + (v & 3)
-  static constexpr int NI = 4, NJ = 4, NV = 16;
-  typedef f32x16 V;
-  static __device__ __forceinline__ int wm(int w) { return w >> 1; }  // 2 x 2 waves
-  static __device__ __forceinline__ int wn(int w) { return w & 1; }
-  static __device__ __forceinline__ int row(int wm, int i, int v, int lane) {
-    return wm * 128 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-  }
-  static __device__ __forceinline__ int col(int wn, int j, int lane) { return wn * 128 + j * 32 + (lane & 31); }
-  static __device__ __forceinline__ float col_max(float x) { return fmaxf(x, __shfl_xor(x, 32, 64)); }
-  static __device__ __forceinline__ float col_sum(float x) { return x + __shfl_xor(x, 32, 64); }
-  static __device__ __forceinline__ bool col_lane(int lane) { return lane < 32; }  // one lane per column
-};
 // 8 x NJ blocks of v_mfma_f32_16x16x*: column l & 15, rows 4 (l >> 4) + v; NJ = 8 for 2 x 2 waves of 128 x 128,
 // NJ = 4 for the 8-wave loop's 2 x 4 waves of 128 x 64.
 template <int NJ_>
@@ -635,8 +445,4 @@ struct Acc16N {
   }
   static __device__ __forceinline__ bool col_lane(int lane) { return lane < 16; }
 };
-// The fp32 path's layout.
-__device__ __forceinline__ int acc_row(int wm, int i, int v, int lane) { return Acc32::row(wm, i, v, lane); }
-__device__ __forceinline__ int acc_col(int wn, int j, int lane) { return Acc32::col(wn, j, lane); }
-
 }  // namespace octo

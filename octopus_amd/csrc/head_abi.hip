@@ -692,7 +692,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
       rc = grad_w_pass(cm.dt, A3, KM_A, B3, V, d, r0, rows, p, L.passes, L.gacc_on, gacc, grad_w, gw_dtype, flags,
                        count, st, true);
     }
-    if (!rc && need_gh) rc = launch_split_sum(s2, o2, st);
+    if (!rc && need_gh) rc = launch_split_sum(s2, o2, false, st);
     if (rc) return rc;
   }
   return OCTO_OK;
@@ -926,7 +926,7 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
     return octo_fail(OCTO_EUNSUPPORTED, "head_bwd: 16-bit grad_w of fp32 weights over several passes");
   hipStream_t st = (hipStream_t)stream;
   char *wsb = (char *)ws;
-  void *wt = wsb + L.wt, *ht = wsb + L.ht, *dza = wsb + L.dza, *dzb = wsb + L.dzb;
+  void *wt = wsb + L.wt, *ht = wsb + L.ht, *dza = wsb + L.dza;
   float *gacc = (float *)(wsb + L.gacc), *hacc = (float *)(wsb + L.hacc);
   const int esz = L.esz;
 
@@ -936,7 +936,7 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
     if (rc) return rc;
   }
   // grad_h reads the chunk's W rows (or their bf16 widening) K-major as stored, or else their staged W^T [d, Vc]
-  const bool wk = gh_reads_w(d, V, w_dtype);
+  const bool wk = esz == 4 || gh_reads_w(d, V, w_dtype);
 
   for (int64_t p = 0; p < L.passes; ++p) {
     const int64_t r0 = p * L.P;
@@ -944,10 +944,8 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
 
     const Operand Bh = hidden_operand(h, ldh, idx, count, r0, rows, cm, gathered, d);
     DzArgs e;
-    e.dzA = (need_gh || (need_gw && esz == 2)) ? dza : nullptr;
+    e.dzA = dza;
     e.ldA = L.Vc;
-    e.dzB = (need_gw && esz == 4) ? dzb : nullptr;
-    e.ldB = L.P;
     e.lse = lse;
     e.lse_pair = (flags & OCTO_LSE_PAIR) != 0;
     e.g = g;
@@ -1046,15 +1044,13 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
           TimedLaunch t("gemm_store_grad_h", st);
           rc = launch_gemm_store(cm.dt, A2, B2, s2, o, st, wk ? KM_B : KM_NONE);
         }
-        if (!rc) rc = launch_split_sum(s2, o, st);
+        if (!rc) rc = launch_split_sum(s2, o, esz == 4, st);
         if (rc) return rc;
       }
       if (need_gw) {  // grad_W[v0 .. v0 + vc) (+)= dz^T . h   (K = this pass's rows)
-        const int kmajor = esz == 2 ? KM_A : KM_NONE;  // dz token-major read K-major, else the fp32 chunk-major copy
-        const Operand A3 = kmajor ? plain_operand(dza, L.Vc * esz, L.P, nullptr, 0)
-                                  : plain_operand(dzb, L.P * esz, L.Vc, nullptr, 0);
+        const Operand A3 = plain_operand(dza, L.Vc * esz, L.Vc, nullptr, 0);  // dz token-major, read K-major
         const Operand B3 = plain_operand(ht, L.P * esz, d, nullptr, 0);
-        rc = grad_w_pass(cm.dt, A3, kmajor, B3, vc, d, r0, rows, p, L.passes, L.gacc_on, gacc + v0 * d,
+        rc = grad_w_pass(cm.dt, A3, KM_A, B3, vc, d, r0, rows, p, L.passes, L.gacc_on, gacc + v0 * d,
                          (char *)grad_w + v0 * d * elem_bytes(gw_dtype), gw_dtype, flags, count, st);
         if (rc) return rc;
       }

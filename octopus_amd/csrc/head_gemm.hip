@@ -3,7 +3,7 @@
 //   gemm_stats : S^T = W . H^T tile -> per (row, vocab tile) online softmax statistics (m, S, U)
 //                (forward; octopus/rl/lm_head.py:102-112 without the [rows, V] logits)
 //   gemm_dz    : the same tile recomputed -> dz = g (onehot - p) / T * post'(z) of one vocabulary chunk, written
-//                token-major [tokens, chunk columns] in the 16-bit MFMA type (fp32 inputs: also chunk-major)
+//                token-major [tokens, chunk columns] in the 16-bit MFMA type
 //                (backward recompute, lm_head.py:118-121 under checkpoint)
 //   gemm_store : plain C = A . B^T with fp32/bf16/f16 output, optionally accumulated or with an fp32 addend:
 //                grad_h = dz . W (dz read K-contiguous, W read K-major as stored), grad_W = dz^T . h (dz read
@@ -13,7 +13,7 @@
 // columns) the tokens. The 16-bit kernels run v_mfma_f32_16x16x32 on 8 waves of 128 x 64 (Acc16N<4>): a lane holds
 // 32 vocabulary rows of each of its 4 token columns, so the softmax reductions over the vocabulary are in registers
 // plus a 4-lane shuffle and one LDS exchange between the two waves of a token column.
-// fp32 operands run v_mfma_f32_32x32x2 on 4 waves (Acc32).
+// fp32 operands have kernels of their own (gemm_f32.hip).
 #include <type_traits>
 
 #include "gemm_nt.h"
@@ -169,44 +169,11 @@ __device__ __forceinline__ void stats_cols(const typename L::V (&acc)[L::NI][L::
   }
 }
 
-// fp32 forward statistics (4-stage loop, 32 x 32 MFMAs); 16-bit operands run gemm_stats8_kernel.
-template <int DT, bool A_FP8, bool TANH>
-__global__ __launch_bounds__(NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_stats_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
-  static_assert(!ring5_ok(DT) && !A_FP8, "16-bit operands run gemm_stats8_kernel");
-  __shared__ __attribute__((aligned(16))) char smem_[SMEM_BYTES];
-  lds_char *smem = (lds_char *)smem_;
-  int mt, nt;
-  if (!tile_of(s, mt, nt)) return;
-  const int64_t m0 = (int64_t)mt * TM, n0 = (int64_t)nt * TN;
-  const int64_t nvalid = min(dev_count(s.count, s.count_off + n0, s.N - n0), (int64_t)TN);  // this tile's tokens
-  if (nvalid <= 0) return;
-
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 1, wn = w & 1;
-  lds_f32x4 *red = (lds_f32x4 *)smem;
-  f32x16 acc[4][4];
-  mainloop_dma<DT, OpRows, OpRows>(A, B, m0, n0, s.K, smem, acc);
-  const int64_t ma = e.v0 + m0;  // first vocabulary row of the tile
-  pre_transform<Acc32, false, TANH>(acc, wm, lane, e.pre);
-  if (ma + TM > e.V) stats_cols<Acc32, true>(acc, ma, wm, wn, lane, e.V, e.c, red);
-  else stats_cols<Acc32, false>(acc, ma, wm, wn, lane, e.V, e.c, red);
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (t < nvalid) {
-    const f32x4 a = red[t], b = red[256 + t];
-    Stat3 sa{a[0], a[1], a[2]}, sb{b[0], b[1], b[2]};
-    Stat3 r = stat_merge(sa, sb);
-    f32x4 o;
-    o[0] = a[0]; o[1] = r.S; o[2] = r.U; o[3] = b[0];
-    e.part[(n0 + t) * e.mtiles + e.v0 / TM + mt] = o;
-  }
-}
-
 // ---- epilogue: dz recompute ------------------------------------------------------------------
 //
 // dz = g (onehot - p) / T x post'(z) of the 256 (vocab) x 256 (token) tile. 16-bit types write it token-major
 // only (dzA [token][vocab]: grad_h reads it K-contiguous, grad_W K-major), through one LDS staging tile as whole
-// 512-byte rows (dz_stage / dz_write below). fp32 is computed in place in the accumulators and stored directly in
-// both layouts (dzB [vocab][token] for grad_W's K-contiguous fp32 loop).
+// 512-byte rows (dz_stage / dz_write below).
 
 // Stream a 256 x 512-byte LDS tile (rows stored with slot swizzle `s(row)` on 8-byte slots) to global
 // rows dst + row * ld_bytes, 16 bytes per thread per row-eighth. Non-temporal stores: dz is read back only by the
@@ -226,94 +193,6 @@ __device__ __forceinline__ void lds_tile_to_global(const lds_char *tile, char *d
     i32x4 v = *(const lds_i32x4 *)(tile + row * 512 + ((2 * c16) ^ (s & ~1)) * 8);
     if (s & 1) v = __builtin_shufflevector(v, v, 2, 3, 0, 1);
     __builtin_nontemporal_store(v, (i32x4 *)(dst + row * ld_bytes + c16 * 16));
-  }
-}
-
-// dz = g (onehot - p) / T * post'(z) of every tile element, in place (fp32), zero outside V and the
-// pass's valid tokens. The one-hot test compares the label, relative to this lane's first vocab row,
-// with each register's compile-time row offset.
-template <bool A_FP8, bool TANH>
-__device__ __forceinline__ void dz_in_place(f32x16 (&acc)[4][4], const DzArgs &e, int64_t m0, int64_t n0,
-                                            int64_t nvalid, int wm, int wn, int lane) {
-  const int64_t lane_row0 = m0 + wm * 128 + 4 * (lane >> 5);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int col = acc_col(wn, j, lane);
-    const bool tok_ok = col < nvalid;
-    const int64_t r = e.row_off + n0 + col;  // compact row
-    float m2 = 0.f, l2s = 0.f, gs = 0.f;
-    int yrel = -1;
-    if (tok_ok) {
-      row_state(e.lse, e.lse_pair, r, m2, l2s);
-      gs = e.g[r] * e.gmul;
-      const int64_t y = e.labels[e.label_idx ? e.label_idx[r] : r] - lane_row0;
-      yrel = (y >= 0 && y < 256) ? (int)y : -1;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int roff = i * 32 + 8 * (v >> 2) + (v & 3);
-        const float hit = (yrel == roff) ? gs : 0.f;
-        const float x = acc[i][j][v];
-        if constexpr (TANH) {
-          const float th = ftanh(e.pre * x);
-          const float p = fexp2(__builtin_fmaf(th, e.c, -m2) - l2s);
-          acc[i][j][v] = __builtin_fmaf(-gs, p, hit) * (1.f - th * th);
-        } else {
-          const float p = fexp2(__builtin_fmaf(x, e.c, -m2) - l2s);
-          acc[i][j][v] = __builtin_fmaf(-gs, p, hit);
-        }
-      }
-  }
-  if constexpr (A_FP8) {  // d/d(raw e4m3 product) = dz * row scale
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t row = lane_row0 + i * 32 + 8 * (v >> 2) + (v & 3);
-        const float sc = row < e.V ? e.wscale[row] : 0.f;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j][v] *= sc;
-      }
-  }
-  if (m0 + TM > e.V || nvalid < TN) {  // edge tile: zero rows past V and tokens past the pass's count
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool tok_ok = acc_col(wn, j, lane) < nvalid;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const bool ok = tok_ok && (lane_row0 + i * 32 + 8 * (v >> 2) + (v & 3) < e.V);
-          acc[i][j][v] = ok ? acc[i][j][v] : 0.f;
-        }
-    }
-  }
-}
-
-// fp32 dz (fp32 inputs): direct 16-byte stores to dzA, 4-byte stores to dzB.
-__device__ __forceinline__ void dz_store_direct(const f32x16 (&acc)[4][4], const DzArgs &e, int64_t m0, int64_t n0,
-                                                int wm, int wn, int lane) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t tk = n0 + acc_col(wn, j, lane);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int g4 = 0; g4 < 4; ++g4) {
-        const int64_t row0 = m0 + acc_row(wm, i, 4 * g4, lane);
-        if (e.dzA) {
-          f32x4 pk;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) pk[u] = acc[i][j][4 * g4 + u];
-          *(f32x4 *)((float *)e.dzA + tk * e.ldA + row0) = pk;
-        }
-        if (e.dzB) {
-#pragma unroll
-          for (int u = 0; u < 4; ++u) ((float *)e.dzB)[(row0 + u) * e.ldB + tk] = acc[i][j][4 * g4 + u];
-        }
-      }
   }
 }
 
@@ -446,25 +325,6 @@ __device__ __forceinline__ void dz_write(const DzArgs &e, int64_t ma, int64_t m0
     lds_tile_to_global<NT>(tile, (char *)e.dzA + (n0 * e.ldA + m0) * 2, e.ldA * 2, [](int row) { return DzSwz<L>::at(row); });
 }
 
-// fp32 dz (4-stage loop, 32 x 32 MFMAs, both layouts stored directly); 16-bit operands run gemm_dz8_kernel.
-template <int DT, bool A_FP8, bool TANH>
-__global__ __launch_bounds__(NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_dz_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
-  static_assert(!ring5_ok(DT) && !A_FP8, "16-bit operands run gemm_dz8_kernel");
-  __shared__ __attribute__((aligned(16))) char smem_[SMEM_BYTES];
-  lds_char *smem = (lds_char *)smem_;
-  int mt, nt;
-  if (!tile_of(s, mt, nt)) return;
-  const int64_t m0 = (int64_t)mt * TM, n0 = (int64_t)nt * TN;
-  const int64_t nvalid = min(dev_count(s.count, s.count_off + n0, s.N - n0), (int64_t)TN);  // this tile's tokens
-  if (nvalid <= 0) return;
-
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 1, wn = w & 1;
-  f32x16 acc[4][4];
-  mainloop_dma<DT, OpRows, OpRows>(A, B, m0, n0, s.K, smem, acc);
-  dz_in_place<false, TANH>(acc, e, e.v0 + m0, n0, nvalid, wm, wn, lane);  // vocabulary rows from v0 + m0
-  dz_store_direct(acc, e, m0, n0, wm, wn, lane);                            // dz columns from m0
-}
-
 // ---- epilogue: plain store -------------------------------------------------------------------
 
 #ifndef OCTO_PART_ATOMIC
@@ -526,21 +386,6 @@ __device__ __forceinline__ void store_any(const typename L::V (&acc)[L::NI][L::N
     if (e.addend) store_edge<L, OT, false, true>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
     else store_edge<L, OT, false, false>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
   }
-}
-
-// True when a tile with no K to contract (a device count of 0 rows) would only add zeros to what C or the partials
-// already hold: it can end before its mainloop. A store that overwrites, or adds an addend, still runs.
-__device__ __forceinline__ bool adds_nothing(const StoreArgs &e, int which, int64_t K_eff) {
-  if (K_eff > 0) return false;
-  return which == 1 ? (e.accumulate && !e.addend) : (which == 2 && e.part_accumulate);
-}
-
-// Which store a row pass's GEMM makes (StoreArgs pass_count / part): 0 none, 1 the final C, 2 the fp32 partials.
-__device__ __forceinline__ int pass_store(const StoreArgs &e) {
-  if (!e.pass_count) return 1;
-  const int64_t c = *e.pass_count;
-  if (e.pass_r0 > 0 && c <= e.pass_r0) return 0;
-  return (e.part && c > e.pass_end) ? 2 : 1;
 }
 
 // The tile's fp32 partials in the blocked layout (StoreArgs::part_blocked): this wave's 8192 values, element v of
@@ -608,62 +453,6 @@ __device__ __forceinline__ void store_pass(const typename L::V (&acc)[L::NI][L::
     p.row_scale = nullptr;
     store_any<L, float>(acc, p, m0, n0, mvalid, nvalid);
   }
-}
-
-// The fp32 GEMMs' store: C = rs[row] x acc (+ addend) (+ C when accumulate), one loop with the run-time choices
-// inside it. Separate loops per choice (store_any) made the compiler move all 256 accumulators out of the AGPRs into
-// VGPRs ahead of the branches: 376 bytes of spills per lane, against none here. fp32 operands store no partials (their
-// sums across passes accumulate into the fp32 output), so `which` is 1 here.
-template <class L, typename OT>
-__device__ __forceinline__ void store_rt(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
-                                         int64_t n0, int64_t mvalid, int64_t nvalid) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
-  OT *C = (OT *)e.C;
-  const bool acc_c = e.accumulate != 0, add = e.addend != nullptr;
-  const bool atomic = OCTO_PART_ATOMIC && acc_c && std::is_same<OT, float>::value;
-#pragma unroll
-  for (int i = 0; i < L::NI; ++i)
-#pragma unroll
-    for (int v = 0; v < L::NV; ++v) {
-      const int rr = L::row(wm, i, v, lane);
-      if (rr >= mvalid) continue;
-      OT *crow = C + (m0 + rr) * e.ldc + n0;
-      const float *arow = add ? e.addend + (m0 + rr) * e.ld_add + n0 : nullptr;
-      const float sc = e.row_scale ? e.row_scale[m0 + rr] : 1.f;
-#pragma unroll
-      for (int j = 0; j < L::NJ; ++j) {
-        const int cc = L::col(wn, j, lane);
-        if (cc >= nvalid) continue;
-        float x = acc[i][j][v] * sc;
-        if (add) x += arow[cc];
-        if (atomic) {
-          __hip_atomic_fetch_add((float *)crow + cc, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        } else {
-          if (acc_c) x += (float)crow[cc];
-          crow[cc] = (OT)x;
-        }
-      }
-    }
-}
-
-// fp32 gradient GEMMs (4-stage loop, 32 x 32 MFMAs).
-template <int DT, int OT>
-__global__ __launch_bounds__(NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_store_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
-  static_assert(!ring5_ok(DT), "16-bit operands run gemm_store8_kernel");
-  __shared__ __attribute__((aligned(16))) char smem_[SMEM_BYTES];
-  lds_char *smem = (lds_char *)smem_;
-  int mt, nt;
-  if (!tile_of(s, mt, nt)) return;
-  const int which = pass_store(e);
-  if (which == 0) return;
-  const int64_t m0 = (int64_t)mt * TM, n0 = (int64_t)nt * TN;
-  int64_t mvalid = s.M - m0, nvalid = s.N - n0, K_eff = s.K;
-  if (s.count_on == 1) mvalid = dev_count(s.count, s.count_off + m0, mvalid);
-  if (s.count_on == 3) K_eff = round_up(dev_count(s.count, s.count_off, s.K), 64);
-  if (mvalid <= 0 || nvalid <= 0 || adds_nothing(e, which, K_eff)) return;
-  f32x16 acc[4][4];
-  mainloop_dma<DT, OpRows, OpRows>(A, B, m0, n0, K_eff, smem, acc);
-  store_rt<Acc32, typename Elem<OT>::T>(acc, e, m0, n0, mvalid, nvalid);
 }
 
 // The 16-bit gradient GEMMs' 8-wave form: 512 threads, two waves per SIMD, each 128 x 64 of the tile; the second
@@ -874,20 +663,15 @@ static inline int64_t split_grid(const GemmShape &s, const StoreArgs &e) {
 
 template <int DT, bool F8, bool TH>
 static int go_stats(const Operand &A, const Operand &B, const GemmShape &s, const StatsArgs &e, hipStream_t st) {
-  if constexpr (ring5_ok(DT)) {
-    if (e.ex && e.xoff) {
-      if constexpr (DT == OCTO_BF16)
-        hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 2>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
-      else
-        return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: row-offset exponentials need bf16 operands");
-    } else if (e.ex) {
-      hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 1>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
-    } else {
-      hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 0>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
-    }
+  if (e.ex && e.xoff) {
+    if constexpr (DT == OCTO_BF16)
+      hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 2>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
+    else
+      return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: row-offset exponentials need bf16 operands");
+  } else if (e.ex) {
+    hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 1>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
   } else {
-    if (e.ex) return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: exponentials of fp32 operands");
-    hipLaunchKernelGGL((gemm_stats_kernel<DT, F8, TH>), grid_of(s), dim3(NTHREADS), 0, st, A, B, s, e);
+    hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 0>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
   }
   OCTO_CHECK_LAUNCH("gemm_stats");
   return OCTO_OK;
@@ -895,10 +679,7 @@ static int go_stats(const Operand &A, const Operand &B, const GemmShape &s, cons
 
 template <int DT, bool F8, bool TH>
 static int go_dz(const Operand &A, const Operand &B, const GemmShape &s, const DzArgs &e, hipStream_t st) {
-  if constexpr (ring5_ok(DT))
-    hipLaunchKernelGGL((gemm_dz8_kernel<DT, F8, TH>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
-  else
-    hipLaunchKernelGGL((gemm_dz_kernel<DT, F8, TH>), grid_of(s), dim3(NTHREADS), 0, st, A, B, s, e);
+  hipLaunchKernelGGL((gemm_dz8_kernel<DT, F8, TH>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
   OCTO_CHECK_LAUNCH("gemm_dz");
   return OCTO_OK;
 }
@@ -912,7 +693,7 @@ int launch_gemm_stats(int dt, bool a_fp8, bool tanh, const Operand &A, const Ope
   switch (dt) {
     case OCTO_BF16: return tanh ? go_stats<OCTO_BF16, false, true>(A, B, s, e, st) : go_stats<OCTO_BF16, false, false>(A, B, s, e, st);
     case OCTO_F16: return tanh ? go_stats<OCTO_F16, false, true>(A, B, s, e, st) : go_stats<OCTO_F16, false, false>(A, B, s, e, st);
-    case OCTO_F32: return tanh ? go_stats<OCTO_F32, false, true>(A, B, s, e, st) : go_stats<OCTO_F32, false, false>(A, B, s, e, st);
+    case OCTO_F32: return launch_gemm_stats_f32(tanh, A, B, s, e, st);
   }
   return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: dtype %d", dt);
 }
@@ -926,28 +707,19 @@ int launch_gemm_dz(int dt, bool a_fp8, bool tanh, const Operand &A, const Operan
   switch (dt) {
     case OCTO_BF16: return tanh ? go_dz<OCTO_BF16, false, true>(A, B, s, e, st) : go_dz<OCTO_BF16, false, false>(A, B, s, e, st);
     case OCTO_F16: return tanh ? go_dz<OCTO_F16, false, true>(A, B, s, e, st) : go_dz<OCTO_F16, false, false>(A, B, s, e, st);
-    case OCTO_F32: return tanh ? go_dz<OCTO_F32, false, true>(A, B, s, e, st) : go_dz<OCTO_F32, false, false>(A, B, s, e, st);
+    case OCTO_F32: return launch_gemm_dz_f32(tanh, A, B, s, e, st);
   }
   return octo_fail(OCTO_EUNSUPPORTED, "gemm_dz: dtype %d", dt);
 }
 
 template <int DT, int KM>
 static int go_store(const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e, hipStream_t st) {
-  if constexpr (ring5_ok(DT)) {
-    const dim3 grid((unsigned)split_grid(s, e));
-    switch (e.dtype) {
-      case OCTO_BF16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_BF16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F32: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F32, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
-      default: return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: output dtype %d", e.dtype);
-    }
-  } else {
-    switch (e.dtype) {
-      case OCTO_BF16: hipLaunchKernelGGL((gemm_store_kernel<DT, OCTO_BF16>), grid_of(s), dim3(NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F16: hipLaunchKernelGGL((gemm_store_kernel<DT, OCTO_F16>), grid_of(s), dim3(NTHREADS), 0, st, A, B, s, e); break;
-      case OCTO_F32: hipLaunchKernelGGL((gemm_store_kernel<DT, OCTO_F32>), grid_of(s), dim3(NTHREADS), 0, st, A, B, s, e); break;
-      default: return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: output dtype %d", e.dtype);
-    }
+  const dim3 grid((unsigned)split_grid(s, e));
+  switch (e.dtype) {
+    case OCTO_BF16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_BF16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+    case OCTO_F16: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F16, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+    case OCTO_F32: hipLaunchKernelGGL((gemm_store8_kernel<DT, OCTO_F32, KM>), grid, dim3(2 * NTHREADS), 0, st, A, B, s, e); break;
+    default: return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: output dtype %d", e.dtype);
   }
   OCTO_CHECK_LAUNCH("gemm_store");
   return OCTO_OK;
@@ -995,9 +767,8 @@ int launch_gemm_grads(int dt, const Operand &Ah, const Operand &Bh, const GemmSh
 int launch_gemm_store(int dt, const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e,
                       hipStream_t st, int kmajor) {
   if (!e.C || !A.base || !B.base) return octo_fail(OCTO_EINVAL, "gemm_store: null operand or output");
-  if (dt == OCTO_F32 && (e.part || e.part_blocked))
-    return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: fp32 operands store no partials");
-  if (e.split && (dt == OCTO_F32 || kmajor == KM_A || e.pass_count))
+  if (dt == OCTO_F32) return launch_gemm_store_f32(A, B, s, e, st, kmajor);
+  if (e.split && (kmajor == KM_A || e.pass_count))
     return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: split K of this product");
   if (kmajor != KM_NONE) {
     if (!kmajor_layout_ok(kmajor == KM_A ? A : B)) return octo_fail(OCTO_EINVAL, "gemm_store: K-major operand layout");
@@ -1010,7 +781,6 @@ int launch_gemm_store(int dt, const Operand &A, const Operand &B, const GemmShap
   switch (dt) {
     case OCTO_BF16: return go_store<OCTO_BF16, KM_NONE>(A, B, s, e, st);
     case OCTO_F16: return go_store<OCTO_F16, KM_NONE>(A, B, s, e, st);
-    case OCTO_F32: return go_store<OCTO_F32, KM_NONE>(A, B, s, e, st);
   }
   return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: dtype %d", dt);
 }

@@ -67,10 +67,8 @@ __device__ __forceinline__ void row_state(const float *lse, int pair, int64_t r,
 // gemm_dz epilogue arguments (tokens are pass-local; compact row = row_off + token). The GEMM's first operand holds
 // the vocabulary rows v0 .. v0 + its M (a chunk of W; v0 a multiple of 256); dz columns are chunk-local.
 struct DzArgs {
-  void *dzA;  // [tokens, ldA] chunk columns contiguous, staged MFMA type, or NULL
+  void *dzA;  // [tokens, ldA] chunk columns contiguous, staged type
   int64_t ldA;
-  void *dzB;  // [chunk columns, ldB] tokens contiguous, fp32 only, or NULL
-  int64_t ldB;
   int64_t v0;
   const float *lse;
   const float *g;
@@ -132,12 +130,28 @@ struct StoreArgs {
   const float *row_scale = nullptr;
   // split K (grad_h; tile_order.h k_splits): with room for split_cap partial tiles of 256 x 256 fp32 at split, the
   // kernels cut each tile's K into the runs k_splits gives for the tiles the device count leaves, run s of tile (mt,
-  // nt) stores its sum at split + ((s tiles + nt mtiles + mt) << 16) in the accumulator's own order, and
+  // nt) stores its sum at split + ((s tiles + nt mtiles + mt) << 16) in the accumulator's own order (fp32 operands: 256
+  // x 128 tiles, << 15), and
   // launch_split_sum makes C of them (all of the above). One run: C is stored by the GEMM and launch_split_sum ends.
   float *split = nullptr;
   int split_cap = 0;
   int split_alone = 0;  // no other tiles in the launch
 };
+
+// True when a tile with no K to contract (a device count of 0 rows) would only add zeros to what C or the partials
+// already hold: it can end before its mainloop. A store that overwrites, or adds an addend, still runs.
+__device__ __forceinline__ bool adds_nothing(const StoreArgs &e, int which, int64_t K_eff) {
+  if (K_eff > 0) return false;
+  return which == 1 ? (e.accumulate && !e.addend) : (which == 2 && e.part_accumulate);
+}
+
+// Which store a row pass's GEMM makes (StoreArgs pass_count / part): 0 none, 1 the final C, 2 the fp32 partials.
+__device__ __forceinline__ int pass_store(const StoreArgs &e) {
+  if (!e.pass_count) return 1;
+  const int64_t c = *e.pass_count;
+  if (e.pass_r0 > 0 && c <= e.pass_r0) return 0;
+  return (e.part && c > e.pass_end) ? 2 : 1;
+}
 
 int launch_gemm_stats(int dt, bool a_fp8, bool tanh, const Operand &A, const Operand &B, const GemmShape &s,
                       const StatsArgs &e, hipStream_t st);
@@ -147,8 +161,17 @@ int launch_gemm_dz(int dt, bool a_fp8, bool tanh, const Operand &A, const Operan
 enum { KM_NONE = 0, KM_A = 1, KM_B = 2 };
 int launch_gemm_store(int dt, const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e,
                       hipStream_t st, int kmajor = KM_NONE);
-// C of a split-K product from its partial tiles (StoreArgs::split), with the shape and store its GEMM had.
-int launch_split_sum(const GemmShape &s, const StoreArgs &e, hipStream_t st);
+// C of a split-K product from its partial tiles (StoreArgs::split), with the shape and store its GEMM had; f32: of fp32
+// operands (256 x 128 partial tiles).
+int launch_split_sum(const GemmShape &s, const StoreArgs &e, bool f32, hipStream_t st);
+// The fp32 operands' products (gemm_f32.hip): grad_h = dz . W with W K-major as stored (KM_B), grad_W = dz^T . h with
+// dz K-major (KM_A; A.rows = dz's columns).
+int launch_gemm_stats_f32(bool tanh, const Operand &A, const Operand &B, const GemmShape &s, const StatsArgs &e,
+                          hipStream_t st);
+int launch_gemm_dz_f32(bool tanh, const Operand &A, const Operand &B, const GemmShape &s, const DzArgs &e,
+                       hipStream_t st);
+int launch_gemm_store_f32(const Operand &A, const Operand &B, const GemmShape &s, const StoreArgs &e, hipStream_t st,
+                          int kmajor);
 // grad_h (Ah = dz K-contiguous, Bh = W K-major as stored when wh_kmajor, else W^T K-contiguous) and grad_W (Aw = dz
 // K-major, Bw = h^T) of one row pass in one launch, each with its own shape and store (16-bit operands).
 int launch_gemm_grads(int dt, const Operand &Ah, const Operand &Bh, const GemmShape &sh, const StoreArgs &eh,

@@ -114,16 +114,16 @@ inline FwdLayout fwd_layout(int64_t n_max, int d, int V, int w_dtype, bool gathe
 // hidden rows transposed to h^T [d, P] for grad_W = dz^T . h, and dz token-major [P, Vc] per vocabulary chunk, which
 // grad_h reads K-contiguous and 16-bit grad_W K-major (transposing LDS reads). 16-bit grad_h = dz . W reads the
 // chunk's W rows K-major as stored when V is a multiple of 64 (the loader's K-row granule) and d of 256 (its column
-// granule); otherwise, and for fp32, the chunk's W^T [d, Vc] is staged. fp32 dz is also written chunk-major [Vc, P]
-// for the fp32 loop, which reads K-contiguous operands only.
+// granule); otherwise the chunk's W^T [d, Vc] is staged. fp32 reads both K-major whatever the sizes (gemm_f32.hip).
 inline bool gh_reads_w(int d, int V, int w_dtype) {
   return elem_bytes(staged_dtype(w_dtype)) == 2 && V % 64 == 0 && d % 256 == 0;
 }
 // Bytes of one fp32 partial tile of a split-K grad_h (StoreArgs::split).
 constexpr size_t kSplitTile = (size_t)kTile * kTile * sizeof(float);
 // Partial tiles a pass of P rows may make, K elements long (0: no split at any row count of the pass).
-inline int64_t gradh_split(int64_t P, int d, int64_t K, bool alone) {
-  return octo_tiles::split_items(ceil_div(P, kTile), ceil_div(d, kTile), ceil_div(K, 64), alone);
+// tile_n: the product's tile columns (128 for fp32 operands, whose partial tiles are half as large).
+inline int64_t gradh_split(int64_t P, int d, int64_t K, bool alone, int64_t tile_n = kTile) {
+  return octo_tiles::split_items(ceil_div(P, kTile), ceil_div(d, tile_n), ceil_div(K, 64), alone);
 }
 struct BwdLayout {
   int64_t P, passes, Vc, chunks, V_pad;
@@ -178,14 +178,18 @@ inline bool bwd_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, boo
   L.hacc_on = need_gh && L.chunks > 1;
   L.gacc_on = need_gw && L.passes > 1 && w_dtype != OCTO_F32;
   size_t off = 0;
-  L.wt = off;  // W^T [d, Vc] of the chunk (grad_h, unless it reads W K-major)
+  // W^T [d, Vc] of the chunk (grad_h, unless it reads W K-major). fp32 operands need neither this nor two copies of dz
+  // (dzb); their room is still counted, so that a workspace keeps the chunks, and the sums their order, it had with
+  // them. This one holds grad_h's partial tiles.
+  L.wt = off;
   if (wt) off += align_up((size_t)d * L.Vc * L.esz);
   L.ht = off;  // h^T [d, P] of the pass's rows (grad_W)
   if (need_gw) off += align_up((size_t)d * L.P * L.esz);
-  L.dza = off;  // dz [P, Vc], token-major (grad_h; 16-bit grad_W)
+  L.dza = off;  // dz [P, Vc], token-major
   if (dz_a) off += align_up((size_t)L.P * L.Vc * L.esz);
-  L.dzb = off;  // dz [Vc, P], chunk-major (fp32 grad_W)
+  L.dzb = off;
   if (dz_b) off += align_up((size_t)L.Vc * L.P * L.esz);
+  if (!dz_a) L.dza = L.dzb;
   L.hit = off;  // dz at each row's label [P] fp32 (16-bit dz epilogue)
   if (L.esz == 2) off += align_up((size_t)L.P * sizeof(float));
   L.wide = off;  // the chunk's fp8 weights widened to bf16 [Vc, d] (the dz recompute's and grad_h's operand)
@@ -203,6 +207,12 @@ inline bool bwd_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, boo
     if (staged + L.split_items * kSplitTile > (budget ? budget : kStagingBudget)) L.split_items = 0;
   }
   off += L.split_items * kSplitTile;
+  if (L.esz == 4 && split && need_gh) {
+    L.split = L.wt;
+    L.split_items = gradh_split(L.P, d, L.Vc, true, 128);
+    const int64_t room = (int64_t)((size_t)d * L.Vc * L.esz / (kSplitTile / 2));
+    if (L.split_items > room) L.split_items = room;
+  }
   L.rows = off;  // the gathered hidden rows (OCTO_WS_GATHER), last
   if (gather) off += gather_bytes(n_max, d, w_dtype == OCTO_FP8E4M3 ? OCTO_BF16 : w_dtype);
   L.total = off;

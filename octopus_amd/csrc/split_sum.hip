@@ -10,37 +10,38 @@
 
 namespace octo {
 
-template <typename OT>
+// NJ: 16-column blocks per wave, 4 waves across the tile (256 columns: 4; fp32 operands, 128 columns: 2).
+template <typename OT, int NJ>
 __global__ __launch_bounds__(256) void split_sum_kernel(GemmShape s, StoreArgs e) {
-  typedef Acc16N<4> L;
-  constexpr int LDT = 260;  // floats per row of the LDS tile: rows 4 banks apart
+  constexpr int NI = 8, NV = 4, TNX = 64 * NJ, WAVE = NI * NJ * NV * 64;
+  constexpr int LDT = TNX + 4;  // floats per row of the LDS tile: rows 4 banks apart
   __shared__ __attribute__((aligned(16))) float tile[16 * LDT];
   int64_t mtiles, ntiles;
   bounded_tiles(s, mtiles, ntiles);
   const int64_t tiles = mtiles * ntiles, at = blockIdx.y;
   const int S = octo_tiles::k_splits((int)tiles, (int)cdiv(s.K, (int64_t)64), e.split_alone != 0, e.split_cap);
   if (S < 2 || at >= tiles) return;
-  const int64_t nt = at / mtiles, mt = at - nt * mtiles, m0 = mt * TM, n0 = nt * TN;
+  const int64_t nt = at / mtiles, mt = at - nt * mtiles, m0 = mt * TM, n0 = nt * TNX;
   int64_t mvalid = s.M - m0;
-  const int64_t nvalid = min(s.N - n0, (int64_t)TN);
+  const int64_t nvalid = min(s.N - n0, (int64_t)TNX);
   if (s.count_on == 1) mvalid = dev_count(s.count, s.count_off + m0, mvalid);
   const int wm = blockIdx.x >> 3, i = blockIdx.x & 7, row0 = wm * 128 + i * 16;
   if (row0 >= mvalid) return;
 
   const int lane = threadIdx.x & 63, wn = threadIdx.x >> 6;
-  const float *p = e.split + (at << 16) + (wm * L::NWN + wn) * (L::NI * L::NJ * L::NV * 64) + i * (L::NJ * L::NV * 64) + lane;
-  float a[L::NJ * L::NV];
+  const float *p = e.split + at * (TM * TNX) + (wm * 4 + wn) * WAVE + i * (NJ * NV * 64) + lane;
+  float a[NJ * NV];
 #pragma unroll
-  for (int k = 0; k < L::NJ * L::NV; ++k) a[k] = 0.f;
+  for (int k = 0; k < NJ * NV; ++k) a[k] = 0.f;
 #pragma unroll 2
-  for (int run = 0; run < S; ++run, p += tiles << 16) {
+  for (int run = 0; run < S; ++run, p += tiles * (TM * TNX)) {
 #pragma unroll
-    for (int k = 0; k < L::NJ * L::NV; ++k) a[k] += p[k * 64];
+    for (int k = 0; k < NJ * NV; ++k) a[k] += p[k * 64];
   }
 #pragma unroll
-  for (int j = 0; j < L::NJ; ++j)
+  for (int j = 0; j < NJ; ++j)
 #pragma unroll
-    for (int v = 0; v < L::NV; ++v) tile[(4 * (lane >> 4) + v) * LDT + L::col(wn, j, lane)] = a[j * L::NV + v];
+    for (int v = 0; v < NV; ++v) tile[(4 * (lane >> 4) + v) * LDT + (wn * NJ + j) * 16 + (lane & 15)] = a[j * NV + v];
   __syncthreads();
 
   const int row = threadIdx.x >> 4;
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(GemmShape s, StoreArgs e
   typedef OT OT4 __attribute__((ext_vector_type(4)));
   const bool whole = (uintptr_t)e.C % sizeof(OT4) == 0 && e.ldc % 4 == 0;  // 4 values of C in one store
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < NJ; ++q) {
     const int c0 = q * 64 + (threadIdx.x & 15) * 4;
     if (c0 >= nvalid) continue;
     const f32x4 t = *(const f32x4 *)(tile + row * LDT + c0);
@@ -78,8 +79,9 @@ __global__ __launch_bounds__(256) void split_sum_kernel(GemmShape s, StoreArgs e
   }
 }
 
-int launch_split_sum(const GemmShape &s, const StoreArgs &e, hipStream_t st) {
-  if (!e.split) return OCTO_OK;
+template <int NJ>
+static int go_split_sum(GemmShape s, const StoreArgs &e, hipStream_t st) {
+  s.ntiles = (int)cdiv(s.N, (int64_t)(64 * NJ));
   // the most tiles that any device count would split (mostly they are not: the launch then ends at once)
   const int nk = (int)cdiv(s.K, (int64_t)64);
   int64_t tiles = 0;
@@ -88,13 +90,18 @@ int launch_split_sum(const GemmShape &s, const StoreArgs &e, hipStream_t st) {
   if (tiles == 0) return OCTO_OK;
   const dim3 grid(16, (unsigned)tiles);
   switch (e.dtype) {
-    case OCTO_BF16: hipLaunchKernelGGL(split_sum_kernel<__bf16>, grid, dim3(256), 0, st, s, e); break;
-    case OCTO_F16: hipLaunchKernelGGL(split_sum_kernel<_Float16>, grid, dim3(256), 0, st, s, e); break;
-    case OCTO_F32: hipLaunchKernelGGL(split_sum_kernel<float>, grid, dim3(256), 0, st, s, e); break;
+    case OCTO_BF16: hipLaunchKernelGGL((split_sum_kernel<__bf16, NJ>), grid, dim3(256), 0, st, s, e); break;
+    case OCTO_F16: hipLaunchKernelGGL((split_sum_kernel<_Float16, NJ>), grid, dim3(256), 0, st, s, e); break;
+    case OCTO_F32: hipLaunchKernelGGL((split_sum_kernel<float, NJ>), grid, dim3(256), 0, st, s, e); break;
     default: return octo_fail(OCTO_EUNSUPPORTED, "split_sum: output dtype %d", e.dtype);
   }
   OCTO_CHECK_LAUNCH("split_sum");
   return OCTO_OK;
+}
+
+int launch_split_sum(const GemmShape &s, const StoreArgs &e, bool f32, hipStream_t st) {
+  if (!e.split) return OCTO_OK;
+  return f32 ? go_split_sum<2>(s, e, st) : go_split_sum<4>(s, e, st);
 }
 
 }  // namespace octo

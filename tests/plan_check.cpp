@@ -102,10 +102,14 @@ static void check_bwd(const BwdLayout &L, int64_t n_max, int d, int V, int w_dty
       {"wide", L.wide, w_dtype == OCTO_FP8E4M3 ? (size_t)L.Vc * d * 2 : 0},
       {"hacc", L.hacc, need_gh && L.chunks > 1 ? (size_t)L.P * d * 4 : 0},
       {"gacc", L.gacc, need_gw && L.passes > 1 && esz == 2 ? (size_t)V * d * 4 : 0},
-      {"split", L.split, (size_t)L.split_items << 18},
+      {"split", L.split, esz == 2 ? (size_t)L.split_items << 18 : 0},
       {"rows", L.rows, gather ? (size_t)n_max * d * hesz : 0},
   };
   check_regions(r, L.total, "bwd", n_max, d, V);
+  if (esz == 4)  // fp32: grad_h's partial tiles in the W^T region, which its products do not use
+    CHECK(L.split_items == 0 || (L.split == L.wt && (size_t)L.split_items << 17 <= (size_t)d * L.Vc * esz),
+          "fp32 partial tiles: %lld of them, d %d Vc %lld", (long long)L.split_items, d, (long long)L.Vc);
+  if (!dz_a) CHECK(L.dza == L.dzb, "fp32 dz for grad_W alone");
   if (n_max > 0) {
     CHECK(L.P % kTile == 0 && L.P * L.passes >= n_max && L.P * (L.passes - 1) < n_max, "bwd passes");
     CHECK(L.Vc % kTile == 0 && L.Vc * L.chunks >= L.V_pad && L.Vc * (L.chunks - 1) < L.V_pad, "bwd chunks: Vc %lld",
@@ -171,9 +175,9 @@ static void check_tiles(int64_t mtiles, int64_t ntiles, int group_m) {
 // grad_h's split K as its GEMM and the sum of its partial tiles work it out, for every row count of a pass of P rows:
 // the runs cover each tile's stages once and none is empty, every (run, tile) is some block's and lands in a partial
 // tile of its own inside the room the plan gave, and no tile count below the room is left out of the sum's grid.
-static void check_split(int64_t P, int d, int64_t K, bool alone, int room) {
+static void check_split(int64_t P, int d, int64_t K, bool alone, int room, int64_t tile_n) {
   using namespace octo_tiles;
-  const int nt = (int)ceil_div(d, kTile), nk = (int)ceil_div(K, 64);
+  const int nt = (int)ceil_div(d, tile_n), nk = (int)ceil_div(K, 64);
   for (int m = 1; m <= (int)ceil_div(P, kTile); ++m) {
     const int tiles = m * nt, S = k_splits(tiles, nk, alone, room);
     CHECK(S >= 1 && (S == 1 || (tiles * S <= room && tiles < room && nk / S >= kSplitStages)),
@@ -248,15 +252,15 @@ int main() {
   for (int64_t P : {256, 512, 1536, 3072, 6400, 8192, 32768})
     for (int d : {64, 256, 1000, 2560, 4096})
       for (int64_t K : {100, 1024, 2100, 32000, 151936})
-        for (int alone = 0; alone < 2; ++alone) {
-          const int room = (int)gradh_split(P, d, K, alone != 0);
-          CHECK(room >= 0 && room <= octo_tiles::kSplitItemsMax, "room %d", room);
-          if (room) {
-            check_split(P, d, K, alone != 0, room);
-            check_split(P, d, K > 5000 ? K / 3 : K, alone != 0, room);  // a last, shorter vocabulary chunk
-            check_split(P, d, K, alone != 0, room / 2);
+        for (int alone = 0; alone < 2; ++alone)
+          for (int64_t tile_n : {128, 256}) {
+            const int room = (int)gradh_split(P, d, K, alone != 0, tile_n);
+            CHECK(room >= 0 && room <= octo_tiles::kSplitItemsMax, "room %d", room);
+            if (!room) continue;
+            check_split(P, d, K, alone != 0, room, tile_n);
+            check_split(P, d, K > 5000 ? K / 3 : K, alone != 0, room, tile_n);  // a last, shorter vocabulary chunk
+            check_split(P, d, K, alone != 0, room / 2, tile_n);
           }
-        }
   for (int64_t m = 1; m <= 40; ++m)
     for (int64_t nn = 1; nn <= 30; ++nn)
       for (int g : {1, 2, 4, 8}) check_tiles(m, nn, g);
