@@ -163,7 +163,9 @@ __device__ __forceinline__ void xmfma(const i32x4 a, const i32x4 b, f32x4 &c) {
   c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// This wave's MFMAs of one stage: the smaller products first.
+// This wave's MFMAs of one stage: the smaller products first. TR as ring5_stage's (gemm_nt.h): a lane's 4 values are 4
+// columns of a row.
+template <bool TR>
 __device__ __forceinline__ void xstage(const lds_char *A, const lds_char *B, int wm, int wn, int lane, XAcc &acc) {
   constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
   i32x4 fb[3][AccX::NJ];
@@ -185,7 +187,10 @@ __device__ __forceinline__ void xstage(const lds_char *A, const lds_char *B, int
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int j = 0; j < AccX::NJ; ++j) xmfma(fa[PA[t]][u], fb[PB[t]][j], acc[i + u][j]);
+        for (int j = 0; j < AccX::NJ; ++j) {
+          if constexpr (TR) xmfma(fb[PB[t]][j], fa[PA[t]][u], acc[i + u][j]);
+          else xmfma(fa[PA[t]][u], fb[PB[t]][j], acc[i + u][j]);
+        }
   }
 }
 
@@ -198,7 +203,7 @@ __device__ __forceinline__ void xbarrier() {
 }
 
 // acc = the tile's sums over nk stages; smem holds two stages. Ends with every wave past its last LDS read.
-template <typename LA, typename LB>
+template <bool TR, typename LA, typename LB>
 __device__ __forceinline__ void mainloop_x(LA &a, LB &b, int nk, lds_char *smem, XAcc &acc) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = w >> 2, wn = w & 3;
@@ -229,7 +234,7 @@ __device__ __forceinline__ void mainloop_x(LA &a, LB &b, int nk, lds_char *smem,
       }
     };
     if (wm == 0) refill();
-    xstage(cur, cur + 3 * XPA, wm, wn, lane, acc);
+    xstage<TR>(cur, cur + 3 * XPA, wm, wn, lane, acc);
     if (wm != 0) refill();
     xbarrier();
   }
@@ -270,7 +275,7 @@ XKERNEL gemm_stats_x_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
     XRows<XN> b;
     a.init(A, m0, s.K);
     b.init(B, n0, s.K);
-    mainloop_x(a, b, (int)cdiv(s.K, (int64_t)XK), smem, acc);
+    mainloop_x<false>(a, b, (int)cdiv(s.K, (int64_t)XK), smem, acc);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
   const int64_t ma = e.v0 + m0;                       // first vocabulary row of the tile
@@ -329,7 +334,7 @@ XKERNEL gemm_dz_x_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
     XRows<XN> b;
     a.init(A, m0, s.K);
     b.init(B, n0, s.K);
-    mainloop_x(a, b, (int)cdiv(s.K, (int64_t)XK), (lds_char *)smem_, acc);
+    mainloop_x<false>(a, b, (int)cdiv(s.K, (int64_t)XK), (lds_char *)smem_, acc);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
   const int64_t ma = e.v0 + m0;
@@ -364,35 +369,53 @@ XKERNEL gemm_dz_x_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
 }
 
 // ---- gradients --------------------------------------------------------------------------------------------------------
-// C = rs[row] x acc (+ addend) (+ C when accumulate), one loop with the run-time choices inside. An fp32 C += acc is
-// one no-return atomic per element (one tile adds to it per launch, so the sums keep launch order).
+// C = rs[row] x acc (+ addend) (+ C when accumulate), one loop with the run-time choices inside. A lane's 4 values of a
+// block are neighbours in C's row (TR). An fp32 C += acc is one no-return atomic per element (one tile adds to it per
+// launch, so the sums keep launch order).
 template <typename OT>
 __device__ __forceinline__ void store_x(const XAcc &acc, const StoreArgs &e, int64_t m0, int64_t n0, int64_t mvalid,
                                         int64_t nvalid) {
+  typedef OT OT4 __attribute__((ext_vector_type(4)));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
+  const bool aligned = (uintptr_t)e.C % sizeof(OT4) == 0 && e.ldc % 4 == 0;
 #pragma unroll
-  for (int i = 0; i < AccX::NI; ++i)
+  for (int i = 0; i < AccX::NI; ++i) {
+    const int rr = wm * 128 + i * 16 + (lane & 15);
+    if (rr >= mvalid) continue;
+    OT *crow = (OT *)e.C + (m0 + rr) * e.ldc + n0;
+    const float *arow = e.addend ? e.addend + (m0 + rr) * e.ld_add + n0 : nullptr;
+    const float sc = e.row_scale ? e.row_scale[m0 + rr] : 1.f;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int rr = AccX::row(wm, i, v, lane);
-      if (rr >= mvalid) continue;
-      OT *crow = (OT *)e.C + (m0 + rr) * e.ldc + n0;
-      const float *arow = e.addend ? e.addend + (m0 + rr) * e.ld_add + n0 : nullptr;
-      const float sc = e.row_scale ? e.row_scale[m0 + rr] : 1.f;
+    for (int j = 0; j < AccX::NJ; ++j) {
+      const int cc = wn * 32 + j * 16 + 4 * (lane >> 4);
+      f32x4 x = acc[i][j];
 #pragma unroll
-      for (int j = 0; j < AccX::NJ; ++j) {
-        const int cc = AccX::col(wn, j, lane);
-        if (cc >= nvalid) continue;
-        float x = acc[i][j][v] * sc;
-        if (arow) x += arow[cc];
-        if (e.accumulate && std::is_same<OT, float>::value) {
-          __hip_atomic_fetch_add((float *)crow + cc, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        } else {
-          if (e.accumulate) x += (float)crow[cc];
-          crow[cc] = (OT)x;
-        }
+      for (int v = 0; v < 4; ++v) {
+        x[v] *= sc;
+        if (arow) x[v] += cc + v < nvalid ? arow[cc + v] : 0.f;
+      }
+      if (e.accumulate && std::is_same<OT, float>::value) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (cc + v < nvalid)
+            __hip_atomic_fetch_add((float *)crow + cc + v, x[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        continue;
+      }
+      if (e.accumulate)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[v] += cc + v < nvalid ? (float)crow[cc + v] : 0.f;
+      if (aligned && cc + 4 <= nvalid) {
+        OT4 o;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (OT)x[v];
+        *(OT4 *)(crow + cc) = o;
+      } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (cc + v < nvalid) crow[cc + v] = (OT)x[v];
       }
     }
+  }
 }
 
 // KM_B: grad_h = dz . W, its K in runs where StoreArgs::split has room (tile_order.h; partial tiles of 256 x 128, summed
@@ -436,23 +459,21 @@ XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
     XRows<XN> b;
     a.init(A, m0, K);
     b.init(B, n0, K);
-    mainloop_x(a, b, stages, (lds_char *)smem_, acc);
+    mainloop_x<true>(a, b, stages, (lds_char *)smem_, acc);
   } else {
     XRows<XM> a;
     XCols<XN> b;
     a.init(A, m0, K);
     b.init(B, n0, K);
-    mainloop_x(a, b, stages, (lds_char *)smem_, acc);
+    mainloop_x<true>(a, b, stages, (lds_char *)smem_, acc);
   }
   if (S > 1) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    float *p = e.split + (((int64_t)run * tiles + (int64_t)nt * mtiles + mt) * (XM * XN)) + w * (XM * XN / 8) + lane;
+    f32x4 *p = (f32x4 *)(e.split + (((int64_t)run * tiles + (int64_t)nt * mtiles + mt) * (XM * XN)) + w * (XM * XN / 8)) + lane;
 #pragma unroll
     for (int i = 0; i < AccX::NI; ++i)
 #pragma unroll
-      for (int j = 0; j < AccX::NJ; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) p[((i * AccX::NJ + j) * 4 + v) * 64] = acc[i][j][v];
+      for (int j = 0; j < AccX::NJ; ++j) p[(i * AccX::NJ + j) * 64] = acc[i][j];
     return;
   }
   store_x<typename Elem<OT>::T>(acc, e, m0, n0, mvalid, nvalid);

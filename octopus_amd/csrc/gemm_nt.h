@@ -70,7 +70,7 @@ __device__ __forceinline__ void bounded_tiles(const GemmShape &s, int64_t &mtile
 // XCD x's k-th tile; false past its tiles.
 __device__ __forceinline__ bool tile_at(const GemmShape &s, int x, int64_t k, int64_t mtiles, int64_t ntiles, int &mt,
                                         int &nt) {
-  if (!octo_tiles::tile_at(s.group_m, x, k, mtiles, ntiles, mt, nt)) return false;
+  if (!octo_tiles::tile_at(s.group_m, x, (int)k, (int)mtiles, (int)ntiles, mt, nt)) return false;
   mt = __builtin_amdgcn_readfirstlane(mt);  // the same in every lane (the divisions leave them in vector registers)
   nt = __builtin_amdgcn_readfirstlane(nt);
   return true;
@@ -142,7 +142,23 @@ struct OpRowsN {
   uint32_t off[NI];
   uint32_t coff;
   int fo;  // fragment byte offset of K-step 0, block 0 (K-step 1: fo ^ 64)
-  __device__ __forceinline__ void init(const Operand &op, int64_t row0, int wsub, uint32_t /*krows*/) {
+  // The mapped rows of this lane's DMA instructions, loaded ahead of the other operand's first DMA: the wait for them
+  // then leaves that DMA in flight.
+  struct Rows {
+    int64_t row[NI];
+  };
+  static __device__ __forceinline__ Rows rows(const Operand &op, int64_t row0) {
+    Rows m;
+    const int w = threadIdx.x >> 6, i = threadIdx.x & 63;
+    const int64_t valid = dev_count(op.count, op.count_off + row0, op.rows - row0);
+#pragma unroll
+    for (int q = 0; q < NI; ++q) {
+      const int r = (NW * q + w) * 8 + (i >> 3);
+      m.row[q] = op.map && r < valid ? op.map[row0 + r] : r;
+    }
+    return m;
+  }
+  __device__ __forceinline__ void init(const Operand &op, int64_t row0, int wsub, const Rows &m) {
     const int w = threadIdx.x >> 6, i = threadIdx.x & 63, lane = i;
     const int64_t valid = dev_count(op.count, op.count_off + row0, op.rows - row0);
     // row (NW q + w) * 8 + (i >> 3): its swizzle ((row >> 1) & 7) = (4 (w & 1) + (i >> 4)) & 7 for every q
@@ -151,7 +167,7 @@ struct OpRowsN {
     for (int q = 0; q < NI; ++q) {
       const int r = (NW * q + w) * 8 + (i >> 3);
       uint32_t rowoff;
-      if (r < valid) rowoff = op.map ? (uint32_t)(op.map[row0 + r] * op.ld) : (uint32_t)(r * op.ld);
+      if (r < valid) rowoff = (uint32_t)(m.row[q] * op.ld);
       else rowoff = 0x80000000u;
       off[q] = rowoff + coff;
     }
@@ -212,7 +228,9 @@ struct OpColsN {
   uint32_t lo[2];    // lane offset (row 8 w + (i >> 5)) of the DMA instructions with q & 1 = 0, 1
   int fo, fx;        // fragment byte offset of K-step 0, read 0; segment XOR of block 0
 
-  __device__ __forceinline__ void init(const Operand &op, int64_t col0, int wsub, uint32_t /*krows*/) {
+  struct Rows {};
+  static __device__ __forceinline__ Rows rows(const Operand &, int64_t) { return Rows(); }
+  __device__ __forceinline__ void init(const Operand &op, int64_t col0, int wsub, const Rows &) {
     const int w = threadIdx.x >> 6, i = threadIdx.x & 63, c = i & 31;
     base = uniform_ptr(op.base + col0 * 2);
     ld = (uint32_t)op.ld;
@@ -276,7 +294,9 @@ template <> struct Mfma16<OCTO_F16> {
 // SPLIT: B_k only frees stage k's slots; the wait for stage k + 1 (vmcnt, then a second barrier L_k) moves to the
 // middle of K-step 1, and stage k + 1's first fragments are read after L_k. The wait then covers DMA issued half a
 // K-step longer ago, for a second barrier per stage.
-template <int DT, typename OA, typename OB, bool DMA, bool NEXT, bool XFRAG, bool SPLIT>
+// TR: the MFMAs' operands change places, so a lane's 4 values of a block are 4 columns of one row (Acc16T) instead of 4
+// rows of one column (Acc16N); each value is the same sum.
+template <int DT, typename OA, typename OB, bool DMA, bool NEXT, bool XFRAG, bool SPLIT, bool TR>
 __device__ __forceinline__ void ring5_stage(const OA &opa, const OB &opb, int kd, int sa, uint32_t kbytes,
                                             lds_char *smem, typename OA::F (&fa)[2][OA::NB],
                                             typename OB::F (&fb)[2][OB::NB], f32x4 (&acc)[OA::NB][OB::NB]) {
@@ -313,9 +333,12 @@ __device__ __forceinline__ void ring5_stage(const OA &opa, const OB &opb, int kd
         __builtin_amdgcn_s_barrier();
         OCTO_FENCE();
       }
-      const int qi = q / NBB;
-      const int qj = (OCTO_MFMA_SNAKE && (qi & 1)) ? NBB - 1 - q % NBB : q % NBB;
-      Mfma16<DT>::run(OA::op(fa[ks][qi]), OB::op(fb[ks][qj]), acc[qi][qj]);
+      // TR: the B block is the MFMA's first operand and the one that stays
+      const int qo = TR ? q / NA : q / NBB, qn = TR ? NA : NBB;  // the block that stays, and how many go by
+      const int qv = (OCTO_MFMA_SNAKE && (qo & 1)) ? qn - 1 - q % qn : q % qn;
+      const int qi = TR ? qv : qo, qj = TR ? qo : qv;
+      if constexpr (TR) Mfma16<DT>::run(OB::op(fb[ks][qj]), OA::op(fa[ks][qi]), acc[qi][qj]);
+      else Mfma16<DT>::run(OA::op(fa[ks][qi]), OB::op(fb[ks][qj]), acc[qi][qj]);
       OCTO_FENCE();
       if (ks == 0 && q < NR) {
         if (q < NA) fa[1][q] = opa.frag(cA, 1, q);
@@ -337,13 +360,18 @@ __device__ __forceinline__ void ring5_stage(const OA &opa, const OB &opb, int kd
 
 __device__ __forceinline__ int ring_slot(int s) { return s >= ENSLOT ? s - ENSLOT : s; }
 
-// The ring loop's prologue: stage 0 into slots (sa0, sa0 + 1), stage 1 (when nk > 1) into (sa0 + 2, sa0 + 3), mod 5.
+// The ring loop's prologue: stage 0 into slots (sa0, sa0 + 1), its A slice first and by itself (the B operand may still
+// wait for its row map then), stage 1 (when nk > 1) into (sa0 + 2, sa0 + 3), mod 5.
+template <typename OA>
+__device__ __forceinline__ void ring5_prologue_a(const OA &opa, int sa0, uint32_t kbytes, lds_char *smem) {
+#pragma unroll
+  for (int q = 0; q < OA::NI; ++q) opa.dma(0, q, kbytes, smem + ring_slot(sa0) * ESLICE);
+  OCTO_FENCE();
+}
 template <typename OA, typename OB>
 __device__ __forceinline__ void ring5_prologue(const OA &opa, const OB &opb, int sa0, uint32_t kbytes, int nk,
                                                lds_char *smem) {
   constexpr int NI = OA::NI;
-#pragma unroll
-  for (int q = 0; q < NI; ++q) opa.dma(0, q, kbytes, smem + ring_slot(sa0) * ESLICE);
 #pragma unroll
   for (int q = 0; q < NI; ++q) opb.dma(0, q, kbytes, smem + ring_slot(sa0 + 1) * ESLICE);
   if (nk > 1) {
@@ -358,7 +386,7 @@ __device__ __forceinline__ void ring5_prologue(const OA &opa, const OB &opb, int
 // here. Ends with every DMA landed and every wave past its last LDS read (the slots are free), and returns the slot
 // that continues the ring, (sa0 + 2 nk) mod 5. VMEM instructions issued after the prologue's (a previous tile's
 // epilogue stores) are fine: loads complete in order among themselves, so at most 2 NI outstanding means stage 0 in.
-template <int DT, typename OA, typename OB, bool SPLIT>
+template <int DT, typename OA, typename OB, bool SPLIT, bool TR>
 __device__ __forceinline__ int ring5_run(const OA &opa, const OB &opb, int sa0, uint32_t kbytes, int nk,
                                          lds_char *smem, f32x4 (&acc)[OA::NB][OB::NB]) {
   constexpr int NI = OA::NI;
@@ -382,22 +410,22 @@ __device__ __forceinline__ int ring5_run(const OA &opa, const OB &opb, int sa0, 
   int sa = sa0;  // slot of stage k's A slice: sa0 + 2 k mod 5
   int k = 0;
   for (; k + 2 < nk; ++k) {
-    ring5_stage<DT, OA, OB, true, true, true, SPLIT>(opa, opb, k + 2, sa, kbytes, smem, fa, fb, acc);
+    ring5_stage<DT, OA, OB, true, true, true, SPLIT, TR>(opa, opb, k + 2, sa, kbytes, smem, fa, fb, acc);
     sa = ring_slot(sa + 2);
   }
   if (k + 1 < nk) {
-    ring5_stage<DT, OA, OB, false, true, true, SPLIT>(opa, opb, k, sa, kbytes, smem, fa, fb, acc);
+    ring5_stage<DT, OA, OB, false, true, true, SPLIT, TR>(opa, opb, k, sa, kbytes, smem, fa, fb, acc);
     sa = ring_slot(sa + 2);
     ++k;
   }
-  ring5_stage<DT, OA, OB, false, false, false, SPLIT>(opa, opb, k, sa, kbytes, smem, fa, fb, acc);
+  ring5_stage<DT, OA, OB, false, false, false, SPLIT, TR>(opa, opb, k, sa, kbytes, smem, fa, fb, acc);
   __builtin_amdgcn_s_waitcnt(waitcnt_vm(0) & WAIT_LGKM0);
   __builtin_amdgcn_s_barrier();
   return ring_slot(sa + 2);
 }
 
 // smem: SMEM_RING5 bytes. 16-bit types only.
-template <int DT, typename OA, typename OB, bool SPLIT = false>
+template <int DT, typename OA, typename OB, bool SPLIT = false, bool TR = false>
 __device__ __forceinline__ void mainloop_ring5(const Operand &A, const Operand &B, int64_t m0, int64_t n0,
                                                int64_t K_eff, lds_char *smem, f32x4 (&acc)[OA::NB][OB::NB]) {
   static_assert(DT == OCTO_BF16 || DT == OCTO_F16, "16-bit operands");
@@ -410,11 +438,12 @@ __device__ __forceinline__ void mainloop_ring5(const Operand &A, const Operand &
   OA opa;
   OB opb;
   if (nk > 0) {
-    opa.init(A, m0, wm, (uint32_t)K_eff);
-    opb.init(B, n0, wn, (uint32_t)K_eff);
+    opa.init(A, m0, wm, OA::rows(A, m0));
+    opb.init(B, n0, wn, OB::rows(B, n0));
+    ring5_prologue_a(opa, 0, kbytes, smem);
     ring5_prologue(opa, opb, 0, kbytes, nk, smem);
   }
-  ring5_run<DT, OA, OB, SPLIT>(opa, opb, 0, kbytes, nk, smem, acc);
+  ring5_run<DT, OA, OB, SPLIT, TR>(opa, opb, 0, kbytes, nk, smem, acc);
 }
 
 // ---- accumulator layouts of a wave's 128 x 128 sub-tile --------------------------------------------
@@ -445,4 +474,15 @@ struct Acc16N {
   }
   static __device__ __forceinline__ bool col_lane(int lane) { return lane < 16; }
 };
+// The 8-wave gradient kernels' blocks, with the MFMA operands in each other's place (ring5_stage TR): row l & 15, columns
+// 4 (l >> 4) + v, so a lane's 4 values are neighbours in a row-major C.
+struct Acc16T {
+  static constexpr int NI = 8, NJ = 4, NV = 4;
+  typedef f32x4 V;
+  static __device__ __forceinline__ int wm(int w) { return w >> 2; }  // 2 x 4 waves
+  static __device__ __forceinline__ int wn(int w) { return w & 3; }
+  static __device__ __forceinline__ int row(int wm, int i, int lane) { return wm * 128 + i * 16 + (lane & 15); }
+  static __device__ __forceinline__ int col(int wn, int j, int lane) { return wn * 64 + j * 16 + 4 * (lane >> 4); }
+};
+
 }  // namespace octo

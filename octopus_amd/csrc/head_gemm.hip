@@ -327,65 +327,86 @@ __device__ __forceinline__ void dz_write(const DzArgs &e, int64_t ma, int64_t m0
 
 // ---- epilogue: plain store -------------------------------------------------------------------
 
-#ifndef OCTO_PART_ATOMIC
-#define OCTO_PART_ATOMIC 1
-#endif
-// C = rs[row] x acc (rs NULL: acc) (+ addend, fp32, row stride ld_add) (+ C when ACC), rounded once to OT. An fp32 C += acc is one no-return
-// atomic add per element, performed in the L2, so the tile's epilogue does not wait for C to be read (grad_W's fp32
-// partials of the fused step at 24,576 rows, d 2560, V 151,936: the gradient launches 28.35 against 28.65 ms per
-// step, same box). A launch adds to each element once (one tile), so the sums keep launch order and are
-// reproducible.
-template <class L, typename OT, bool ACC, bool ADD, bool EDGE>
-__device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::NJ], OT *C, const float *addend,
-                                           int64_t ldc, int64_t ld_add, int64_t m0, int64_t n0, int64_t mvalid,
-                                           int64_t nvalid, int wm, int wn, int lane, const float *rs) {
+// C = rs[row] x acc (rs NULL: acc) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to OT, value
+// by value. An fp32 C += acc is one no-return atomic add per element, performed in the L2, so the tile's epilogue does
+// not wait for C to be read (grad_W's fp32 partials of the fused step at 24,576 rows, d 2560, V 151,936: the gradient
+// launches 28.35 against 28.65 ms per step, same box). A launch adds to each element once (one tile), so the sums keep
+// launch order and are reproducible.
+template <class L, typename OT>
+__device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
+                                           int64_t n0, int64_t mvalid, int64_t nvalid) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
 #pragma unroll
-  for (int i = 0; i < L::NI; ++i)
+  for (int i = 0; i < L::NI; ++i) {
+    const int rr = L::row(wm, i, lane);
+    if (rr >= mvalid) continue;
+    OT *crow = (OT *)e.C + (m0 + rr) * e.ldc + n0;
+    const float *arow = e.addend ? e.addend + (m0 + rr) * e.ld_add + n0 : nullptr;
+    const float sc = e.row_scale ? e.row_scale[m0 + rr] : 1.f;
 #pragma unroll
-    for (int v = 0; v < L::NV; ++v) {
-      const int rr = L::row(wm, i, v, lane);
-      if (EDGE && rr >= mvalid) continue;
-      OT *crow = C + (m0 + rr) * ldc + n0;
-      const float *arow = ADD ? addend + (m0 + rr) * ld_add + n0 : nullptr;
-      const float sc = rs ? rs[m0 + rr] : 1.f;
+    for (int j = 0; j < L::NJ; ++j)
 #pragma unroll
-      for (int j = 0; j < L::NJ; ++j) {
-        const int cc = L::col(wn, j, lane);
-        if (EDGE && cc >= nvalid) continue;
+      for (int v = 0; v < L::NV; ++v) {
+        const int cc = L::col(wn, j, lane) + v;
+        if (cc >= nvalid) continue;
         float x = acc[i][j][v] * sc;
-        if (ADD) x += arow[cc];
-        if constexpr (OCTO_PART_ATOMIC && ACC && std::is_same<OT, float>::value) {
-          __hip_atomic_fetch_add(crow + cc, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (arow) x += arow[cc];
+        if (e.accumulate && std::is_same<OT, float>::value) {
+          __hip_atomic_fetch_add((float *)crow + cc, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           continue;
         }
-        if (ACC) x += (float)crow[cc];
+        if (e.accumulate) x += (float)crow[cc];
         crow[cc] = (OT)x;
       }
-    }
+  }
 }
 
-template <class L, typename OT, bool ACC, bool ADD>
-__device__ __forceinline__ void store_edge(const typename L::V (&acc)[L::NI][L::NJ], OT *C, const float *addend,
-                                           int64_t ldc, int64_t ld_add, int64_t m0, int64_t n0, int64_t mvalid,
-                                           int64_t nvalid, int wm, int wn, int lane, const float *rs) {
-  if (mvalid < TM || nvalid < TN)
-    store_tile<L, OT, ACC, ADD, true>(acc, C, addend, ldc, ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
-  else store_tile<L, OT, ACC, ADD, false>(acc, C, addend, ldc, ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
+// A whole-width 16-bit tile with nothing to add: through the LDS (the ring, free after the mainloop) and out in rows of
+// 512 bytes, 16 bytes per lane. Stored from the registers, as four 2-byte stores (the MFMA's own layout) or one of 8
+// bytes per block, a wave's store covers 32-byte pieces of 4 or 16 lines, and tiles of few K-stages, grad_W's of a short
+// call, spend longer storing than multiplying: at d 2560, V 151,936 and 64 rows (one stage) grad_W takes 195 us this
+// way, 264 with 2-byte and 294 with 8-byte stores; at 225 rows 298, 376 and 401; at 3,000 1,765, 1,783 and 1,811. Its
+// floor is the write of 0.78 GB, 114 us at this card's fill rate. With the operands exchanged (Acc16T) a lane's 4 values
+// go into the LDS in one write.
+template <class L, typename OT>
+__device__ __forceinline__ void store_staged(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
+                                             int64_t n0, int64_t mvalid, lds_char *smem) {
+  typedef typename std::conditional<std::is_same<OT, __bf16>::value, bf16x2, f16x2_t>::type P2;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
+#pragma unroll
+  for (int i = 0; i < L::NI; ++i) {
+    const int rr = L::row(wm, i, lane), sw = DzSwz<Acc16N<4>>::at(rr);
+    const float sc = e.row_scale && rr < mvalid ? e.row_scale[m0 + rr] : 1.f;
+#pragma unroll
+    for (int j = 0; j < L::NJ; ++j) {
+      i32x2 p;
+      p[0] = (int)pack2(acc[i][j][0] * sc, acc[i][j][1] * sc, (P2 *)nullptr);
+      p[1] = (int)pack2(acc[i][j][2] * sc, acc[i][j][3] * sc, (P2 *)nullptr);
+      *(lds_i32x2 *)(smem + rr * 512 + (((L::col(wn, j, lane) >> 2) ^ sw) << 3)) = p;
+    }
+  }
+  __syncthreads();
+  const int c16 = threadIdx.x & 31;
+  char *dst = (char *)e.C + (m0 * e.ldc + n0) * 2 + c16 * 16;
+#pragma unroll 4
+  for (int p = 0; p < 256 / 16; ++p) {
+    const int row = p * 16 + (threadIdx.x >> 5), s = DzSwz<Acc16N<4>>::at(row);
+    i32x4 v = *(const lds_i32x4 *)(smem + row * 512 + ((2 * c16) ^ (s & ~1)) * 8);
+    if (s & 1) v = __builtin_shufflevector(v, v, 2, 3, 0, 1);
+    if (row < mvalid) __builtin_nontemporal_store(v, (i32x4 *)(dst + row * e.ldc * 2));
+  }
 }
 
 template <class L, typename OT>
 __device__ __forceinline__ void store_any(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
-                                          int64_t n0, int64_t mvalid, int64_t nvalid) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
-  OT *c = (OT *)e.C;
-  const float *rs = e.row_scale;
-  if (e.accumulate) {
-    if (e.addend) store_edge<L, OT, true, true>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
-    else store_edge<L, OT, true, false>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
-  } else {
-    if (e.addend) store_edge<L, OT, false, true>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
-    else store_edge<L, OT, false, false>(acc, c, e.addend, e.ldc, e.ld_add, m0, n0, mvalid, nvalid, wm, wn, lane, rs);
+                                          int64_t n0, int64_t mvalid, int64_t nvalid, lds_char *smem) {
+  if constexpr (sizeof(OT) == 2) {
+    if ((uintptr_t)e.C % 16 == 0 && e.ldc % 8 == 0 && !e.addend && !e.accumulate && nvalid >= TN) {
+      store_staged<L, OT>(acc, e, m0, n0, mvalid, smem);
+      return;
+    }
   }
+  store_tile<L, OT>(acc, e, m0, n0, mvalid, nvalid);
 }
 
 // The tile's fp32 partials in the blocked layout (StoreArgs::part_blocked): this wave's 8192 values, element v of
@@ -412,17 +433,16 @@ __device__ __forceinline__ void store_blocked(const typename L::V (&acc)[L::NI][
       }
 }
 
-// A split-K run's partial tile (StoreArgs::split): the accumulators in their own order, 256 contiguous bytes per store.
+// A split-K run's partial tile (StoreArgs::split): the accumulators in their own order, [wave][i][j][lane][v], 1 KB per
+// store of a wave.
 template <class L>
 __device__ __forceinline__ void store_split(const typename L::V (&acc)[L::NI][L::NJ], float *tile) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  float *b = tile + w * (L::NI * L::NJ * L::NV * 64) + lane;
+  f32x4 *b = (f32x4 *)tile + w * (L::NI * L::NJ * 64) + lane;
 #pragma unroll
   for (int i = 0; i < L::NI; ++i)
 #pragma unroll
-    for (int j = 0; j < L::NJ; ++j)
-#pragma unroll
-      for (int v = 0; v < L::NV; ++v) b[((i * L::NJ + j) * L::NV + v) * 64] = acc[i][j][v];
+    for (int j = 0; j < L::NJ; ++j) b[(i * L::NJ + j) * 64] = acc[i][j];
 }
 
 // acc += the blocked partials of the earlier passes (the pass that stores C).
@@ -440,9 +460,9 @@ __device__ __forceinline__ void add_blocked(typename L::V (&acc)[L::NI][L::NJ], 
 
 template <class L, typename OT>
 __device__ __forceinline__ void store_pass(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int which,
-                                           int64_t m0, int64_t n0, int64_t mvalid, int64_t nvalid) {
+                                           int64_t m0, int64_t n0, int64_t mvalid, int64_t nvalid, lds_char *smem) {
   if (which == 1) {
-    store_any<L, OT>(acc, e, m0, n0, mvalid, nvalid);
+    store_any<L, OT>(acc, e, m0, n0, mvalid, nvalid, smem);
   } else if (e.part_blocked) {
     store_blocked<L>(acc, e, m0, n0);
   } else {
@@ -451,7 +471,7 @@ __device__ __forceinline__ void store_pass(const typename L::V (&acc)[L::NI][L::
     p.addend = nullptr;
     p.accumulate = e.part_accumulate;
     p.row_scale = nullptr;
-    store_any<L, float>(acc, p, m0, n0, mvalid, nvalid);
+    store_any<L, float>(acc, p, m0, n0, mvalid, nvalid, smem);
   }
 }
 
@@ -471,26 +491,27 @@ __device__ __forceinline__ void store8_tile(const Operand &A, const Operand &B, 
   if (s.count_on == 1) mvalid = dev_count(s.count, s.count_off + m0, mvalid);
   if (s.count_on == 3) K_eff = round_up(dev_count(s.count, s.count_off, s.K), 64);
   if (mvalid <= 0 || nvalid <= 0 || adds_nothing(e, which, K_eff)) return;
+  typedef Acc16T L;
   f32x4 acc[8][4];
-  if constexpr (KM == KM_A) mainloop_ring5<DT, OpColsN<8, 128>, OpRowsN<8, 64>>(A, B, m0, n0, K_eff, smem, acc);
-  else if constexpr (KM == KM_B) mainloop_ring5<DT, OpRowsN<8, 128>, OpColsN<8, 64>, true>(A, B, m0, n0, K_eff, smem, acc);
-  else mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true>(A, B, m0, n0, K_eff, smem, acc);
+  if constexpr (KM == KM_A) mainloop_ring5<DT, OpColsN<8, 128>, OpRowsN<8, 64>, false, true>(A, B, m0, n0, K_eff, smem, acc);
+  else if constexpr (KM == KM_B) mainloop_ring5<DT, OpRowsN<8, 128>, OpColsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
+  else mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
   if (KM != KM_A && part) {
-    store_split<Acc16N<4>>(acc, part);
+    store_split<L>(acc, part);
     return;
   }
   StoreArgs eb = e;
   if (e.part_blocked && which == 1 && e.addend) {  // the blocked partials added here, C stored as usual
-    add_blocked<Acc16N<4>>(acc, e.addend, e.ldc, m0, n0);
+    add_blocked<L>(acc, e.addend, e.ldc, m0, n0);
     eb.addend = nullptr;
   }
   if constexpr (OT >= 0) {
-    store_pass<Acc16N<4>, typename Elem<OT>::T>(acc, eb, which, m0, n0, mvalid, nvalid);
+    store_pass<L, typename Elem<OT>::T>(acc, eb, which, m0, n0, mvalid, nvalid, smem);
   } else {
     switch (eb.dtype) {
-      case OCTO_BF16: store_pass<Acc16N<4>, __bf16>(acc, eb, which, m0, n0, mvalid, nvalid); break;
-      case OCTO_F16: store_pass<Acc16N<4>, _Float16>(acc, eb, which, m0, n0, mvalid, nvalid); break;
-      default: store_pass<Acc16N<4>, float>(acc, eb, which, m0, n0, mvalid, nvalid); break;
+      case OCTO_BF16: store_pass<L, __bf16>(acc, eb, which, m0, n0, mvalid, nvalid, smem); break;
+      case OCTO_F16: store_pass<L, _Float16>(acc, eb, which, m0, n0, mvalid, nvalid, smem); break;
+      default: store_pass<L, float>(acc, eb, which, m0, n0, mvalid, nvalid, smem); break;
     }
   }
 }

@@ -2,15 +2,15 @@
 // rounded once to C's type.
 //
 // Bound by memory: S partial tiles of 256 KB read per tile of C. One workgroup per 16 rows of a tile, 256 threads: each
-// wave reads its accumulator blocks in the order the GEMM's wave left them (256 contiguous bytes per load, the runs in
-// order, so the sum is the same every time), and the 16 x 256 result goes through the LDS to be stored 4 values a
-// thread along the rows. 225 rows at d 2560, V 151,936 (26 runs of 10 tiles, 68 MB): 16 us.
+// wave reads its accumulator blocks in the order the GEMM's wave left them (1 KB per load, the runs in order, so the
+// sum is the same every time), and the 16 x 256 result goes through the LDS to be stored in whole rows. 225 rows at d 2560, V 151,936 (26 runs of 10 tiles, 68 MB): 16 us.
 #include "gemm_nt.h"
 #include "octo_internal.h"
 
 namespace octo {
 
-// NJ: 16-column blocks per wave, 4 waves across the tile (256 columns: 4; fp32 operands, 128 columns: 2).
+// NJ: 16-column blocks per wave, 4 waves across the tile (256 columns: 4; fp32 operands, 128 columns: 2). A
+// lane's 4 values of a block are 4 columns of a row (Acc16T).
 template <typename OT, int NJ>
 __global__ __launch_bounds__(256) void split_sum_kernel(GemmShape s, StoreArgs e) {
   constexpr int NI = 8, NV = 4, TNX = 64 * NJ, WAVE = NI * NJ * NV * 64;
@@ -29,19 +29,22 @@ __global__ __launch_bounds__(256) void split_sum_kernel(GemmShape s, StoreArgs e
   if (row0 >= mvalid) return;
 
   const int lane = threadIdx.x & 63, wn = threadIdx.x >> 6;
-  const float *p = e.split + at * (TM * TNX) + (wm * 4 + wn) * WAVE + i * (NJ * NV * 64) + lane;
-  float a[NJ * NV];
+  const f32x4 *p = (const f32x4 *)(e.split + at * (TM * TNX) + (wm * 4 + wn) * WAVE + i * (NJ * NV * 64)) + lane;
+  f32x4 a[NJ];
 #pragma unroll
-  for (int k = 0; k < NJ * NV; ++k) a[k] = 0.f;
-#pragma unroll 2
-  for (int run = 0; run < S; ++run, p += tiles * (TM * TNX)) {
+  for (int j = 0; j < NJ; ++j) a[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int run = 0; run < S; ++run, p += tiles * (TM * TNX / 4)) {
 #pragma unroll
-    for (int k = 0; k < NJ * NV; ++k) a[k] += p[k * 64];
+    for (int j = 0; j < NJ; ++j) {
+      const f32x4 x = p[j * 64];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) a[j][v] += x[v];
+    }
   }
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
-#pragma unroll
-    for (int v = 0; v < NV; ++v) tile[(4 * (lane >> 4) + v) * LDT + (wn * NJ + j) * 16 + (lane & 15)] = a[j * NV + v];
+    *(f32x4 *)(tile + (lane & 15) * LDT + (wn * NJ + j) * 16 + 4 * (lane >> 4)) = a[j];
   __syncthreads();
 
   const int row = threadIdx.x >> 4;
