@@ -60,6 +60,11 @@ SIGNATURES = {
     "octo_head_step_grpo_pairs": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _p, _i64, _i32, _i32, _i32,
                                   _f32, _f32, _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail),
                                   _p, _i64, _i32, _p, _i32, _p, _sz, _p],
+    "octo_head_stage_bytes": [_i64, _i32, _i32, _i32, ctypes.POINTER(_sz)],
+    "octo_head_fwd_stage": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
+                            _f32, _i32, _p, _p, _i64, _p, _sz, _p],
+    "octo_head_bwd_stage": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
+                            _f32, _i32, _p, _p, _p, _p, _i64, _i32, _p, _i32, _p, _sz, _p],
     "octo_columns_fwd": [_p, _i64, _i32, _p, _i64, _i32, _f32, _p, _p, _p],
     "octo_columns_bwd": [_p, _i64, _i32, _p, _i64, _i32, _f32, _p, _p, _p, _i64, _p],
     "octo_pairs_expand": [_p, _i64, _i32, _p, _i64, _p, _p],
@@ -132,6 +137,13 @@ def bwd_plan(n_max: int, d: int, V: int, w_dtype: int, flags: int, ws_bytes: int
     WS_STEP in flags, octo_head_step_grpo's (rows per pass, passes, V rounded up to 256, 1)."""
     out = (_i64 * 4)()
     call("octo_head_bwd_plan", n_max, d, V, w_dtype, flags, ws_bytes, out)
+    return tuple(out)
+
+
+def stage_bytes(n_max: int, d: int, V: int, w_dtype: int) -> tuple[int, int]:
+    """(octo_head_fwd_stage's buffer, octo_head_bwd_stage's workspace); zeros for a call that is not staged."""
+    out = (_sz * 2)()
+    call("octo_head_stage_bytes", n_max, d, V, w_dtype, out)
     return tuple(out)
 
 

@@ -263,21 +263,27 @@ __global__ __launch_bounds__(256) void dz_scale_kernel(DzScaleArgs a) {
   const int64_t i = blockIdx.y;  // row of the pass
   const int64_t r = a.r0 + i;
   const int64_t cnt = a.count ? min((int64_t)(*a.count), a.n_max) : a.n_max;
-  if (r >= cnt) return;
+  char *row = (char *)a.dz + i * a.ld * 2;
+  const char *src = a.ex ? (const char *)a.ex + i * a.ld * 2 : row;
+  const int64_t chunk0 = (int64_t)blockIdx.x * (256 * kScaleChunks) + threadIdx.x;
+  if (r >= cnt) {
+    if (a.ex && r < (cnt + 63) / 64 * 64)
+      for (int k = 0; k < kScaleChunks; ++k)
+        if ((chunk0 + 256 * k) * 8 < a.V_pad) *(i32x4 *)(row + (chunk0 + 256 * k) * 16) = i32x4{0, 0, 0, 0};
+    return;
+  }
   float m2, l2s;
   row_state(a.lse, a.lse_pair, r, m2, l2s);
   const float ngs = -(a.g[r] * a.gmul);
   const int64_t y = a.labels[a.label_idx ? a.label_idx[r] : r];
   const bool f16 = a.dtype == OCTO_F16;
   const f32x4 *pr = a.part + i * a.mtiles;
-  char *row = (char *)a.dz + i * a.ld * 2;
-  const int64_t chunk0 = (int64_t)blockIdx.x * (256 * kScaleChunks) + threadIdx.x;
   i32x4 v[kScaleChunks];
 #pragma unroll
   for (int k = 0; k < kScaleChunks; ++k) {
     const int64_t c0 = (chunk0 + 256 * k) * 8;
     if (c0 < a.V_pad)
-      v[k] = OCTO_SCALE_NT_LOAD ? __builtin_nontemporal_load((const i32x4 *)(row + c0 * 2)) : *(const i32x4 *)(row + c0 * 2);
+      v[k] = OCTO_SCALE_NT_LOAD ? __builtin_nontemporal_load((const i32x4 *)(src + c0 * 2)) : *(const i32x4 *)(src + c0 * 2);
   }
 #pragma unroll
   for (int k = 0; k < kScaleChunks; ++k) {
@@ -426,7 +432,7 @@ int launch_ex_fix(const ExFixArgs &a, hipStream_t st) {
 // x = NULL: y = c s. The product and the sum are formed in fp32 and rounded once to the vector's type. In place (s =
 // y) with c = 1 and no x to add, y is already the result and every workgroup ends at once. Bound by memory: 16 bytes
 // per load, kScaleLoads of them in flight per thread, a grid of 8 workgroups per CU walking the vector. [151,936, 2560]
-// bf16 out of place: @US@ us, against 1,350 us for the same arithmetic as three elementwise kernels (widen, multiply,
+// bf16 out of place: 268 us, against 1,350 us for the same arithmetic as three elementwise kernels (widen, multiply,
 // narrow).
 constexpr int kScaleLoads = 4;
 __global__ __launch_bounds__(256) void scale_add_kernel(void *y, const void *src, const void *x, int dtype, int64_t n,

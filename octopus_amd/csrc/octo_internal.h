@@ -290,6 +290,8 @@ int launch_ex_fix(const ExFixArgs &a, hipStream_t st);
 // read dz stop at the count).
 struct DzScaleArgs {
   void *dz;  // [rows, ld] 16-bit: f16 exponentials in, dz in dtype (bf16 / f16) out
+  const void *ex = nullptr;  // the exponentials where they are not in dz's place: kept, and dz zero from the count to the
+                             // next multiple of 64, the rows a count-bounded grad_W reads
   int64_t ld, V_pad;
   int dtype;
   const f32x4 *part;  // [rows, mtiles], local rows

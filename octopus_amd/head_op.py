@@ -415,14 +415,7 @@ def _head_backward(ctx, gout, _glse):
     need_rows, need_weight = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
     if need_weight and weight.dtype == torch.float8_e4m3fn:
         raise NotImplementedError("octohead: no gradient for fp8 weights")
-    gout = gout.float()
-    if scatter:  # g of compact row r is the output gradient at its hidden row idx[r]
-        col = gout[:, 0].contiguous()
-        idx64 = idx.to(torch.int64).contiguous()
-        g = torch.empty(idx.numel(), dtype=torch.float32, device=gout.device)
-        _lib.call("octo_gather_f32", _p(col), 1, _p(idx64), _p(count), idx.numel(), _p(g), _stream(gout))
-    else:
-        g = gout[:, 0].contiguous()
+    g = _compact_g(gout, idx, count, scatter)
     grad_rows, grad_w = head_bwd(rows, weight, w_scale, labels, idx, count, lse, g, inv_T, pre, post, use_tanh,
                                  labels_via_idx, need_rows, need_weight)
     return (grad_rows if need_rows else None, grad_w if need_weight else None,
@@ -432,6 +425,140 @@ def _head_backward(ctx, gout, _glse):
 torch.library.register_autograd("octohead::head_fwd", _head_backward, setup_context=_head_setup)
 
 
+# ---- the head with its exponentials kept between forward and backward (octo_head_fwd_stage) --------------------------
+
+_STAGE_BYTES = 2 << 30  # of the kept exponentials, padded to 256 rows and columns: the backward's own staging budget
+# fused_head keeps them from this many multiply-adds of the logits on (n d V). The recompute they save takes 1.5 ns per
+# 2^20 of them; the wider store and the pass that makes dz cost a small call some 10 us, 2^33 multiply-adds' worth.
+_STAGE_WORK = 1 << 33
+
+
+def _pad256(n: int) -> int:
+    return (n + 255) // 256 * 256
+
+
+def _stage_numel(n_max: int, V: int) -> int:
+    """Bytes of the buffer, as octo_head_stage_bytes has them: exponentials, label entries, the forward's workspace."""
+    return _pad256(n_max) * _pad256(V) * 2 + _pad256(_pad256(n_max) * 4) + _pad256(n_max * (_pad256(V) // 256) * 16) + 256
+
+
+def _stages(rows: Tensor, weight: Tensor, idx: Optional[Tensor], scale: float) -> bool:
+    """Whether fused_head keeps the exponentials: a gradient is wanted, octo_head_fwd_stage takes the call and the
+    recompute would cost more. Not while a compiler traces (a guard on the sizes), nor with a backward workspace set."""
+    if BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not torch.is_grad_enabled():
+        return False
+    if not (rows.requires_grad or weight.requires_grad) or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
+        return False
+    if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not 1e-30 < scale < 1e30:
+        return False
+    n = idx.numel() if idx is not None else rows.shape[0]
+    V, d = weight.shape
+    # rows through idx lie below 2 GiB, as they are or (twice the numel covers any stride _rows2d keeps) copied
+    return (0 < n <= 32768 and _pad256(n) * _pad256(V) * 2 <= _STAGE_BYTES and n * d * V >= _STAGE_WORK
+            and not (idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff))
+
+
+@torch.library.custom_op("octohead::head_fwd_stage", mutates_args=(), device_types="cuda")
+def head_fwd_stage(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
+                   inv_T: float, pre: float, post: float, use_tanh: bool, labels_via_idx: bool,
+                   scatter: bool) -> tuple[Tensor, Tensor, Tensor]:
+    """head_fwd's (out, lse) and the buffer head_bwd_stage makes the gradients of."""
+    rows, weight = _rows2d(rows), _rows2d(weight)
+    labels, idx = _index(labels), _index(idx)
+    n_max = idx.numel() if idx is not None else rows.shape[0]
+    V, d = weight.shape
+    flags = (_lib.ROWS_VIA_IDX if labels_via_idx else 0) | (_lib.OUT_SCATTER if scatter else 0) | _lib.LSE_PAIR
+    out = torch.zeros(rows.shape[0] if scatter else n_max, 2, dtype=torch.float32, device=rows.device)
+    lse = torch.zeros(n_max, 2, dtype=torch.float32, device=rows.device)
+    code = _dtype_code(weight)
+    stage = _workspace(_lib.stage_bytes(n_max, d, V, code)[0], rows)
+    _lib.call("octo_head_fwd_stage", _p(rows), rows.shape[0], rows.stride(0), code, _p(weight), weight.stride(0), code,
+              _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse), _p(out), 2,
+              _p(stage), stage.numel(), _stream(rows))
+    return out, lse, stage
+
+
+@head_fwd_stage.register_fake
+def _(rows, weight, labels, idx, count, inv_T, pre, post, use_tanh, labels_via_idx, scatter):
+    n_max = idx.shape[0] if idx is not None else rows.shape[0]
+    return (rows.new_empty(rows.shape[0] if scatter else n_max, 2, dtype=torch.float32),
+            rows.new_empty(n_max, 2, dtype=torch.float32),
+            rows.new_empty(_stage_numel(n_max, weight.shape[0]), dtype=torch.uint8))
+
+
+@torch.library.custom_op("octohead::head_bwd_stage", mutates_args=(), device_types="cuda")
+def head_bwd_stage(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
+                   lse: Tensor, stage: Tensor, g: Tensor, inv_T: float, pre: float, post: float, use_tanh: bool,
+                   labels_via_idx: bool, need_rows: bool, need_weight: bool) -> tuple[Tensor, Tensor]:
+    """head_bwd's (grad_rows, grad_weight) from head_fwd_stage's buffer."""
+    rows2, weight2 = _rows2d(rows), _rows2d(weight)
+    labels, idx = _index(labels), _index(idx)
+    n_max = idx.numel() if idx is not None else rows2.shape[0]
+    V, d = weight2.shape
+    grad_rows = _zeros(rows) if need_rows else rows.new_empty(0)
+    grad_w = _empty(weight) if need_weight else weight.new_empty(0)
+    if not (need_rows or need_weight):
+        return grad_rows, grad_w
+    flags = (_lib.ROWS_VIA_IDX if labels_via_idx else 0) | _lib.LSE_PAIR
+    gh = None
+    if need_rows:  # compact-order rows; scattered (runs of equal idx summed) into grad_rows below
+        gh = grad_rows if idx is None else torch.empty(n_max, d, dtype=rows2.dtype, device=rows2.device)
+    code = _dtype_code(weight2)
+    ws = _workspace(_lib.stage_bytes(n_max, d, V, code)[1], rows2)
+    lse_c, g_c = lse.contiguous(), g.contiguous()  # kept alive until the call has queued its kernels
+    _lib.call("octo_head_bwd_stage", _p(rows2), rows2.shape[0], rows2.stride(0), code, _p(weight2), weight2.stride(0),
+              code, _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse_c),
+              _p(g_c), _p(stage), _p(gh), d, code, _p(grad_w if need_weight else None), code, _p(ws), ws.numel(),
+              _stream(rows2))
+    if need_rows and idx is not None:
+        _lib.call("octo_rows_scatter", _p(gh), d, code, _p(idx), _p(count), n_max, d, _p(grad_rows),
+                  grad_rows.stride(0), code, 0, _stream(rows2))
+    return grad_rows, grad_w
+
+
+@head_bwd_stage.register_fake
+def _(rows, weight, labels, idx, count, lse, stage, g, inv_T, pre, post, use_tanh, labels_via_idx, need_rows,
+      need_weight):
+    return (_empty(rows) if need_rows else rows.new_empty(0),
+            _empty(weight) if need_weight else weight.new_empty(0))
+
+
+def _compact_g(gout: Tensor, idx: Optional[Tensor], count: Optional[Tensor], scatter: bool) -> Tensor:
+    """dL/dlogprob per compact row from the columns' gradient."""
+    gout = gout.float()
+    if not scatter:
+        return gout[:, 0].contiguous()
+    col = gout[:, 0].contiguous()  # g of compact row r is the output gradient at its hidden row idx[r]
+    idx64 = idx.to(torch.int64).contiguous()
+    g = torch.empty(idx.numel(), dtype=torch.float32, device=gout.device)
+    _lib.call("octo_gather_f32", _p(col), 1, _p(idx64), _p(count), idx.numel(), _p(g), _stream(gout))
+    return g
+
+
+def _stage_setup(ctx, inputs, output):
+    rows, weight, labels, idx, count = inputs[:5]
+    # the weight and the buffer are held by reference, not saved: a pack hook never copies them to the host
+    ctx.weight = weight
+    ctx.stage = output[2].detach()
+    ctx.params = inputs[5:]
+    ctx.save_for_backward(rows, labels, idx, count, output[1])
+
+
+def _stage_backward(ctx, gout, _glse, _gstage):
+    rows, labels, idx, count, lse = ctx.saved_tensors
+    inv_T, pre, post, use_tanh, labels_via_idx, scatter = ctx.params
+    need_rows, need_weight = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+    g = _compact_g(gout, idx, count, scatter)
+    grad_rows, grad_w = head_bwd_stage(rows, ctx.weight, labels, idx, count, lse, ctx.stage, g, inv_T, pre, post,
+                                       use_tanh, labels_via_idx, need_rows, need_weight)
+    if not torch._C._autograd._get_current_graph_task_keep_graph():
+        ctx.stage = None  # as the saved tensors: a loss kept for its value does not keep the buffer
+    return (grad_rows if need_rows else None, grad_w if need_weight else None) + (None,) * 9
+
+
+torch.library.register_autograd("octohead::head_fwd_stage", _stage_backward, setup_context=_stage_setup)
+
+
 def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float, post: Post = Post(), *,
                idx: Optional[Tensor] = None, count: Optional[Tensor] = None, labels_via_idx: bool = False,
                scatter: bool = False, w_scale: Optional[Tensor] = None) -> Tensor:
@@ -439,8 +566,10 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
     with scatter, a [rows, 2] tensor holding each compact row at idx[r] and 0 elsewhere."""
     if temperature <= 0:
         raise ValueError("temperature must be positive")
-    out, _ = head_fwd(rows, weight, w_scale, labels, idx, count, 1.0 / float(temperature), float(post.pre),
-                      float(post.post), bool(post.tanh), labels_via_idx, scatter)
+    xf = (1.0 / float(temperature), float(post.pre), float(post.post), bool(post.tanh), labels_via_idx, scatter)
+    if _stages(rows, weight, idx, xf[0] * (1.0 if post.tanh else xf[1]) * xf[2]):
+        return head_fwd_stage(rows, weight, labels, idx, count, *xf)[0]
+    out, _ = head_fwd(rows, weight, w_scale, labels, idx, count, *xf)
     return out
 
 
