@@ -842,10 +842,11 @@ __global__ __launch_bounds__(NT) void columns_fwd_kernel(const void *logits, int
       u += red[2][k];
     }
     const float l2S = flog2(s);
-    const float lse = (m2 + l2S) * OCTO_LN2;
     const int64_t y = labels[r];
-    const float sy = (y >= 0 && y < V) ? (float)row[y] * inv_T : __builtin_nanf("");
-    out2[2 * r] = sy - lse;
+    // the label's logit as the sums have it, base 2 and relative to the maximum: close to a probability of 1 the logprob
+    // is far smaller than the logits, and lse's own rounding (1e-6 at 18) would be a part of it
+    const float ty = (y >= 0 && y < V) ? __builtin_fmaf((float)row[y], c, -m2) : __builtin_nanf("");
+    out2[2 * r] = (ty - l2S) * OCTO_LN2;
     out2[2 * r + 1] = (l2S - u / s) * OCTO_LN2;
     if (lse_out) {  // the row state (m2, l2S) for columns_bwd, as row_state's paired form
       lse_out[2 * r] = m2;
