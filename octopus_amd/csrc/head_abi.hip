@@ -224,7 +224,13 @@ StoreArgs grad_w_store(int d, int64_t r0, int64_t rows, int64_t p, int64_t passe
   const bool last_pass = p + 1 == passes;
   StoreArgs o;
   const bool acc_out = flags & OCTO_GRADW_ACCUMULATE;
-  if (gacc_on && !last_pass && !count) {  // fp32 partial sums of the passes so far
+  o.part_blocked = (blocked && gacc_on && d % TN == 0) ? 1 : 0;
+  if (gacc_on && !last_pass && !count && o.part_blocked) {  // as below, chosen here
+    o.C = gw;
+    o.dtype = gw_dtype;
+    o.part = gacc;
+    o.part_accumulate = p > 0 ? 1 : 0;
+  } else if (gacc_on && !last_pass && !count) {  // fp32 partial sums of the passes so far
     o.C = gacc;
     o.addend = nullptr;
     o.dtype = OCTO_F32;
@@ -249,8 +255,6 @@ StoreArgs grad_w_store(int d, int64_t r0, int64_t rows, int64_t p, int64_t passe
     o.part = gacc;
     o.part_accumulate = p > 0 ? 1 : 0;
   }
-  // with a device count every pass reaches the partials through part / addend, so their layout may be blocked
-  o.part_blocked = (blocked && count && gacc_on && d % TN == 0) ? 1 : 0;
   o.ldc = d;
   o.ld_add = d;
   return o;

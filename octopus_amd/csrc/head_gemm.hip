@@ -328,36 +328,53 @@ __device__ __forceinline__ void dz_write(const DzArgs &e, int64_t ma, int64_t m0
 // ---- epilogue: plain store -------------------------------------------------------------------
 
 // C = rs[row] x acc (rs NULL: acc) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to OT, value
-// by value. An fp32 C += acc is one no-return atomic add per element, performed in the L2, so the tile's epilogue does
+// by value: ragged and unaligned tiles, fp32 output, sums. The accumulators go through the LDS (the ring, free after the
+// mainloop) in two halves of 128 rows, so that a wave stores, adds to or reads 64 neighbours of a row; from the
+// registers it would cover 16 bytes of each of 16 rows (Acc16T), and the fp32 partials of several passes, read and
+// added to at every pass, made the step's gradients slower: 20,110 rows without a row count, d 2048, V 128,256, 26.3 ms
+// a step so, 25.3 with 64-byte pieces (Acc16N).
+// An fp32 C += acc is one no-return atomic add per element, performed in the L2, so the tile's epilogue does
 // not wait for C to be read (grad_W's fp32 partials of the fused step at 24,576 rows, d 2560, V 151,936: the gradient
 // launches 28.35 against 28.65 ms per step, same box). A launch adds to each element once (one tile), so the sums keep
 // launch order and are reproducible.
 template <class L, typename OT>
 __device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
-                                           int64_t n0, int64_t mvalid, int64_t nvalid) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
+                                           int64_t n0, int64_t mvalid, int64_t nvalid, lds_char *smem) {
+  static_assert(128 * TN * 4 <= SMEM_RING5 && L::NI == 8, "half a tile of fp32 in the LDS");
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = L::wm(w), wn = L::wn(w);
+  typedef __attribute__((address_space(3))) float lds_float;
+  // 16-byte slot c / 4 of row r sits at slot (c / 4) ^ (r & 15): a wave's write, 16 rows of 4 slots, covers all banks
+  for (int half = 0; half < 2; ++half) {
+    if (half) __syncthreads();  // the first half's reads are done
+    if (wm == half) {
 #pragma unroll
-  for (int i = 0; i < L::NI; ++i) {
-    const int rr = L::row(wm, i, lane);
-    if (rr >= mvalid) continue;
-    OT *crow = (OT *)e.C + (m0 + rr) * e.ldc + n0;
-    const float *arow = e.addend ? e.addend + (m0 + rr) * e.ld_add + n0 : nullptr;
-    const float sc = e.row_scale ? e.row_scale[m0 + rr] : 1.f;
+      for (int i = 0; i < L::NI; ++i)
 #pragma unroll
-    for (int j = 0; j < L::NJ; ++j)
+        for (int j = 0; j < L::NJ; ++j) {
+          const int r = L::row(0, i, lane);
+          *(lds_f32x4 *)(smem + r * (TN * 4) + (((L::col(wn, j, lane) >> 2) ^ (r & 15)) << 4)) = acc[i][j];
+        }
+    }
+    __syncthreads();
+    for (int r = w; r < 128 && half * 128 + r < mvalid; r += 8) {
+      const int64_t row = m0 + half * 128 + r;
+      OT *crow = (OT *)e.C + row * e.ldc + n0;
+      const float *arow = e.addend ? e.addend + row * e.ld_add + n0 : nullptr;
+      const float sc = e.row_scale ? e.row_scale[row] : 1.f;
 #pragma unroll
-      for (int v = 0; v < L::NV; ++v) {
-        const int cc = L::col(wn, j, lane) + v;
-        if (cc >= nvalid) continue;
-        float x = acc[i][j][v] * sc;
-        if (arow) x += arow[cc];
+      for (int q = 0; q < TN / 64; ++q) {
+        const int c = 64 * q + lane;
+        if (c >= nvalid) continue;
+        float x = *(const lds_float *)(smem + r * (TN * 4) + (((c >> 2) ^ (r & 15)) << 4) + (c & 3) * 4) * sc;
+        if (arow) x += arow[c];
         if (e.accumulate && std::is_same<OT, float>::value) {
-          __hip_atomic_fetch_add((float *)crow + cc, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add((float *)crow + c, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
           continue;
         }
-        if (e.accumulate) x += (float)crow[cc];
-        crow[cc] = (OT)x;
+        if (e.accumulate) x += (float)crow[c];
+        crow[c] = (OT)x;
       }
+    }
   }
 }
 
@@ -406,7 +423,7 @@ __device__ __forceinline__ void store_any(const typename L::V (&acc)[L::NI][L::N
       return;
     }
   }
-  store_tile<L, OT>(acc, e, m0, n0, mvalid, nvalid);
+  store_tile<L, OT>(acc, e, m0, n0, mvalid, nvalid, smem);
 }
 
 // The tile's fp32 partials in the blocked layout (StoreArgs::part_blocked): this wave's 8192 values, element v of

@@ -117,7 +117,7 @@ struct StoreArgs {
   // a pass that starts at or past the count (pass_r0 > 0) stores nothing. With fp32 partials (part != NULL, laid out
   // as C with row stride ldc), the pass whose end reaches the count (count <= pass_end) stores the final C as above
   // (addend = the earlier passes' partials); an earlier pass stores its sum to part instead (= or += by
-  // part_accumulate). No count: C as above, the host having chosen the destination.
+  // part_accumulate). No count: the host has chosen, part when it is set, else C as above.
   const int32_t *pass_count = nullptr;
   int64_t pass_r0 = 0, pass_end = 0;
   float *part = nullptr;
@@ -147,7 +147,7 @@ __device__ __forceinline__ bool adds_nothing(const StoreArgs &e, int which, int6
 
 // Which store a row pass's GEMM makes (StoreArgs pass_count / part): 0 none, 1 the final C, 2 the fp32 partials.
 __device__ __forceinline__ int pass_store(const StoreArgs &e) {
-  if (!e.pass_count) return 1;
+  if (!e.pass_count) return e.part ? 2 : 1;
   const int64_t c = *e.pass_count;
   if (e.pass_r0 > 0 && c <= e.pass_r0) return 0;
   return (e.part && c > e.pass_end) ? 2 : 1;
