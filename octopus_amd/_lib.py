@@ -60,6 +60,10 @@ SIGNATURES = {
     "octo_head_step_grpo_pairs": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _p, _i64, _i32, _i32, _i32,
                                   _f32, _f32, _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail),
                                   _p, _i64, _i32, _p, _i32, _p, _sz, _p],
+    "octo_head_later_bytes": [_i64, _i32, _i32, _i32, _i32, ctypes.POINTER(_sz)],
+    "octo_head_step_later": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
+                             _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail), _p, _i64, _i32, _p, _sz, _p],
+    "octo_head_later_grad_w": [_p, _p, _i64, _i32, _i32, _i32, _i32, _p, _p, _i32, _p],
     "octo_head_stage_bytes": [_i64, _i32, _i32, _i32, ctypes.POINTER(_sz)],
     "octo_head_fwd_stage": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
                             _f32, _i32, _p, _p, _i64, _p, _sz, _p],
@@ -138,6 +142,13 @@ def bwd_plan(n_max: int, d: int, V: int, w_dtype: int, flags: int, ws_bytes: int
     out = (_i64 * 4)()
     call("octo_head_bwd_plan", n_max, d, V, w_dtype, flags, ws_bytes, out)
     return tuple(out)
+
+
+def later_bytes(n_max: int, d: int, V: int, w_dtype: int, need_gh: bool) -> int:
+    """The buffer octo_head_step_later works in and its caller keeps; 0 for a call it does not take."""
+    out = _sz(0)
+    call("octo_head_later_bytes", n_max, d, V, w_dtype, int(need_gh), ctypes.byref(out))
+    return out.value
 
 
 def stage_bytes(n_max: int, d: int, V: int, w_dtype: int) -> tuple[int, int]:

@@ -403,12 +403,13 @@ struct StepPairs {
   int64_t ld_out;
 };
 
+// later: without grad_W (grad_w NULL), its operands left in the workspace (later_plan).
 int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
               const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
               int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *logp, float *ent,
               float *lse, float *out2, int64_t ld_out2, const octo_grpo_tail *gt, void *grad_h, int64_t ld_gh,
               int gh_dtype, void *grad_w, int gw_dtype, void *ws, size_t ws_bytes, void *stream,
-              const StepPairs *pm = nullptr) {
+              const StepPairs *pm = nullptr, bool later = false) {
   Common cm;
   int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, n_max, d, V, flags, inv_T,
                         pre, post, use_tanh, cm);
@@ -434,7 +435,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     if (cm.dt == OCTO_F32) return octo_fail(OCTO_EUNSUPPORTED, "head_step_grpo_pairs: fp32 operands");
   }
   if (n_max == 0 && !pm) return OCTO_OK;
-  if (!need_gh && !need_gw && !pm)  // no gradient asked for: the forward with its GRPO tail (its own workspace size)
+  if (!need_gh && !need_gw && !pm && !later)  // no gradient asked for: the forward with its GRPO tail (its own workspace size)
     return head_fwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, count, n_max, d, V, flags, inv_T,
                     pre, post, use_tanh, logp, ent, lse, out2, ld_out2, gt, ws, ws_bytes, stream);
   if (cm.dt == OCTO_F32) {  // fp32: the forward, then the backward
@@ -449,7 +450,12 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
                          ws_bytes, stream);
   }
   StepLayout L;
-  if (!ws || !step_plan_for(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, ws_bytes, L)) {
+  if (later) {
+    if (cm.gather || !later_plan(n_max, d, V, w_dtype, need_gh, L))
+      return octo_fail(OCTO_EUNSUPPORTED, "head_step_later: not for this call");
+    if (!ws || ws_bytes < L.total)
+      return octo_fail(OCTO_EWORKSPACE, "head_step_later: buffer %zu < %zu bytes", ws ? ws_bytes : (size_t)0, L.total);
+  } else if (!ws || !step_plan_for(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, ws_bytes, L)) {
     StepLayout Lmin;
     size_t least = 0;
     for (int q = kBudgetQMin; q <= kBudgetQMax && !least; ++q)
@@ -468,7 +474,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
 
   rc = launch_grpo_count(gt->mask, gt->n_tokens, z, gt->loss, st);  // Z, and the loss zeroed
   if (rc) return rc;
-  const bool grads = need_gh || need_gw;
+  const bool grads = need_gh || need_gw || later;
   float *rowout = (float *)(wsb + L.rowout);
   if (pm && L.passes == 0) {  // no pair row: every flat token's columns are 0
     PairsGrpoArgs pa{};
@@ -692,7 +698,7 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     // grad_W (+)= dz^T . h   (K = this pass's rows)
     const Operand A3 = plain_operand(dz, L.V_pad * esz, L.P, nullptr, 0);
     const Operand B3 = plain_operand(ht, L.P * esz, d, nullptr, 0);
-    if (need_gw) {  // h^T [d, P] of the pass's rows, zero past the count
+    if (need_gw || later) {  // h^T [d, P] of the pass's rows, zero past the count
       const int64_t rows_pad = round_up(rows, TN);
       rc = launch_transpose(idx ? h : (const char *)h + r0 * ldh * cm.hesz, ldh, h_dtype, rowoff ? rscale : nullptr,
                             idx ? idx + r0 : nullptr, count, r0, rows, rows_pad, d, ht, L.P, cm.dt, st);
@@ -907,6 +913,42 @@ int octo_head_step_grpo_pairs(const void *h, int64_t h_rows, int64_t ldh, int h_
   return head_step(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, pair_label, pair_pos, pair_count, n_pairs, d,
                    V, flags, inv_T, pre, post, use_tanh, nullptr, nullptr, lse, nullptr, 2, grpo, grad_h, ld_gh,
                    gh_dtype, grad_w, gw_dtype, ws, ws_bytes, stream, &pm);
+}
+
+int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *bytes) {
+  OCTO_CHECK_ARG(bytes && n_max >= 0 && d > 0 && V > 0, "head_later_bytes: bad arguments");
+  StepLayout L;
+  *bytes = later_plan(n_max, d, V, w_dtype, need_gh != 0, L) ? L.total : 0;
+  return OCTO_OK;
+}
+
+int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
+                         int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
+                         int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
+                         const int64_t *flat_pair, int64_t n_flat, float *out2, int64_t ld_out2,
+                         const octo_grpo_tail *grpo, void *grad_h, int64_t ld_gh, int gh_dtype, void *kept,
+                         size_t kept_bytes, void *stream) {
+  OCTO_CHECK_ARG(!flat_pair || idx, "head_step_later: pair rows without idx");
+  OCTO_CHECK_ARG(n_max > 0, "head_step_later: no rows");
+  const StepPairs pm{flat_pair, n_flat, out2, ld_out2};
+  return head_step(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T,
+                   pre, post, use_tanh, nullptr, nullptr, lse, flat_pair ? nullptr : out2, flat_pair ? 2 : ld_out2, grpo,
+                   grad_h, ld_gh, gh_dtype, nullptr, OCTO_F32, kept, kept_bytes, stream, flat_pair ? &pm : nullptr, true);
+}
+
+int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype, int need_gh,
+                           const float *c, void *grad_w, int gw_dtype, void *stream) {
+  StepLayout L;
+  if (d <= 0 || d % 8 || V <= 0 || !later_plan(n_max, d, V, w_dtype, need_gh != 0, L))
+    return octo_fail(OCTO_EUNSUPPORTED, "head_later_grad_w: not for this call");
+  OCTO_CHECK_ARG(kept && c && grad_w, "head_later_grad_w: null pointer");
+  OCTO_CHECK_ARG(gw_dtype == OCTO_BF16 || gw_dtype == OCTO_F16 || gw_dtype == OCTO_F32, "head_later_grad_w: dtype");
+  const Operand A3 = plain_operand((const char *)kept + L.dz, L.V_pad * 2, L.P, nullptr, 0);
+  const Operand B3 = plain_operand((const char *)kept + L.ht, L.P * 2, d, nullptr, 0);
+  StoreArgs o = grad_w_store(d, 0, n_max, 0, 1, false, nullptr, grad_w, gw_dtype, 0, count);
+  o.alpha = c;
+  TimedLaunch t("gemm_store_grad_w", (hipStream_t)stream);
+  return launch_gemm_store(w_dtype, A3, B3, shape(V, d, n_max, kGroupM, 3, count, 0), o, (hipStream_t)stream, KM_A);
 }
 
 int octo_head_stage_bytes(int64_t n_max, int d, int V, int w_dtype, size_t bytes[2]) {

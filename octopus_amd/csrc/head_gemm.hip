@@ -327,7 +327,7 @@ __device__ __forceinline__ void dz_write(const DzArgs &e, int64_t ma, int64_t m0
 
 // ---- epilogue: plain store -------------------------------------------------------------------
 
-// C = rs[row] x acc (rs NULL: acc) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to OT, value
+// C = rs[row] x acc (rs NULL: acc; x alpha) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to OT, value
 // by value: ragged and unaligned tiles, fp32 output, sums. The accumulators go through the LDS (the ring, free after the
 // mainloop) in two halves of 128 rows, so that a wave stores, adds to or reads 64 neighbours of a row; from the
 // registers it would cover 16 bytes of each of 16 rows (Acc16T), and the fp32 partials of several passes, read and
@@ -343,6 +343,7 @@ __device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::
   static_assert(128 * TN * 4 <= SMEM_RING5 && L::NI == 8, "half a tile of fp32 in the LDS");
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = L::wm(w), wn = L::wn(w);
   typedef __attribute__((address_space(3))) float lds_float;
+  const float alpha = e.alpha ? *e.alpha : 1.f;
   // 16-byte slot c / 4 of row r sits at slot (c / 4) ^ (r & 15): a wave's write, 16 rows of 4 slots, covers all banks
   for (int half = 0; half < 2; ++half) {
     if (half) __syncthreads();  // the first half's reads are done
@@ -360,7 +361,7 @@ __device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::
       const int64_t row = m0 + half * 128 + r;
       OT *crow = (OT *)e.C + row * e.ldc + n0;
       const float *arow = e.addend ? e.addend + row * e.ld_add + n0 : nullptr;
-      const float sc = e.row_scale ? e.row_scale[row] : 1.f;
+      const float sc = e.row_scale ? e.row_scale[row] * alpha : alpha;
 #pragma unroll
       for (int q = 0; q < TN / 64; ++q) {
         const int c = 64 * q + lane;
@@ -390,10 +391,11 @@ __device__ __forceinline__ void store_staged(const typename L::V (&acc)[L::NI][L
                                              int64_t n0, int64_t mvalid, lds_char *smem) {
   typedef typename std::conditional<std::is_same<OT, __bf16>::value, bf16x2, f16x2_t>::type P2;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
+  const float alpha = e.alpha ? *e.alpha : 1.f;
 #pragma unroll
   for (int i = 0; i < L::NI; ++i) {
     const int rr = L::row(wm, i, lane), sw = DzSwz<Acc16N<4>>::at(rr);
-    const float sc = e.row_scale && rr < mvalid ? e.row_scale[m0 + rr] : 1.f;
+    const float sc = e.row_scale && rr < mvalid ? e.row_scale[m0 + rr] * alpha : alpha;
 #pragma unroll
     for (int j = 0; j < L::NJ; ++j) {
       i32x2 p;
@@ -487,7 +489,7 @@ __device__ __forceinline__ void store_pass(const typename L::V (&acc)[L::NI][L::
     p.C = e.part;
     p.addend = nullptr;
     p.accumulate = e.part_accumulate;
-    p.row_scale = nullptr;
+    p.row_scale = p.alpha = nullptr;
     store_any<L, float>(acc, p, m0, n0, mvalid, nvalid, smem);
   }
 }

@@ -128,6 +128,7 @@ struct StoreArgs {
   int part_blocked = 0;
   // row_scale: C's row m takes row_scale[m] x acc (before any addend); the final store only (not the partials)
   const float *row_scale = nullptr;
+  const float *alpha = nullptr;  // all of C times *alpha, the same way
   // split K (grad_h; tile_order.h k_splits): with room for split_cap partial tiles of 256 x 256 fp32 at split, the
   // kernels cut each tile's K into the runs k_splits gives for the tiles the device count leaves, run s of tile (mt,
   // nt) stores its sum at split + ((s tiles + nt mtiles + mt) << 16) in the accumulator's own order (fp32 operands: 256

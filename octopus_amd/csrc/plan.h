@@ -408,6 +408,18 @@ inline bool stage_plan(int64_t n_max, int d, int V, int w_dtype, StageLayout &L)
   return true;
 }
 
+// The step without grad_W, whose operands (dz and the pass's h^T) stay in the workspace for octo_head_later_grad_w: one
+// pass of 16-bit weights within the staging budget. grad_h's partial tiles, one round of the CUs at most, lie behind.
+inline bool later_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, StepLayout &L) {
+  if ((w_dtype != OCTO_BF16 && w_dtype != OCTO_F16) || n_max <= 0) return false;
+  if (!step_plan(n_max, d, V, w_dtype, need_gh, true, false, kStagingBudget, L, false, false) || L.passes != 1) return false;
+  L.split_items = need_gh ? gradh_split(L.P, d, V, true) : 0;
+  if (L.split_items > octo_tiles::kCus) L.split_items = octo_tiles::kCus;
+  L.split = L.total;
+  L.total += L.split_items * kSplitTile;
+  return true;
+}
+
 // Workspace of the step for fp32 operands: the forward's, then the backward's (at the default budget), in turn.
 inline size_t step_fallback_bytes(int64_t n_max, int d, int V, int w_dtype, bool need_gw, bool gather) {
   const size_t f = fwd_layout(n_max, d, V, w_dtype, gather).total;

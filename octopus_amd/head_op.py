@@ -542,12 +542,15 @@ def _stage_setup(ctx, inputs, output):
     ctx.stage = output[2].detach()
     ctx.params = inputs[5:]
     ctx.save_for_backward(rows, labels, idx, count, output[1])
+    ctx.set_materialize_grads(False)  # no zeros the size of the buffer for the gradient it does not have
 
 
 def _stage_backward(ctx, gout, _glse, _gstage):
     rows, labels, idx, count, lse = ctx.saved_tensors
     inv_T, pre, post, use_tanh, labels_via_idx, scatter = ctx.params
     need_rows, need_weight = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
+    if gout is None:  # no loss reads the columns
+        return (_zeros(rows) if need_rows else None, _zeros(ctx.weight) if need_weight else None) + (None,) * 9
     g = _compact_g(gout, idx, count, scatter)
     grad_rows, grad_w = head_bwd_stage(rows, ctx.weight, labels, idx, count, lse, ctx.stage, g, inv_T, pre, post,
                                        use_tanh, labels_via_idx, need_rows, need_weight)
@@ -573,6 +576,124 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
     return out
 
 
+# ---- the GRPO step with its weight gradient made in the backward (octo_head_step_later) ------------------------------
+
+# From this many weights on, and up to this many rows. Scaling a held weight gradient costs a read and a write of it, 264 us
+# at 2^28.5 weights whatever the rows; leaving it to the backward costs a few launches of 5 us and, in proportion to the
+# rows, the tiles of grad_W that ran beside grad_h's in one launch. us a pass, held and left for later: 225 rows at d 2560,
+# V 151,936 1,005 and 772; 1,351 at d 2304, V 64,000 (f16) 1,238 and 1,199; 3,000 at d 2560, V 151,936 6,434 and 6,850.
+_LATER_WEIGHTS = 1 << 25
+_LATER_ROWS = 1536
+
+
+def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows: bool, need_weight: bool) -> int:
+    """The buffer of a step whose weight gradient is left to the backward, 0 where it is not. At most twice as many rows as
+    the hidden width: what is kept, dz, then takes at most twice the bytes of the weight gradient that would be."""
+    if not need_weight or STEP_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not rows.is_cuda:
+        return 0
+    if rows.dim() != 2 or weight.dim() != 2 or weight.numel() < _LATER_WEIGHTS or rows.dtype != weight.dtype:
+        return 0
+    if weight.dtype not in (torch.bfloat16, torch.float16):
+        return 0
+    V, d = weight.shape
+    n = idx.numel() if idx is not None else rows.shape[0]
+    if not 0 < n <= min(_LATER_ROWS, 2 * d) or (idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff):
+        return 0
+    return _lib.later_bytes(n, d, V, _dtype_code(weight), need_rows)
+
+
+@torch.library.custom_op("octohead::head_step_later", mutates_args=(), device_types="cuda")
+def head_step_later(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
+                    flat_pair: Optional[Tensor], inv_T: float, pre: float, post: float, use_tanh: bool,
+                    labels_via_idx: bool, scatter: bool, prox: Optional[Tensor], old: Optional[Tensor], adv: Tensor,
+                    mask: Tensor, eps_lo: float, eps_hi: float, reject_upper: float, need_rows: bool,
+                    nbytes: int) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
+    """head_step_grpo's (or, with flat_pair, head_step_grpo_pairs') (out, loss, grad_rows), the buffer of nbytes that
+    later_grad_w makes grad_weight of, and the row count as the call found it."""
+    rows2, weight2 = _rows2d(rows), _rows2d(weight)
+    labels, idx, flat_pair = _index(labels), _index(idx), _index(flat_pair)
+    n_max = idx.numel() if idx is not None else rows2.shape[0]
+    V, d = weight2.shape
+    dev = rows2.device
+    flags = (_lib.ROWS_VIA_IDX if labels_via_idx else 0) | (_lib.OUT_SCATTER if scatter else 0) | _lib.LSE_PAIR
+    n_out = flat_pair.numel() if flat_pair is not None else rows2.shape[0] if scatter else n_max
+    out = torch.zeros(n_out, 2, dtype=torch.float32, device=dev)
+    lse = torch.empty(n_max, 2, dtype=torch.float32, device=dev)
+    g = torch.empty(n_max, dtype=torch.float32, device=dev)
+    loss = torch.zeros((), dtype=torch.float32, device=dev)
+    grad_rows = _zeros(rows) if need_rows else rows.new_empty(0)
+    kept_count = torch.full((1,), n_max, dtype=torch.int32, device=dev) if count is None \
+        else count.reshape(-1)[:1].to(torch.int32, copy=True)
+    f = lambda t: None if t is None else t.float().contiguous().reshape(-1)  # noqa: E731
+    prox_, old_, adv_, mask_ = f(prox), f(old), f(adv), f(mask)
+    tail = _lib.GrpoTail(_p(prox_), _p(old_), _p(adv_), _p(mask_), adv_.numel(), eps_lo, eps_hi, reject_upper,
+                         _p(g), _p(loss))
+    code = _dtype_code(weight2)
+    kept = _workspace(nbytes, rows2)
+    gh = None
+    if need_rows:  # compact-order rows; scattered into grad_rows below
+        gh = grad_rows if idx is None else torch.empty(n_max, d, dtype=rows2.dtype, device=dev)
+    _lib.call("octo_head_step_later", _p(rows2), rows2.shape[0], rows2.stride(0), code, _p(weight2), weight2.stride(0),
+              code, _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse),
+              _p(flat_pair), n_out, _p(out), 2, ctypes.byref(tail), _p(gh), d, code, _p(kept), kept.numel(),
+              _stream(rows2))
+    if need_rows and idx is not None:
+        _lib.call("octo_rows_scatter", _p(gh), d, code, _p(idx), _p(count), n_max, d, _p(grad_rows),
+                  grad_rows.stride(0), code, 0, _stream(rows2))
+    return out, loss, grad_rows, kept, kept_count
+
+
+@head_step_later.register_fake
+def _(rows, weight, labels, idx, count, flat_pair, inv_T, pre, post, use_tanh, labels_via_idx, scatter, prox, old, adv,
+      mask, eps_lo, eps_hi, reject_upper, need_rows, nbytes):
+    n_max = idx.shape[0] if idx is not None else rows.shape[0]
+    n_out = flat_pair.shape[0] if flat_pair is not None else rows.shape[0] if scatter else n_max
+    return (rows.new_empty(n_out, 2, dtype=torch.float32), rows.new_empty((), dtype=torch.float32),
+            _empty(rows) if need_rows else rows.new_empty(0), rows.new_empty(nbytes, dtype=torch.uint8),
+            rows.new_empty(1, dtype=torch.int32))
+
+
+@torch.library.custom_op("octohead::later_grad_w", mutates_args=(), device_types="cuda")
+def later_grad_w(kept: Tensor, count: Tensor, c: Tensor, n_max: int, d: int, V: int, dtype: torch.dtype,
+                 need_rows: bool) -> Tensor:
+    """grad_weight [V, d] of the loss times c, from head_step_later's buffer."""
+    grad_w = torch.empty(V, d, dtype=dtype, device=kept.device)
+    c = c.float().contiguous()
+    _lib.call("octo_head_later_grad_w", _p(kept), _p(count), n_max, d, V, _DT[dtype], int(need_rows), _p(c), _p(grad_w),
+              _DT[dtype], _stream(kept))
+    return grad_w
+
+
+@later_grad_w.register_fake
+def _(kept, count, c, n_max, d, V, dtype, need_rows):
+    return torch.empty(V, d, dtype=dtype, device=kept.device)
+
+
+def _later_setup(ctx, inputs, output):
+    rows, weight, idx = inputs[0], inputs[1], inputs[3]
+    # held on ctx, not saved, as _step_setup's gradients
+    ctx.held = (output[2].detach(), output[3].detach(), output[4].detach())
+    ctx.sizes = (idx.numel() if idx is not None else rows.shape[0], weight.shape[1], weight.shape[0], weight.dtype)
+    ctx.need_rows = inputs[-2]
+    ctx.n_inputs = len(inputs)
+    ctx.set_materialize_grads(False)
+
+
+def _later_backward(ctx, _gout, gloss, _ggr, _gkept, _gcount):
+    grad_rows, kept, count = ctx.held
+    n_max, d, V, dtype = ctx.sizes
+    gr = gw = None
+    if ctx.need_rows and ctx.needs_input_grad[0]:
+        gr = torch.zeros_like(grad_rows) if gloss is None else scaled(grad_rows, gloss)
+    if ctx.needs_input_grad[1]:
+        gw = torch.zeros(V, d, dtype=dtype, device=kept.device) if gloss is None \
+            else later_grad_w(kept, count, gloss, n_max, d, V, dtype, ctx.need_rows)
+    return (gr, gw) + (None,) * (ctx.n_inputs - 2)
+
+
+torch.library.register_autograd("octohead::head_step_later", _later_backward, setup_context=_later_setup)
+
+
 def fused_grpo_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float, adv: Tensor, mask: Tensor, *,
                     prox: Optional[Tensor] = None, old: Optional[Tensor] = None, post: Post = Post(),
                     idx: Optional[Tensor] = None, count: Optional[Tensor] = None, labels_via_idx: bool = False,
@@ -580,14 +701,22 @@ def fused_grpo_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: f
                     eps_hi: float = 0.28, reject_upper: float = 5.0) -> tuple[Tensor, Tensor]:
     """(loss, out): the GRPO objective (grpo_loss's, on the head's logprobs) and fused_head's [n, 2] (logprob,
     entropy) columns, from one octo_head_step_grpo call that also computes the loss's gradients with respect to rows
-    and weight (each when it requires grad and grad mode is on); loss.backward() then only scales them. The columns
+    and weight (each when it requires grad and grad mode is on); loss.backward() then only scales them, or, for a short
+    call, makes the weight's from the operands kept (head_step_later). The columns
     carry no gradient: for losses other than this objective, use fused_head. prox, old, adv, mask are per flat
-    token (row of `rows`), as grpo_loss takes them. The gradients are held from this call to the backward."""
+    token (row of `rows`), as grpo_loss takes them. The gradients or operands are held from this call to the backward."""
     if temperature <= 0:
         raise ValueError("temperature must be positive")
     grad_on = torch.is_grad_enabled()
     need_rows = grad_on and rows.requires_grad
     need_weight = grad_on and weight.requires_grad
+    nbytes = _later_bytes(rows, weight, idx, need_rows, need_weight)
+    if nbytes:
+        out, loss, _gr, _kept, _count = head_step_later(
+            rows, weight, labels, idx, count, None, 1.0 / float(temperature), float(post.pre), float(post.post),
+            bool(post.tanh), labels_via_idx, scatter, prox, old, adv, mask, float(eps_lo), float(eps_hi),
+            float(reject_upper), need_rows, nbytes)
+        return loss, out.detach()
     out, _lse, _g, loss, _gr, _gw = head_step_grpo(
         rows, weight, w_scale, labels, idx, count, 1.0 / float(temperature), float(post.pre), float(post.post),
         bool(post.tanh), labels_via_idx, scatter, prox, old, adv, mask, float(eps_lo), float(eps_hi),
@@ -610,6 +739,13 @@ def fused_grpo_tree_head(hidden: Tensor, weight: Tensor, meta, temperature: floa
     grad_on = torch.is_grad_enabled()
     need_rows = grad_on and hidden.requires_grad
     need_weight = grad_on and weight.requires_grad
+    nbytes = _later_bytes(rows, weight, meta.pair_pos, need_rows, need_weight)
+    if nbytes:
+        out, loss, _gr, _kept, _count = head_step_later(
+            rows, weight, meta.pair_label, meta.pair_pos, meta.pair_count, meta.flat_pair, 1.0 / float(temperature),
+            float(post.pre), float(post.post), bool(post.tanh), False, False, prox, old, adv, mask, float(eps_lo),
+            float(eps_hi), float(reject_upper), need_rows, nbytes)
+        return loss, out.detach().unsqueeze(0)
     out, _lse, _g, loss, _gr, _gw = head_step_grpo_pairs(
         rows, weight, w_scale, meta.pair_label, meta.pair_pos, meta.pair_count, meta.flat_pair,
         1.0 / float(temperature), float(post.pre), float(post.post), bool(post.tanh), prox, old, adv, mask,
