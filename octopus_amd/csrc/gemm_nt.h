@@ -4,8 +4,8 @@
 //
 // One workgroup computes a 256 x 256 tile of C. The 16-bit loop runs 512 threads = 8 wave64s, two per SIMD, sat
 // 2 x 4, each owning a 128 x 64 sub-tile as 8 x 4 blocks of v_mfma_f32_16x16x32_{bf16,f16} (Acc16N<4>, 128
-// accumulation registers): while one wave of a SIMD waits on a stage the other issues MFMAs. The fp32 loop runs 4
-// waves, 2 x 2, each 128 x 128 as 4 x 4 blocks of v_mfma_f32_32x32x2_f32 (Acc32). Under the part's power limit the
+// accumulation registers): while one wave of a SIMD waits on a stage the other issues MFMAs. fp32 operands have a loop of
+// their own (gemm_f32.hip). Under the part's power limit the
 // 16x16x32 form sustains 12% more bf16 FLOP/s than the 32x32x16 one on random operands (2.10 against 1.88 PFLOP/s,
 // a register-only loop on every SIMD), and each MFMA streams fewer accumulator bytes per FLOP.
 //
@@ -105,7 +105,7 @@ __device__ __forceinline__ void lds_dma16(__amdgpu_buffer_rsrc_t rs, uint32_t vo
 // ---- full-line mainloop: K = 64 per stage, a 5-slot ring ------------------------------------------
 //
 // For 16-bit types. A stage holds K = 64 (128 bytes of every operand row), so each row fetch of a K-contiguous
-// operand is one whole 128-byte cache line; with 64-byte rows (the 4-stage ring above) every line is requested
+// operand is one whole 128-byte cache line; with 64-byte rows every line is requested
 // twice, once per half, which doubles the L1 -> L2 requests and stalls the address unit on the L1.
 //
 // A stage is two 32 KB slices (A, B). The LDS holds five slices, 2.5 stages: stage j's A slice sits in slot
@@ -259,8 +259,7 @@ struct OpColsN {
   }
 };
 
-// The 16-bit GEMMs (bf16 / f16 operands; fp8 weights are widened to bf16 before the GEMM) run the ring loop, fp32
-// the 4-stage one.
+// What runs the ring loop: bf16 and f16 operands (fp8 weights are widened to bf16 before the GEMM).
 __host__ __device__ constexpr bool ring5_ok(int dt) { return dt == OCTO_BF16 || dt == OCTO_F16; }
 
 // MFMA order within a K-step: A block i fixed for NBB consecutive MFMAs, B blocks walked forward for even i and

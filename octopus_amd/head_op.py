@@ -429,7 +429,9 @@ torch.library.register_autograd("octohead::head_fwd", _head_backward, setup_cont
 
 _STAGE_BYTES = 2 << 30  # of the kept exponentials, padded to 256 rows and columns: the backward's own staging budget
 # fused_head keeps them from this many multiply-adds of the logits on (n d V). The recompute they save takes 1.5 ns per
-# 2^20 of them; the wider store and the pass that makes dz cost a small call some 10 us, 2^33 multiply-adds' worth.
+# 2^20 of them; the wider store and the pass that makes dz cost a small call some 10 us, 2^33 multiply-adds' worth. And
+# for at most twice as many rows as the hidden width: what is kept until the backward then takes at most twice the bytes
+# of the weight's gradient, which a training step has room for anyway; beyond, the head keeps no [n, V] between calls.
 _STAGE_WORK = 1 << 33
 
 
@@ -445,7 +447,7 @@ def _stage_numel(n_max: int, V: int) -> int:
 def _stages(rows: Tensor, weight: Tensor, idx: Optional[Tensor], scale: float) -> bool:
     """Whether fused_head keeps the exponentials: a gradient is wanted, octo_head_fwd_stage takes the call and the
     recompute would cost more. Not while a compiler traces (a guard on the sizes), nor with a backward workspace set."""
-    if BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not torch.is_grad_enabled():
+    if not torch.is_grad_enabled() or BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling():
         return False
     if not (rows.requires_grad or weight.requires_grad) or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
         return False
@@ -453,8 +455,8 @@ def _stages(rows: Tensor, weight: Tensor, idx: Optional[Tensor], scale: float) -
         return False
     n = idx.numel() if idx is not None else rows.shape[0]
     V, d = weight.shape
-    # rows through idx lie below 2 GiB, as they are or (twice the numel covers any stride _rows2d keeps) copied
-    return (0 < n <= 32768 and _pad256(n) * _pad256(V) * 2 <= _STAGE_BYTES and n * d * V >= _STAGE_WORK
+    # rows through idx lie below 2 GiB, as they are or copied (_rows2d)
+    return (0 < n <= min(32768, 2 * d) and _pad256(n) * _pad256(V) * 2 <= _STAGE_BYTES and n * d * V >= _STAGE_WORK
             and not (idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff))
 
 

@@ -3,7 +3,7 @@ the forward, over what both take."""
 import pytest
 import torch
 
-from octopus_amd import _lib, head_op
+from octopus_amd import head_op
 from octopus_amd.rl.prefix_tree import TreeMeta
 
 pytestmark = pytest.mark.gpu
@@ -92,9 +92,3 @@ def test_later_weight_gradient_of_a_tree(monkeypatch):
     assert abs(a[0] - b[0]) <= 1e-6 * max(1.0, abs(b[0])) and torch.equal(a[1], b[1])
     _close(a[2], b[2], torch.bfloat16)
     _close(a[3], b[3], torch.bfloat16)
-
-
-def test_what_is_not_left_for_later():
-    assert _lib.later_bytes(300, 512, 5003, _lib.FP8E4M3, True) == _lib.later_bytes(300, 512, 5003, _lib.F32, True) == 0
-    assert _lib.later_bytes(32768, 2560, 151936, _lib.BF16, True) == 0  # several passes
-    assert _lib.later_bytes(4608, 2560, 151936, _lib.BF16, True) > 4608 * 151936 * 2
