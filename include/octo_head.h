@@ -177,22 +177,23 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype,
                   void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w, int gw_dtype,
                   void *ws, size_t ws_bytes, void *stream);
 
-/* octo_head_fwd and octo_head_bwd without the logits' recompute: the forward leaves every element's exponential in a
- * buffer that the caller keeps, and the backward makes dz of it (the buffer is left as it was, for another backward).
- * Arguments as theirs; bf16 operands, at most 32,768 rows whose exponentials, padded to 256 rows and columns, take at
- * most 2 GiB (the budget octo_head_bwd stages within), hidden rows through idx below 2 GiB. octo_head_stage_bytes gives
- * {buffer, octo_head_bwd_stage's workspace}, both 0 for a call that is not staged (OCTO_EUNSUPPORTED from the others).
+/* octo_head_fwd and octo_head_bwd without the logits' recompute for the first logit_rows compact rows (a multiple of 256,
+ * padding included): the forward leaves their fp32 logits (tanh(pre z) with the soft-cap) in logits [logit_rows,
+ * ld_logits], ld_logits >= V rounded up to 256, a multiple of 4, 16-byte aligned; the backward reads dz off them and leaves
+ * them as they were, for another backward. Arguments, workspaces and results (to the bit) as theirs; bf16 operands. The
+ * logits are those of the forward's weights: a caller that changes the weights in between calls octo_head_bwd.
  * No counterpart in the reference, which keeps or recomputes the logits. */
-int octo_head_stage_bytes(int64_t n_max, int d, int V, int w_dtype, size_t bytes[2]);
-int octo_head_fwd_stage(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
-                        int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
-                        int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
-                        float *out2, int64_t ld_out2, void *stage, size_t stage_bytes, void *stream);
-int octo_head_bwd_stage(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
-                        int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
-                        int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, const float *lse,
-                        const float *g, const void *stage, void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w,
-                        int gw_dtype, void *ws, size_t ws_bytes, void *stream);
+int octo_head_fwd_logits(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
+                         int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
+                         int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
+                         float *out2, int64_t ld_out2, float *logits, int64_t ld_logits, int64_t logit_rows, void *ws,
+                         size_t ws_bytes, void *stream);
+int octo_head_bwd_logits(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
+                         int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
+                         int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, const float *lse,
+                         const float *g, const float *logits, int64_t ld_logits, int64_t logit_rows, void *grad_h,
+                         int64_t ld_gh, int gh_dtype, void *grad_w, int gw_dtype, void *ws, size_t ws_bytes,
+                         void *stream);
 
 /* _head_columns on materialised logits [n, ld] (dtype BF16, F16 or F32):
  * out2[r] = {log_softmax(s)[y_r], entropy}, s = logits * inv_T; the row state saved (may be NULL) as two floats

@@ -64,11 +64,10 @@ SIGNATURES = {
     "octo_head_step_later": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
                              _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail), _p, _i64, _i32, _p, _sz, _p],
     "octo_head_later_grad_w": [_p, _p, _i64, _i32, _i32, _i32, _i32, _p, _p, _i32, _p],
-    "octo_head_stage_bytes": [_i64, _i32, _i32, _i32, ctypes.POINTER(_sz)],
-    "octo_head_fwd_stage": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
-                            _f32, _i32, _p, _p, _i64, _p, _sz, _p],
-    "octo_head_bwd_stage": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
-                            _f32, _i32, _p, _p, _p, _p, _i64, _i32, _p, _i32, _p, _sz, _p],
+    "octo_head_fwd_logits": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
+                             _f32, _i32, _p, _p, _i64, _p, _i64, _i64, _p, _sz, _p],
+    "octo_head_bwd_logits": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
+                             _f32, _i32, _p, _p, _p, _i64, _i64, _p, _i64, _i32, _p, _i32, _p, _sz, _p],
     "octo_columns_fwd": [_p, _i64, _i32, _p, _i64, _i32, _f32, _p, _p, _p],
     "octo_columns_bwd": [_p, _i64, _i32, _p, _i64, _i32, _f32, _p, _p, _p, _i64, _p],
     "octo_pairs_expand": [_p, _i64, _i32, _p, _i64, _p, _p],
@@ -149,13 +148,6 @@ def later_bytes(n_max: int, d: int, V: int, w_dtype: int, need_gh: bool) -> int:
     out = _sz(0)
     call("octo_head_later_bytes", n_max, d, V, w_dtype, int(need_gh), ctypes.byref(out))
     return out.value
-
-
-def stage_bytes(n_max: int, d: int, V: int, w_dtype: int) -> tuple[int, int]:
-    """(octo_head_fwd_stage's buffer, octo_head_bwd_stage's workspace); zeros for a call that is not staged."""
-    out = (_sz * 2)()
-    call("octo_head_stage_bytes", n_max, d, V, w_dtype, out)
-    return tuple(out)
 
 
 def timing_read(kernel: str) -> tuple[int, float]:

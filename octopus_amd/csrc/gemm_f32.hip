@@ -490,7 +490,7 @@ static dim3 xgrid(const GemmShape &s) { return dim3((unsigned)tile_grid(s.mtiles
 
 int launch_gemm_stats_f32(bool tanh, const Operand &A, const Operand &B, const GemmShape &s0, const StatsArgs &e,
                           hipStream_t st) {
-  if (e.ex) return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: exponentials of fp32 operands");
+  if (e.ex || e.z) return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: exponentials or kept logits of fp32 operands");
   const GemmShape s = xshape(s0);
   if (tanh) hipLaunchKernelGGL(gemm_stats_x_kernel<true>, xgrid(s), dim3(XTHREADS), 0, st, A, B, s, e);
   else hipLaunchKernelGGL(gemm_stats_x_kernel<false>, xgrid(s), dim3(XTHREADS), 0, st, A, B, s, e);

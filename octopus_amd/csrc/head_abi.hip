@@ -314,18 +314,19 @@ MergeArgs merge_args(const f32x4 *part, int64_t mtiles, const void *h, int64_t l
   return m;
 }
 
-// What octo_head_fwd_stage keeps besides the forward's workspace: the exponentials [P, ldx] f16 and the label entries.
+// The logits that octo_head_fwd_logits leaves for octo_head_bwd_logits: those of the first `rows` compact rows.
 struct Kept {
-  void *ex;
-  int64_t ldx;
-  float *hit;
+  float *z = nullptr;
+  int64_t ld = 0, rows = 0;
+  Kept() = default;
+  Kept(const float *z_, int64_t ld_, int64_t rows_) : z(const_cast<float *>(z_)), ld(ld_), rows(rows_) {}
 };
 
 int head_fwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
              const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
              int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *logp, float *ent,
              float *lse, float *out2, int64_t ld_out2, const octo_grpo_tail *gt, void *ws, size_t ws_bytes,
-             void *stream, bool timed = true, const Kept *kept = nullptr) {
+             void *stream, bool timed = true, const Kept &kept = Kept()) {
   Common cm;
   int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, n_max, d, V, flags, inv_T,
                         pre, post, use_tanh, cm);
@@ -360,9 +361,10 @@ int head_fwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void
   e.wscale = w_scale;
   e.c = cm.c;
   e.pre = cm.pre;
-  if (kept) {
-    e.ex = kept->ex;
-    e.ldx = kept->ldx;
+  if (kept.rows) {
+    e.z = kept.z;
+    e.ldx = kept.ld;
+    e.z_rows = kept.rows;
   }
   for (int64_t c = 0; c < L.chunks; ++c) {  // one chunk covering V, except for fp8 weights (widened chunk by chunk)
     e.v0 = c * L.Vc;
@@ -377,12 +379,8 @@ int head_fwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void
     if (rc) return rc;
   }
 
-  MergeArgs m = merge_args(e.part, L.mtiles, h, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, count,
+  const MergeArgs m = merge_args(e.part, L.mtiles, h, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, count,
                                  n_max, d, V, flags, inv_T, pre, post, use_tanh, logp, ent, lse, out2, ld_out2, gt, z);
-  if (kept) {
-    m.c = cm.c;
-    m.hit = kept->hit;
-  }
   return launch_merge(m, st);
 }
 
@@ -951,131 +949,11 @@ int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max
   return launch_gemm_store(w_dtype, A3, B3, shape(V, d, n_max, kGroupM, 3, count, 0), o, (hipStream_t)stream, KM_A);
 }
 
-int octo_head_stage_bytes(int64_t n_max, int d, int V, int w_dtype, size_t bytes[2]) {
-  OCTO_CHECK_ARG(bytes && n_max >= 0 && d > 0 && V > 0, "head_stage_bytes: bad arguments");
-  StageLayout L;
-  const bool ok = stage_plan(n_max, d, V, w_dtype, L);
-  bytes[0] = ok ? L.total : 0;
-  bytes[1] = ok ? L.bwd_total : 0;
-  return OCTO_OK;
-}
-
-int octo_head_fwd_stage(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
-                        int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
-                        int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
-                        float *out2, int64_t ld_out2, void *stage, size_t stage_bytes, void *stream) {
-  Common cm;
-  int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, n_max, d, V, flags, inv_T, pre,
-                        post, use_tanh, cm);
-  if (rc) return rc;
-  StageLayout L;
-  if (cm.gather || !stage_plan(n_max, d, V, w_dtype, L))
-    return octo_fail(OCTO_EUNSUPPORTED, "head_fwd_stage: this call is not staged");
-  OCTO_CHECK_ARG(lse && stage && (uintptr_t)stage % 16 == 0, "head_fwd_stage: null lse, null or misaligned buffer");
-  if (stage_bytes < L.total)
-    return octo_fail(OCTO_EWORKSPACE, "head_fwd_stage: buffer %zu < %zu bytes", stage_bytes, L.total);
-  char *base = (char *)stage;
-  const Kept kept{base + L.ex, L.V_pad, (float *)(base + L.hit)};
-  return head_fwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T, pre,
-                  post, use_tanh, nullptr, nullptr, lse, out2, ld_out2, nullptr, base + L.fwd, L.total - L.fwd, stream,
-                  true, &kept);
-}
-
-int octo_head_bwd_stage(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
-                        int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
-                        int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, const float *lse,
-                        const float *g, const void *stage, void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w,
-                        int gw_dtype, void *ws, size_t ws_bytes, void *stream) {
-  Common cm;
-  int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, n_max, d, V, flags, inv_T, pre,
-                        post, use_tanh, cm);
-  if (rc) return rc;
-  StageLayout L;
-  if (cm.gather || !stage_plan(n_max, d, V, w_dtype, L))
-    return octo_fail(OCTO_EUNSUPPORTED, "head_bwd_stage: this call is not staged");
-  OCTO_CHECK_ARG(lse && g && stage, "head_bwd_stage: null lse, g or buffer");
-  OCTO_CHECK_ARG(!grad_h || ((gh_dtype == OCTO_BF16 || gh_dtype == OCTO_F16 || gh_dtype == OCTO_F32) && ld_gh >= d),
-                 "head_bwd_stage: grad_h dtype or stride");
-  OCTO_CHECK_ARG(!grad_w || gw_dtype == OCTO_BF16 || gw_dtype == OCTO_F16 || gw_dtype == OCTO_F32,
-                 "head_bwd_stage: grad_w dtype");
-  if (!grad_h && !grad_w) return OCTO_OK;
-  if (!ws || ws_bytes < L.bwd_total)
-    return octo_fail(OCTO_EWORKSPACE, "head_bwd_stage: workspace %zu < %zu bytes", ws ? ws_bytes : (size_t)0, L.bwd_total);
-  hipStream_t st = (hipStream_t)stream;
-  const char *base = (const char *)stage;
-  char *wsb = (char *)ws;
-  const FwdLayout F = fwd_layout(n_max, d, V, w_dtype, false);
-
-  DzScaleArgs sa;  // dz = g (onehot - p) / T x post'(z) from the exponentials, beside them
-  sa.dz = wsb + L.dz;
-  sa.ex = base + L.ex;
-  sa.ld = sa.V_pad = L.V_pad;
-  sa.dtype = cm.dt;
-  sa.part = (const f32x4 *)(base + L.fwd + F.part);
-  sa.mtiles = F.mtiles;
-  sa.lse = lse;
-  sa.lse_pair = (flags & OCTO_LSE_PAIR) != 0;
-  sa.g = g;
-  sa.gmul = cm.gmul;
-  sa.wscale = nullptr;
-  sa.labels = labels;
-  sa.label_idx = (flags & OCTO_ROWS_VIA_IDX) ? idx : nullptr;
-  sa.hit = (const float *)(base + L.hit);
-  sa.count = count;
-  sa.r0 = 0;
-  sa.rows = L.P;
-  sa.n_max = n_max;
-  sa.V = V;
-  {
-    TimedLaunch t("dz_scale", st);
-    rc = launch_dz_scale(sa, st);
-  }
-  if (rc) return rc;
-
-  const bool wk = gh_reads_w(d, V, w_dtype);
-  const Operand Aw = weight_operand(w, ldw, cm, V);
-  if (grad_h && !wk) {  // W^T [d, V_pad], zero past V
-    rc = launch_transpose(w, ldw, cm.dt, nullptr, nullptr, nullptr, 0, V, L.V_pad, d, wsb + L.wt, L.V_pad, cm.dt, st);
-    if (rc) return rc;
-  }
-  if (grad_w) {  // h^T [d, P], zero past the count
-    rc = launch_transpose(h, ldh, h_dtype, nullptr, idx, count, 0, n_max, L.P, d, wsb + L.ht, L.P, cm.dt, st);
-    if (rc) return rc;
-  }
-  const Operand A2 = plain_operand(wsb + L.dz, L.V_pad * 2, n_max, count, 0);
-  const Operand B2 = wk ? plain_operand(w, Aw.ld, d, nullptr, 0) : plain_operand(wsb + L.wt, L.V_pad * 2, d, nullptr, 0);
-  const GemmShape s2 = shape(n_max, d, wk ? V : L.V_pad, kGroupM, 1, count, 0);
-  StoreArgs o2;
-  o2.C = grad_h;
-  o2.ldc = ld_gh;
-  o2.dtype = gh_dtype;
-  if (L.split_items) {
-    o2.split = (float *)(wsb + L.split);
-    o2.split_cap = (int)L.split_items;
-    o2.split_alone = !grad_w;
-  }
-  const Operand A3 = plain_operand(wsb + L.dz, L.V_pad * 2, L.P, nullptr, 0);
-  const Operand B3 = plain_operand(wsb + L.ht, L.P * 2, d, nullptr, 0);
-  const GemmShape s3 = shape(V, d, n_max, kGroupM, 3, count, 0);
-  if (grad_h && grad_w) {
-    const StoreArgs o3 = grad_w_store(d, 0, n_max, 0, 1, false, nullptr, grad_w, gw_dtype, 0, count);
-    TimedLaunch t("gemm_grads", st);
-    rc = launch_gemm_grads(cm.dt, A2, B2, s2, o2, wk, A3, B3, s3, o3, st);
-  } else if (grad_h) {
-    TimedLaunch t("gemm_store_grad_h", st);
-    rc = launch_gemm_store(cm.dt, A2, B2, s2, o2, st, wk ? KM_B : KM_NONE);
-  } else {
-    rc = grad_w_pass(cm.dt, A3, KM_A, B3, V, d, 0, n_max, 0, 1, false, nullptr, grad_w, gw_dtype, 0, count, st);
-  }
-  if (!rc && grad_h) rc = launch_split_sum(s2, o2, false, st);
-  return rc;
-}
-
-int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
-                  const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count,
-                  int64_t n_max, int d, int V, int flags, float inv_T, float pre, float post, int use_tanh,
-                  const float *lse, const float *g, void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w,
-                  int gw_dtype, void *ws, size_t ws_bytes, void *stream) {
+static int head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
+                    const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count,
+                    int64_t n_max, int d, int V, int flags, float inv_T, float pre, float post, int use_tanh,
+                    const float *lse, const float *g, void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w,
+                    int gw_dtype, void *ws, size_t ws_bytes, void *stream, const Kept &kept = Kept()) {
   Common cm;
   int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, n_max, d, V, flags, inv_T,
                         pre, post, use_tanh, cm);
@@ -1186,9 +1064,41 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
       const Operand Aw = gemm_weight(w, ldw, cm, v0, vc, d, wsb + L.wide, st, rc);
       if (rc) return rc;
       e.v0 = v0;
-      {
+      const int64_t kr = kept.rows <= r0 ? 0 : (kept.rows - r0 < L.P ? kept.rows - r0 : L.P);  // of the pass, with logits
+      if (kr) {
+        DzLogitsArgs za{};
+        za.dz = dza;
+        za.ld = L.Vc;
+        za.z = kept.z + r0 * kept.ld;
+        za.ldz = kept.ld;
+        za.v0 = v0;
+        za.cols = vc_pad;
+        za.V = V;
+        za.lse = lse;
+        za.lse_pair = e.lse_pair;
+        za.g = g;
+        za.gmul = cm.gmul;
+        za.c = cm.c;
+        za.use_tanh = use_tanh;
+        za.labels = labels;
+        za.label_idx = e.label_idx;
+        za.hit = e.hit;
+        za.count = count;
+        za.r0 = r0;
+        za.rows = kr;
+        za.n_max = n_max;
+        TimedLaunch t("dz_logits", st);
+        rc = launch_dz_logits(za, st);
+      }
+      if (rc) return rc;
+      if (kr < rows) {  // the rest of the rows
+        DzArgs er = e;
+        er.dzA = (char *)dza + kr * L.Vc * esz;
+        er.row_off = r0 + kr;
+        if (e.hit) er.hit = e.hit + kr;
+        const Operand Br = kr ? hidden_operand(h, ldh, idx, count, r0 + kr, rows - kr, cm, gathered, d) : Bh;
         TimedLaunch t("gemm_dz", st);
-        rc = launch_gemm_dz(cm.dt, cm.fp8, use_tanh != 0, Aw, Bh, shape(vc, rows, d, kGroupM, 2, count, r0), e, st);
+        rc = launch_gemm_dz(cm.dt, cm.fp8, use_tanh != 0, Aw, Br, shape(vc, rows - kr, d, kGroupM, 2, count, r0 + kr), er, st);
       }
       if (rc) return rc;
 
@@ -1238,6 +1148,50 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const
     }
   }
   return OCTO_OK;
+}
+
+// The kept logits' arguments: bf16, whole tiles of rows.
+static int check_kept(const float *logits, int64_t ld, int64_t rows, int V, int w_dtype) {
+  OCTO_CHECK_ARG(rows >= 0 && rows % TN == 0, "head logits: %lld rows", (long long)rows);
+  if (rows == 0) return OCTO_OK;
+  if (w_dtype != OCTO_BF16) return octo_fail(OCTO_EUNSUPPORTED, "head logits: dtype %d", w_dtype);
+  OCTO_CHECK_ARG(logits && (uintptr_t)logits % 16 == 0, "head logits: null or misaligned");
+  OCTO_CHECK_ARG(ld % 4 == 0 && ld >= round_up(V, TM), "head logits: row stride %lld", (long long)ld);
+  return OCTO_OK;
+}
+
+int octo_head_fwd_logits(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
+                         int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
+                         int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
+                         float *out2, int64_t ld_out2, float *logits, int64_t ld_logits, int64_t logit_rows, void *ws,
+                         size_t ws_bytes, void *stream) {
+  const int rc = check_kept(logits, ld_logits, logit_rows, V, w_dtype);
+  if (rc) return rc;
+  return head_fwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T, pre,
+                  post, use_tanh, nullptr, nullptr, lse, out2, ld_out2, nullptr, ws, ws_bytes, stream, true,
+                  Kept{logits, ld_logits, logit_rows});
+}
+
+int octo_head_bwd_logits(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
+                         int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
+                         int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, const float *lse,
+                         const float *g, const float *logits, int64_t ld_logits, int64_t logit_rows, void *grad_h,
+                         int64_t ld_gh, int gh_dtype, void *grad_w, int gw_dtype, void *ws, size_t ws_bytes,
+                         void *stream) {
+  const int rc = check_kept(logits, ld_logits, logit_rows, V, w_dtype);
+  if (rc) return rc;
+  return head_bwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T, pre,
+                  post, use_tanh, lse, g, grad_h, ld_gh, gh_dtype, grad_w, gw_dtype, ws, ws_bytes, stream,
+                  Kept{logits, ld_logits, logit_rows});
+}
+
+int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
+                  const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count,
+                  int64_t n_max, int d, int V, int flags, float inv_T, float pre, float post, int use_tanh,
+                  const float *lse, const float *g, void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w,
+                  int gw_dtype, void *ws, size_t ws_bytes, void *stream) {
+  return head_bwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, count, n_max, d, V, flags, inv_T, pre,
+                  post, use_tanh, lse, g, grad_h, ld_gh, gh_dtype, grad_w, gw_dtype, ws, ws_bytes, stream);
 }
 
 }  // extern "C"

@@ -608,13 +608,27 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
   }
 }
 
+// The tile's accumulators as they are (StatsArgs::z): a lane's 4 vocabulary rows are 16 bytes of its token's row.
+template <class L>
+__device__ __forceinline__ void store_logits(const typename L::V (&acc)[L::NI][L::NJ], float *z, int64_t ldz,
+                                             int64_t nvalid, int wm, int wn, int lane) {
+#pragma unroll
+  for (int j = 0; j < L::NJ; ++j) {
+    const int t = L::col(wn, j, lane);
+    if (t >= nvalid) continue;
+    float *row = z + t * ldz;
+#pragma unroll
+    for (int i = 0; i < L::NI; ++i) *(f32x4 *)(row + L::row(wm, i, 0, lane)) = acc[i][j];
+  }
+}
+
 // The logits-shaped GEMMs on the 8-wave loop (16-bit operands): 512 threads, two waves per SIMD, each 128 x 64, with
 // the split stage barrier. Same box, 24,576 rows, d 2560, V 151,936 (against the 4-wave loop): gemm_stats 14.3
 // against 15.1 ms, gemm_dz 15.3 against 16.5 ms; without the split barrier gemm_dz was 0.4 ms slower than the 4-wave
 // loop.
 // EX: also store the exponentials (StatsArgs::ex) through the LDS staging tile, as gemm_dz8 stores dz; the per-wave
 // statistics then sit past that tile. EX 1: f16 relative to each half tile's maximum; EX 2: bf16 relative to each
-// token's offset (StatsArgs::xoff).
+// token's offset (StatsArgs::xoff). EX 3: the fp32 accumulators of the first tokens (StatsArgs::z).
 template <int DT, bool A_FP8, bool TANH, int EX>
 __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_stats8_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
   static_assert(ring5_ok(DT), "16-bit operands");
@@ -628,7 +642,8 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
   const int64_t nvalid = min(dev_count(s.count, s.count_off + n0, s.N - n0), (int64_t)TN);  // this tile's tokens
   if (nvalid <= 0) return;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = L::wm(w), wn = L::wn(w);
-  lds_f32x4 *red = (lds_f32x4 *)(smem + (EX ? 256 * 512 : 0));
+  constexpr int EXM = EX == 3 ? 0 : EX;  // what goes through the staging tile
+  lds_f32x4 *red = (lds_f32x4 *)(smem + (EXM ? 256 * 512 : 0));
   f32x4 acc[8][4];
   mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true>(A, B, m0, n0, s.K, smem, acc);
   const int64_t ma = e.v0 + m0;  // first vocabulary row of the tile
@@ -648,9 +663,12 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
     __syncthreads();
   }
   pre_transform<L, A_FP8, TANH>(acc, wm, lane, e.pre, wsl);
+  if constexpr (EX == 3) {
+    if (n0 < e.z_rows) store_logits<L>(acc, e.z + n0 * e.ldx + ma, e.ldx, nvalid, wm, wn, lane);
+  }
   const float *xo = EX == 2 ? e.xoff + n0 : nullptr;
-  if (ma + TM > e.V) stats_cols<L, true, EX, TANH, A_FP8>(acc, ma, wm, wn, lane, e.V, e.c, red, smem, nvalid, xo, wsl);
-  else stats_cols<L, false, EX, TANH, A_FP8>(acc, ma, wm, wn, lane, e.V, e.c, red, smem, nvalid, xo, wsl);
+  if (ma + TM > e.V) stats_cols<L, true, EXM, TANH, A_FP8>(acc, ma, wm, wn, lane, e.V, e.c, red, smem, nvalid, xo, wsl);
+  else stats_cols<L, false, EXM, TANH, A_FP8>(acc, ma, wm, wn, lane, e.V, e.c, red, smem, nvalid, xo, wsl);
   __syncthreads();  // per-wave statistics (and the staging tile) written
   const int t = threadIdx.x;
   if (t < nvalid) {  // (m_a, S, U, m_b): S and U relative to max(m_a, m_b), the halves' maxima kept
@@ -661,7 +679,7 @@ __global__ __launch_bounds__(2 * NTHREADS, 1) __attribute__((amdgpu_waves_per_eu
     o[0] = a[0]; o[1] = r.S; o[2] = r.U; o[3] = b[0];
     e.part[(n0 + t) * e.mtiles + e.v0 / TM + mt] = o;
   }
-  if constexpr (EX)
+  if constexpr (EXM != 0)
     lds_tile_to_global<2 * NTHREADS>(smem, (char *)e.ex + (n0 * e.ldx + ma) * 2, e.ldx * 2,
                                      [](int row) { return DzSwz<L>::at(row); });
 }
@@ -703,7 +721,12 @@ static inline int64_t split_grid(const GemmShape &s, const StoreArgs &e) {
 
 template <int DT, bool F8, bool TH>
 static int go_stats(const Operand &A, const Operand &B, const GemmShape &s, const StatsArgs &e, hipStream_t st) {
-  if (e.ex && e.xoff) {
+  if (e.z) {
+    if constexpr (DT == OCTO_BF16 && !F8)
+      hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 3>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
+    else
+      return octo_fail(OCTO_EUNSUPPORTED, "gemm_stats: kept logits need bf16 operands");
+  } else if (e.ex && e.xoff) {
     if constexpr (DT == OCTO_BF16)
       hipLaunchKernelGGL((gemm_stats8_kernel<DT, F8, TH, 2>), grid_of(s), dim3(2 * NTHREADS), 0, st, A, B, s, e);
     else

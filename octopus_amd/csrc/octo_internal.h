@@ -41,6 +41,10 @@ struct StatsArgs {
   void *ex = nullptr;
   int64_t ldx = 0;
   const float *xoff = nullptr;  // per-token base-2 offsets of the stored exponentials (tokens of this GEMM), or NULL
+  // z != NULL (bf16 operands, no ex): the accumulators themselves (tanh(pre z) with the soft-cap) of tokens below z_rows,
+  // a multiple of 256, [z_rows, ldx] fp32, V_pad columns of each row written; launch_dz_logits reads them.
+  float *z = nullptr;
+  int64_t z_rows = 0;
 };
 
 // The row-offset form's constants (base-2 units): the offset sits kExAbove above the label's logit, and a half tile's
@@ -291,8 +295,6 @@ int launch_ex_fix(const ExFixArgs &a, hipStream_t st);
 // read dz stop at the count).
 struct DzScaleArgs {
   void *dz;  // [rows, ld] 16-bit: f16 exponentials in, dz in dtype (bf16 / f16) out
-  const void *ex = nullptr;  // the exponentials where they are not in dz's place: kept, and dz zero from the count to the
-                             // next multiple of 64, the rows a count-bounded grad_W reads
   int64_t ld, V_pad;
   int dtype;
   const f32x4 *part;  // [rows, mtiles], local rows
@@ -310,6 +312,28 @@ struct DzScaleArgs {
   int64_t V;
 };
 int launch_dz_scale(const DzScaleArgs &a, hipStream_t st);
+
+// dz of a row pass over a vocabulary chunk from kept logits (StatsArgs::z), with gemm_dz's own formula and rounding: dz[i]
+// [k] for local rows i < rows (compact rows r0 + i) and chunk columns k < cols (vocabulary v0 + k; 0 from V on), the label
+// entry hit[i] (launch_hit's). Rows from the count to the next multiple of 64, which a count-bounded grad_W reads, get 0.
+struct DzLogitsArgs {
+  void *dz;  // bf16
+  int64_t ld;
+  const float *z;  // row i at z + i ldz: the accumulators, or tanh(pre z) with the soft-cap
+  int64_t ldz;
+  int64_t v0, cols, V;
+  const float *lse;  // compact rows (row_state)
+  int lse_pair;
+  const float *g;  // compact rows
+  float gmul, c;
+  int use_tanh;
+  const int64_t *labels;
+  const int64_t *label_idx;  // labels[label_idx[r]] when set
+  const float *hit;          // local rows
+  const int32_t *count;
+  int64_t r0, rows, n_max;
+};
+int launch_dz_logits(const DzLogitsArgs &a, hipStream_t st);
 
 // The GRPO tail of the fused step over prefix-tree pair rows: flat token t reads its pair row p = flat_pair[t]; for
 // the pass's rows (r0 <= p < r0 + rows, below the row count) it takes the row's (logprob, entropy) from rowout (2

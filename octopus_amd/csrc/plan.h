@@ -371,43 +371,6 @@ inline bool step_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh
   return false;
 }
 
-// ---- forward and backward with the exponentials kept between them (octo_head_fwd_stage, octo_head_bwd_stage) ------
-// One row pass of bf16 operands. The buffer the caller keeps: every element's exponential [P, V_pad] (f16, relative to its
-// half tile's maximum), the label entries [P] and the forward's workspace (its statistics at the front are read again).
-// The exponentials are bounded by the staging budget. The backward's workspace: dz [P, V_pad], h^T, W^T where grad_h
-// cannot read W as stored, grad_h's partial tiles.
-struct StageLayout {
-  int64_t P, V_pad, split_items;
-  size_t ex, hit, fwd, total;          // of the buffer
-  size_t dz, ht, wt, split, bwd_total;  // of the backward's workspace
-};
-inline bool stage_plan(int64_t n_max, int d, int V, int w_dtype, StageLayout &L) {
-  if (w_dtype != OCTO_BF16 || n_max <= 0 || n_max > kPassRowsMax) return false;
-  L.P = round_to(n_max, kTile);
-  L.V_pad = round_to(V, kTile);
-  const size_t staged = (size_t)L.P * L.V_pad * 2;
-  if (staged > kStagingBudget) return false;
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    const size_t at = off;
-    off += align_up(bytes);
-    return at;
-  };
-  L.ex = take(staged);
-  L.hit = take((size_t)L.P * sizeof(float));
-  L.fwd = take(fwd_layout(n_max, d, V, w_dtype, false).total);
-  L.total = off;
-  off = 0;
-  L.dz = take(staged);
-  L.ht = take((size_t)d * L.P * 2);
-  L.wt = take(gh_reads_w(d, V, w_dtype) ? 0 : (size_t)d * L.V_pad * 2);
-  const int64_t beside = gradh_split(L.P, d, V, false), alone = gradh_split(L.P, d, V, true);
-  L.split_items = beside > alone ? beside : alone;
-  L.split = take(L.split_items * kSplitTile);
-  L.bwd_total = off;
-  return true;
-}
-
 // The step without grad_W, whose operands (dz and the pass's h^T) stay in the workspace for octo_head_later_grad_w: one
 // pass of 16-bit weights within the staging budget. grad_h's partial tiles, one round of the CUs at most, lie behind.
 inline bool later_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, StepLayout &L) {

@@ -165,9 +165,10 @@ def _(rows, weight, w_scale, labels, idx, count, inv_T, pre, post, use_tanh, lab
 @torch.library.custom_op("octohead::head_bwd", mutates_args=(), device_types="cuda")
 def head_bwd(rows: Tensor, weight: Tensor, w_scale: Optional[Tensor], labels: Tensor, idx: Optional[Tensor],
              count: Optional[Tensor], lse: Tensor, g: Tensor, inv_T: float, pre: float, post: float,
-             use_tanh: bool, labels_via_idx: bool, need_rows: bool, need_weight: bool) -> tuple[Tensor, Tensor]:
+             use_tanh: bool, labels_via_idx: bool, need_rows: bool, need_weight: bool,
+             logits: Optional[Tensor] = None) -> tuple[Tensor, Tensor]:
     """(grad_rows [rows, d] in rows' dtype, grad_weight [V, d] in weight's dtype) for g = dL/dlogprob per
-    compact row; an output not asked for is an empty tensor."""
+    compact row; an output not asked for is an empty tensor. logits: what head_fwd_logits kept (bf16)."""
     rows2, weight2 = _rows2d(rows), _rows2d(weight)
     labels, idx = _index(labels), _index(idx)
     n_max = idx.numel() if idx is not None else rows2.shape[0]
@@ -193,10 +194,11 @@ def head_bwd(rows: Tensor, weight: Tensor, w_scale: Optional[Tensor], labels: Te
     if need_weight:  # written in the weight's dtype (summed in fp32 inside, rounded once)
         grad_w = torch.empty(V, d, dtype=weight.dtype, device=rows2.device)
     lse_c, g_c = lse.contiguous(), g.contiguous()  # kept alive until the call has queued its kernels
-    _lib.call("octo_head_bwd", _p(rows2), rows2.shape[0], rows2.stride(0), _dtype_code(rows2),
-              _p(weight2), weight2.stride(0), w_code, _p(w_scale), _p(labels), _p(idx), _p(count),
-              n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse_c),
-              _p(g_c), _p(gh), d, _dtype_code(rows2) if need_rows else _lib.F32,
+    head = (_p(rows2), rows2.shape[0], rows2.stride(0), _dtype_code(rows2), _p(weight2), weight2.stride(0), w_code)
+    args = (_p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse_c), _p(g_c))
+    kept = () if logits is None else (_p(logits), logits.stride(0), logits.shape[0])
+    _lib.call(*(("octo_head_bwd", *head, _p(w_scale)) if logits is None else ("octo_head_bwd_logits", *head)),
+              *args, *kept, _p(gh), d, _dtype_code(rows2) if need_rows else _lib.F32,
               _p(grad_w if need_weight else None), _dtype_code(grad_w) if need_weight else _lib.F32,
               _p(ws), ws.numel(), _stream(rows2))
     if need_rows and idx is not None:
@@ -207,7 +209,7 @@ def head_bwd(rows: Tensor, weight: Tensor, w_scale: Optional[Tensor], labels: Te
 
 @head_bwd.register_fake
 def _(rows, weight, w_scale, labels, idx, count, lse, g, inv_T, pre, post, use_tanh, labels_via_idx,
-      need_rows, need_weight):
+      need_rows, need_weight, logits=None):
     return (_empty(rows) if need_rows else rows.new_empty(0),
             _empty(weight) if need_weight else weight.new_empty(0))
 
@@ -398,6 +400,17 @@ torch.library.register_autograd("octohead::head_step_grpo", _step_backward, setu
 torch.library.register_autograd("octohead::head_step_grpo_pairs", _step_backward, setup_context=_step_setup)
 
 
+def _compact_g(gout: Tensor, idx: Optional[Tensor], count: Optional[Tensor], scatter: bool) -> Tensor:
+    """dL/dlogprob per compact row from the columns' gradient."""
+    col = gout.float()[:, 0].contiguous()
+    if not scatter:
+        return col
+    idx64 = idx.to(torch.int64).contiguous()  # g of compact row r is the output gradient at its hidden row idx[r]
+    g = torch.empty(idx.numel(), dtype=torch.float32, device=gout.device)
+    _lib.call("octo_gather_f32", _p(col), 1, _p(idx64), _p(count), idx.numel(), _p(g), _stream(gout))
+    return g
+
+
 def _head_setup(ctx, inputs, output):
     rows, weight, w_scale, labels, idx, count, inv_T, pre, post, use_tanh, labels_via_idx, scatter = inputs
     # The weight is held by reference, not saved: the backward reads the weight the module holds, as the reference's
@@ -425,13 +438,16 @@ def _head_backward(ctx, gout, _glse):
 torch.library.register_autograd("octohead::head_fwd", _head_backward, setup_context=_head_setup)
 
 
-# ---- the head with its exponentials kept between forward and backward (octo_head_fwd_stage) --------------------------
+# ---- the head with logits kept between forward and backward (octo_head_fwd_logits) ------------------------------------
 
-_STAGE_BYTES = 2 << 30  # of the kept exponentials, padded to 256 rows and columns: the backward's own staging budget
-# fused_head keeps them from this many multiply-adds of the logits on (n d V). The recompute they save takes 1.5 ns per
-# 2^20 of them; the wider store and the pass that makes dz cost a small call some 10 us, 2^33 multiply-adds' worth. And
-# for at most twice as many rows as the hidden width: what is kept until the backward then takes at most twice the bytes
-# of the weight's gradient, which a training step has room for anyway; beyond, the head keeps no [n, V] between calls.
+# Bytes of fp32 logits one call keeps; the rows past them are recomputed, as all are without. In fp32, so that dz is
+# rounded once, to bf16, and the gradients are the recomputing backward's to the bit.
+_KEEP_BYTES = 2 << 30
+# fused_head keeps logits from this many multiply-adds on (n d V), and for at most twice as many rows as the width (beyond,
+# fewer than half of the rows would be kept). us a forward and backward, kept and recomputed: 64 rows at d 1024, V 32,000
+# (2^31) 462 and 460, 256 rows 463 and 463, 1,024 rows 466 and 467; 32 rows at d 2560, V 151,936 (2^33.5) 623 and 787,
+# 3,000 rows, three quarters of them scored, 4,795 and 5,602; 8,192 rows at d 4096, V 128,256 (4,096 kept) 22,200 and
+# 24,250, 3,584 of them scored 9,196 and 11,149.
 _STAGE_WORK = 1 << 33
 
 
@@ -439,32 +455,31 @@ def _pad256(n: int) -> int:
     return (n + 255) // 256 * 256
 
 
-def _stage_numel(n_max: int, V: int) -> int:
-    """Bytes of the buffer, as octo_head_stage_bytes has them: exponentials, label entries, the forward's workspace."""
-    return _pad256(n_max) * _pad256(V) * 2 + _pad256(_pad256(n_max) * 4) + _pad256(n_max * (_pad256(V) // 256) * 16) + 256
+def _kept_rows(n: int, d: int, V: int) -> int:
+    """The rows (a multiple of 256) whose logits a call of n rows keeps: as many as _KEEP_BYTES hold, and at most d, so
+    that they take at most twice the bytes of the weight's gradient."""
+    return min(_pad256(n), _pad256(d), _KEEP_BYTES // (_pad256(V) * 4) // 256 * 256)
 
 
-def _stages(rows: Tensor, weight: Tensor, idx: Optional[Tensor], scale: float) -> bool:
-    """Whether fused_head keeps the exponentials: a gradient is wanted, octo_head_fwd_stage takes the call and the
-    recompute would cost more. Not while a compiler traces (a guard on the sizes), nor with a backward workspace set."""
+def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
+    """The rows whose logits fused_head keeps, 0 where the backward recomputes them all."""
     if not torch.is_grad_enabled() or BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling():
-        return False
+        return 0
     if not (rows.requires_grad or weight.requires_grad) or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
-        return False
-    if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not 1e-30 < scale < 1e30:
-        return False
+        return 0
+    if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+        return 0
     n = idx.numel() if idx is not None else rows.shape[0]
     V, d = weight.shape
-    # rows through idx lie below 2 GiB, as they are or copied (_rows2d)
-    return (0 < n <= min(32768, 2 * d) and _pad256(n) * _pad256(V) * 2 <= _STAGE_BYTES and n * d * V >= _STAGE_WORK
-            and not (idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff))
+    return _kept_rows(n, d, V) if 0 < n <= 2 * d and n * d * V >= _STAGE_WORK else 0
 
 
-@torch.library.custom_op("octohead::head_fwd_stage", mutates_args=(), device_types="cuda")
-def head_fwd_stage(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
-                   inv_T: float, pre: float, post: float, use_tanh: bool, labels_via_idx: bool,
-                   scatter: bool) -> tuple[Tensor, Tensor, Tensor]:
-    """head_fwd's (out, lse) and the buffer head_bwd_stage makes the gradients of."""
+@torch.library.custom_op("octohead::head_fwd_logits", mutates_args=(), device_types="cuda")
+def head_fwd_logits(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
+                    inv_T: float, pre: float, post: float, use_tanh: bool, labels_via_idx: bool, scatter: bool,
+                    keep: int) -> tuple[Tensor, Tensor, Tensor]:
+    """head_fwd's (out, lse) and the fp32 logits of the first `keep` compact rows [keep, V padded to 256], which
+    head_bwd takes."""
     rows, weight = _rows2d(rows), _rows2d(weight)
     labels, idx = _index(labels), _index(idx)
     n_max = idx.numel() if idx is not None else rows.shape[0]
@@ -472,96 +487,49 @@ def head_fwd_stage(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[T
     flags = (_lib.ROWS_VIA_IDX if labels_via_idx else 0) | (_lib.OUT_SCATTER if scatter else 0) | _lib.LSE_PAIR
     out = torch.zeros(rows.shape[0] if scatter else n_max, 2, dtype=torch.float32, device=rows.device)
     lse = torch.zeros(n_max, 2, dtype=torch.float32, device=rows.device)
+    logits = torch.empty(keep, _pad256(V), dtype=torch.float32, device=rows.device)
     code = _dtype_code(weight)
-    stage = _workspace(_lib.stage_bytes(n_max, d, V, code)[0], rows)
-    _lib.call("octo_head_fwd_stage", _p(rows), rows.shape[0], rows.stride(0), code, _p(weight), weight.stride(0), code,
-              _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse), _p(out), 2,
-              _p(stage), stage.numel(), _stream(rows))
-    return out, lse, stage
+    ws = _workspace(_lib.workspace_bytes(n_max, d, V, code, _gather_flag(rows, idx)), rows)
+    _lib.call("octo_head_fwd_logits", _p(rows), rows.shape[0], rows.stride(0), _dtype_code(rows), _p(weight),
+              weight.stride(0), code, _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post,
+              int(use_tanh), _p(lse), _p(out), 2, _p(logits), logits.stride(0), keep, _p(ws), ws.numel(),
+              _stream(rows))
+    return out, lse, logits
 
 
-@head_fwd_stage.register_fake
-def _(rows, weight, labels, idx, count, inv_T, pre, post, use_tanh, labels_via_idx, scatter):
+@head_fwd_logits.register_fake
+def _(rows, weight, labels, idx, count, inv_T, pre, post, use_tanh, labels_via_idx, scatter, keep):
     n_max = idx.shape[0] if idx is not None else rows.shape[0]
     return (rows.new_empty(rows.shape[0] if scatter else n_max, 2, dtype=torch.float32),
             rows.new_empty(n_max, 2, dtype=torch.float32),
-            rows.new_empty(_stage_numel(n_max, weight.shape[0]), dtype=torch.uint8))
+            rows.new_empty(keep, _pad256(weight.shape[0]), dtype=torch.float32))
 
 
-@torch.library.custom_op("octohead::head_bwd_stage", mutates_args=(), device_types="cuda")
-def head_bwd_stage(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[Tensor], count: Optional[Tensor],
-                   lse: Tensor, stage: Tensor, g: Tensor, inv_T: float, pre: float, post: float, use_tanh: bool,
-                   labels_via_idx: bool, need_rows: bool, need_weight: bool) -> tuple[Tensor, Tensor]:
-    """head_bwd's (grad_rows, grad_weight) from head_fwd_stage's buffer."""
-    rows2, weight2 = _rows2d(rows), _rows2d(weight)
-    labels, idx = _index(labels), _index(idx)
-    n_max = idx.numel() if idx is not None else rows2.shape[0]
-    V, d = weight2.shape
-    grad_rows = _zeros(rows) if need_rows else rows.new_empty(0)
-    grad_w = _empty(weight) if need_weight else weight.new_empty(0)
-    if not (need_rows or need_weight):
-        return grad_rows, grad_w
-    flags = (_lib.ROWS_VIA_IDX if labels_via_idx else 0) | _lib.LSE_PAIR
-    gh = None
-    if need_rows:  # compact-order rows; scattered (runs of equal idx summed) into grad_rows below
-        gh = grad_rows if idx is None else torch.empty(n_max, d, dtype=rows2.dtype, device=rows2.device)
-    code = _dtype_code(weight2)
-    ws = _workspace(_lib.stage_bytes(n_max, d, V, code)[1], rows2)
-    lse_c, g_c = lse.contiguous(), g.contiguous()  # kept alive until the call has queued its kernels
-    _lib.call("octo_head_bwd_stage", _p(rows2), rows2.shape[0], rows2.stride(0), code, _p(weight2), weight2.stride(0),
-              code, _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse_c),
-              _p(g_c), _p(stage), _p(gh), d, code, _p(grad_w if need_weight else None), code, _p(ws), ws.numel(),
-              _stream(rows2))
-    if need_rows and idx is not None:
-        _lib.call("octo_rows_scatter", _p(gh), d, code, _p(idx), _p(count), n_max, d, _p(grad_rows),
-                  grad_rows.stride(0), code, 0, _stream(rows2))
-    return grad_rows, grad_w
-
-
-@head_bwd_stage.register_fake
-def _(rows, weight, labels, idx, count, lse, stage, g, inv_T, pre, post, use_tanh, labels_via_idx, need_rows,
-      need_weight):
-    return (_empty(rows) if need_rows else rows.new_empty(0),
-            _empty(weight) if need_weight else weight.new_empty(0))
-
-
-def _compact_g(gout: Tensor, idx: Optional[Tensor], count: Optional[Tensor], scatter: bool) -> Tensor:
-    """dL/dlogprob per compact row from the columns' gradient."""
-    gout = gout.float()
-    if not scatter:
-        return gout[:, 0].contiguous()
-    col = gout[:, 0].contiguous()  # g of compact row r is the output gradient at its hidden row idx[r]
-    idx64 = idx.to(torch.int64).contiguous()
-    g = torch.empty(idx.numel(), dtype=torch.float32, device=gout.device)
-    _lib.call("octo_gather_f32", _p(col), 1, _p(idx64), _p(count), idx.numel(), _p(g), _stream(gout))
-    return g
-
-
-def _stage_setup(ctx, inputs, output):
+def _logits_setup(ctx, inputs, output):
     rows, weight, labels, idx, count = inputs[:5]
-    # the weight and the buffer are held by reference, not saved: a pack hook never copies them to the host
+    # the weight and the logits are held by reference, not saved: a pack hook never copies them to the host
     ctx.weight = weight
-    ctx.stage = output[2].detach()
-    ctx.params = inputs[5:]
+    ctx.logits = output[2].detach()
+    ctx.params = inputs[5:11]
     ctx.save_for_backward(rows, labels, idx, count, output[1])
-    ctx.set_materialize_grads(False)  # no zeros the size of the buffer for the gradient it does not have
+    ctx.set_materialize_grads(False)  # no zeros the size of the logits for the gradient they do not have
 
 
-def _stage_backward(ctx, gout, _glse, _gstage):
+def _logits_backward(ctx, gout, _glse, _glogits):
     rows, labels, idx, count, lse = ctx.saved_tensors
     inv_T, pre, post, use_tanh, labels_via_idx, scatter = ctx.params
     need_rows, need_weight = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
     if gout is None:  # no loss reads the columns
-        return (_zeros(rows) if need_rows else None, _zeros(ctx.weight) if need_weight else None) + (None,) * 9
+        return (_zeros(rows) if need_rows else None, _zeros(ctx.weight) if need_weight else None) + (None,) * 10
     g = _compact_g(gout, idx, count, scatter)
-    grad_rows, grad_w = head_bwd_stage(rows, ctx.weight, labels, idx, count, lse, ctx.stage, g, inv_T, pre, post,
-                                       use_tanh, labels_via_idx, need_rows, need_weight)
+    grad_rows, grad_w = head_bwd(rows, ctx.weight, None, labels, idx, count, lse, g, inv_T, pre, post, use_tanh,
+                                 labels_via_idx, need_rows, need_weight, ctx.logits)
     if not torch._C._autograd._get_current_graph_task_keep_graph():
-        ctx.stage = None  # as the saved tensors: a loss kept for its value does not keep the buffer
-    return (grad_rows if need_rows else None, grad_w if need_weight else None) + (None,) * 9
+        ctx.logits = None  # as the saved tensors: a loss kept for its value does not keep them
+    return (grad_rows if need_rows else None, grad_w if need_weight else None) + (None,) * 10
 
 
-torch.library.register_autograd("octohead::head_fwd_stage", _stage_backward, setup_context=_stage_setup)
+torch.library.register_autograd("octohead::head_fwd_logits", _logits_backward, setup_context=_logits_setup)
 
 
 def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float, post: Post = Post(), *,
@@ -572,8 +540,9 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
     if temperature <= 0:
         raise ValueError("temperature must be positive")
     xf = (1.0 / float(temperature), float(post.pre), float(post.post), bool(post.tanh), labels_via_idx, scatter)
-    if _stages(rows, weight, idx, xf[0] * (1.0 if post.tanh else xf[1]) * xf[2]):
-        return head_fwd_stage(rows, weight, labels, idx, count, *xf)[0]
+    keep = _keeps(rows, weight, idx)
+    if keep:
+        return head_fwd_logits(rows, weight, labels, idx, count, *xf, keep)[0]
     out, _ = head_fwd(rows, weight, w_scale, labels, idx, count, *xf)
     return out
 

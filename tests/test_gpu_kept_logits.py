@@ -1,0 +1,73 @@
+"""fused_head with logits kept for the backward (octo_head_fwd_logits, octo_head_bwd_logits): to the bit what the
+recomputing backward gives, over what both take."""
+import pytest
+import torch
+
+from octopus_amd import head_op
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _both(n, d, V, scored, T, cap, monkeypatch, need=(True, True), rows=None, ws=None, bad_labels=False):
+    """(columns, grad_rows, grad_weight) with logits kept (of `rows` rows at most) and without; ws: the backward's
+    workspace."""
+    g = torch.Generator(device=DEV).manual_seed(n + V)
+    W = (torch.randn(V, d, generator=g, device=DEV) * 0.05).bfloat16()
+    h = torch.randn(n, d, generator=g, device=DEV).bfloat16()
+    y = torch.randint(0, V, (n,), generator=g, device=DEV)
+    if bad_labels:
+        y[::3] = -100
+        y[1::7] = V
+    coef = torch.randn(n, generator=g, device=DEV)
+    mask = torch.rand(n, generator=g, device=DEV) < scored
+    kw = {}
+    if scored < 1:
+        idx, count = head_op.compact_rows(mask)
+        kw = dict(idx=idx, count=count, labels_via_idx=True, scatter=True)
+    post = head_op.Post(1 / 30.0, 30.0, True) if cap else head_op.Post()
+    if rows is not None:
+        monkeypatch.setattr(head_op, "_KEEP_BYTES", rows * head_op._pad256(V) * 4)
+    got = []
+    for least in (0, 1 << 62):
+        monkeypatch.setattr(head_op, "_STAGE_WORK", least)
+        hd, Wd = h.clone().requires_grad_(need[0]), W.clone().requires_grad_(need[1])
+        assert bool(head_op._keeps(hd, Wd, kw.get("idx"))) == (least == 0 and n <= 2 * d)
+        out = head_op.fused_head(hd, Wd, y, T, post, **kw)
+        with monkeypatch.context() as m:
+            if ws is not None:
+                m.setattr(head_op, "BWD_WORKSPACE_BYTES", ws)
+            (coef * out[:, 0])[~torch.isnan(out[:, 0])].sum().backward()
+        got.append((out.detach(), hd.grad, Wd.grad))
+    return got
+
+
+# one row; ragged rows; widths and vocabularies read through W^T (d % 256, V % 64); no scored row; the softcap; a
+# temperature at which most probabilities are far below 2^-25 of the row's largest; labels outside the vocabulary
+@pytest.mark.parametrize("n,d,V,scored,T,cap,bad", [
+    (1, 256, 640, 1.0, 1.0, False, False),
+    (300, 512, 5003, 0.7, 0.7, False, True),
+    (257, 136, 1000, 0.5, 1.0, False, False),
+    (300, 512, 3000, 0.0, 1.0, False, False),
+    (333, 256, 1500, 0.9, 1.0, True, True),
+    (700, 512, 2048, 0.8, 0.012, False, False),
+])
+def test_as_recomputed(n, d, V, scored, T, cap, bad, monkeypatch):
+    a, b = _both(n, d, V, scored, T, cap, monkeypatch, bad_labels=bad)
+    assert all(torch.equal(torch.nan_to_num(x), torch.nan_to_num(y)) for x, y in zip(a, b))
+
+
+# fewer rows kept than there are, the count below and above them; vocabulary chunks and several row passes
+@pytest.mark.parametrize("n,scored,rows,ws", [
+    (900, 0.9, 256, None), (900, 0.2, 256, None), (900, 1.0, 512, 8 << 20), (700, 1.0, 256, 3 << 20),
+])
+@pytest.mark.parametrize("cap", [False, True])
+def test_some_rows_kept(n, scored, rows, ws, cap, monkeypatch):
+    a, b = _both(n, 512, 2500, scored, 0.7, cap, monkeypatch, rows=rows, ws=ws)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("need", [(True, False), (False, True)])
+def test_one_gradient(need, monkeypatch):
+    a, b = _both(300, 512, 3000, 0.7, 1.0, False, monkeypatch, need=need)
+    assert all((x is None and y is None) or torch.equal(x, y) for x, y in zip(a, b))

@@ -1,4 +1,4 @@
-"""fused_head with its exponentials kept for the backward (octo_head_fwd_stage, octo_head_bwd_stage): gradients against 64
+"""fused_head with its logits kept for the backward (octo_head_fwd_logits, octo_head_bwd_logits): gradients against 64
 bits and against the recomputing route, at the edges of what takes this route."""
 import pytest
 import torch

@@ -4,19 +4,15 @@ import pytest
 from octopus_amd import _lib, head_op
 
 
-@pytest.mark.parametrize("n,d,V", [(1, 256, 640), (300, 136, 1000), (5119, 2560, 151936), (8192, 4096, 128256)])
-def test_stage_size_is_the_one_a_traced_call_expects(n, d, V):
-    buf, ws = _lib.stage_bytes(n, d, V, _lib.BF16)
-    P, Vp = -(-n // 256) * 256, -(-V // 256) * 256
-    assert buf == head_op._stage_numel(n, V) and buf >= P * Vp * 2 + P * 4 + n * (Vp // 256) * 16
-    assert ws >= P * Vp * 2 + d * P * 2 + (d * Vp * 2 if V % 64 or d % 256 else 0)
-
-
-def test_what_is_not_staged():
-    for w in (_lib.F16, _lib.F32, _lib.FP8E4M3):
-        assert _lib.stage_bytes(256, 256, 1024, w) == (0, 0)
-    assert _lib.stage_bytes(0, 256, 1024, _lib.BF16) == (0, 0)
-    assert _lib.stage_bytes(32768, 256, 151936, _lib.BF16) == (0, 0)  # past 2 GiB
+@pytest.mark.parametrize("n,d,V,rows", [
+    (1, 256, 640, 256), (300, 136, 1000, 256), (300, 512, 5003, 512),
+    (5119, 2560, 151936, 2560),  # as many as the width
+    (8192, 4096, 128256, 4096), (8192, 4096, 151936, 3328),  # 2 GiB
+    (8192, 4096, 3 << 20, 0),  # not one tile of rows
+])
+def test_rows_whose_logits_are_kept(n, d, V, rows):
+    assert head_op._kept_rows(n, d, V) == rows
+    assert rows * head_op._pad256(V) * 4 <= head_op._KEEP_BYTES
 
 
 def test_what_is_left_for_later():
