@@ -465,7 +465,8 @@ def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
     """The rows whose logits fused_head keeps, 0 where the backward recomputes them all."""
     if not torch.is_grad_enabled() or BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling():
         return 0
-    if not (rows.requires_grad or weight.requires_grad) or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
+    # a frozen weight has no gradient for the kept bytes to stand beside
+    if not weight.requires_grad or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
         return 0
     if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
         return 0

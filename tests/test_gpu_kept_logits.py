@@ -32,7 +32,7 @@ def _both(n, d, V, scored, T, cap, monkeypatch, need=(True, True), rows=None, ws
     for least in (0, 1 << 62):
         monkeypatch.setattr(head_op, "_STAGE_WORK", least)
         hd, Wd = h.clone().requires_grad_(need[0]), W.clone().requires_grad_(need[1])
-        assert bool(head_op._keeps(hd, Wd, kw.get("idx"))) == (least == 0 and n <= 2 * d)
+        assert bool(head_op._keeps(hd, Wd, kw.get("idx"))) == (least == 0 and n <= 2 * d and need[1])
         out = head_op.fused_head(hd, Wd, y, T, post, **kw)
         with monkeypatch.context() as m:
             if ws is not None:

@@ -1,5 +1,7 @@
 """Which calls keep a buffer between forward and backward, and its size (host planning only)."""
 import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from octopus_amd import _lib, head_op
 
@@ -24,3 +26,20 @@ def test_what_is_left_for_later():
         plain = _lib.later_bytes(n, 2560, 151936, _lib.BF16, False)
         assert plain >= P * (-(-151936 // 256) * 256) * 2 + 2560 * P * 2  # dz and h^T
         assert 0 <= _lib.later_bytes(n, 2560, 151936, _lib.BF16, True) - plain <= 256 * 256 * 256 * 4  # one round of runs
+
+
+def _operands(n=512, d=1024, V=33024, weight_grad=True):
+    """Operands without storage, of a size that keeps logits (under FakeTensorMode)."""
+    return (torch.empty(n, d, dtype=torch.bfloat16, device="cuda", requires_grad=True),
+            torch.empty(V, d, dtype=torch.bfloat16, device="cuda", requires_grad=weight_grad),
+            torch.zeros(n, dtype=torch.int64, device="cuda"))
+
+
+def _kept(out):
+    return "head_fwd_logits" in type(out.grad_fn).__name__
+
+
+def test_a_frozen_weight_keeps_no_logits():
+    with FakeTensorMode():
+        assert _kept(head_op.fused_head(*_operands(), 1.0))
+        assert not _kept(head_op.fused_head(*_operands(weight_grad=False), 1.0))
