@@ -465,6 +465,9 @@ def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
     """The rows whose logits fused_head keeps, 0 where the backward recomputes them all."""
     if not torch.is_grad_enabled() or BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling():
         return 0
+    # inside checkpoint or an offload's hooks the caller has said that little is to stay on the device until the backward
+    if torch._C._autograd._top_saved_tensors_default_hooks(False) is not None:
+        return 0
     # a frozen weight has no gradient for the kept bytes to stand beside
     if not weight.requires_grad or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
         return 0

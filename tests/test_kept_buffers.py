@@ -2,6 +2,7 @@
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils.checkpoint import checkpoint
 
 from octopus_amd import _lib, head_op
 
@@ -43,3 +44,21 @@ def test_a_frozen_weight_keeps_no_logits():
     with FakeTensorMode():
         assert _kept(head_op.fused_head(*_operands(), 1.0))
         assert not _kept(head_op.fused_head(*_operands(weight_grad=False), 1.0))
+
+
+def test_checkpointed_and_offloaded_calls_keep_no_logits():
+    """What such a caller's hooks do not reach would stay on the device, once per checkpointed chunk."""
+    with FakeTensorMode():
+        rows, weight, y = _operands()
+        routes = []
+
+        def head(h):
+            out = head_op.fused_head(h, weight, y, 1.0)
+            routes.append(_kept(out))
+            return out
+
+        checkpoint(head, rows, use_reentrant=False)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+            head(rows)
+        head(rows)
+        assert routes == [False, False, True]
