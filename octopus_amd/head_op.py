@@ -12,6 +12,7 @@ here and raises. All work is queued on the current stream; nothing synchronises 
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import NamedTuple, Optional
 
 import torch
@@ -440,8 +441,8 @@ torch.library.register_autograd("octohead::head_fwd", _head_backward, setup_cont
 
 # ---- the head with logits kept between forward and backward (octo_head_fwd_logits) ------------------------------------
 
-# Bytes of fp32 logits one call keeps; the rows past them are recomputed, as all are without. In fp32, so that dz is
-# rounded once, to bf16, and the gradients are the recomputing backward's to the bit.
+# Bytes of fp32 logits one call keeps, and all live ones on a device together; the rows past them are recomputed, as all
+# are without. In fp32, so that dz is rounded once, to bf16, and the gradients are the recomputing backward's to the bit.
 _KEEP_BYTES = 2 << 30
 # fused_head keeps logits from this many multiply-adds on (n d V), and for at most twice as many rows as the width (beyond,
 # fewer than half of the rows would be kept). us a forward and backward, kept and recomputed: 64 rows at d 1024, V 32,000
@@ -459,6 +460,27 @@ def _kept_rows(n: int, d: int, V: int) -> int:
     """The rows (a multiple of 256) whose logits a call of n rows keeps: as many as _KEEP_BYTES hold, and at most d, so
     that they take at most twice the bytes of the weight's gradient."""
     return min(_pad256(n), _pad256(d), _KEEP_BYTES // (_pad256(V) * 4) // 256 * 256)
+
+
+class _Room:
+    """A share of the _KEEP_BYTES that the kept logits of a device take together, given back when this object goes. A
+    caller that holds several losses before their backwards keeps one call's logits, or two smaller ones'; the other calls
+    recompute, to the same bits."""
+
+    _lock = threading.RLock()  # a collection inside the lock may free another share
+    _taken: dict = {}
+    pending = threading.local()  # .room: the calling thread's share, for the node that its forward makes
+
+    def __init__(self, device: torch.device, nbytes: int):
+        self.device, self.nbytes = device, 0
+        with self._lock:
+            if self._taken.get(device, 0) + nbytes <= _KEEP_BYTES:
+                self._taken[device] = self._taken.get(device, 0) + nbytes
+                self.nbytes = nbytes
+
+    def __del__(self):
+        with self._lock:
+            self._taken[self.device] = self._taken.get(self.device, 0) - self.nbytes
 
 
 def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
@@ -514,6 +536,7 @@ def _logits_setup(ctx, inputs, output):
     # the weight and the logits are held by reference, not saved: a pack hook never copies them to the host
     ctx.weight = weight
     ctx.logits = output[2].detach()
+    ctx.room = getattr(_Room.pending, "room", None)
     ctx.params = inputs[5:11]
     ctx.save_for_backward(rows, labels, idx, count, output[1])
     ctx.set_materialize_grads(False)  # no zeros the size of the logits for the gradient they do not have
@@ -526,10 +549,17 @@ def _logits_backward(ctx, gout, _glse, _glogits):
     if gout is None:  # no loss reads the columns
         return (_zeros(rows) if need_rows else None, _zeros(ctx.weight) if need_weight else None) + (None,) * 10
     g = _compact_g(gout, idx, count, scatter)
-    grad_rows, grad_w = head_bwd(rows, ctx.weight, None, labels, idx, count, lse, g, inv_T, pre, post, use_tanh,
-                                 labels_via_idx, need_rows, need_weight, ctx.logits)
-    if not torch._C._autograd._get_current_graph_task_keep_graph():
-        ctx.logits = None  # as the saved tensors: a loss kept for its value does not keep them
+    args = (rows, ctx.weight, None, labels, idx, count, lse, g, inv_T, pre, post, use_tanh, labels_via_idx, need_rows,
+            need_weight)
+    got = None
+    if ctx.logits is not None:
+        try:
+            got = head_bwd(*args, ctx.logits)
+        except torch.OutOfMemoryError:  # recomputed below, without what is kept
+            pass
+    if got is None or not torch._C._autograd._get_current_graph_task_keep_graph():
+        ctx.logits = ctx.room = None  # as the saved tensors: a loss kept for its value does not keep them
+    grad_rows, grad_w = head_bwd(*args) if got is None else got
     return (grad_rows if need_rows else None, grad_w if need_weight else None) + (None,) * 10
 
 
@@ -546,7 +576,16 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
     xf = (1.0 / float(temperature), float(post.pre), float(post.post), bool(post.tanh), labels_via_idx, scatter)
     keep = _keeps(rows, weight, idx)
     if keep:
-        return head_fwd_logits(rows, weight, labels, idx, count, *xf, keep)[0]
+        room = _Room(rows.device, keep * _pad256(weight.shape[0]) * 4)
+        if room.nbytes:
+            _Room.pending.room = room
+            try:
+                return head_fwd_logits(rows, weight, labels, idx, count, *xf, keep)[0]
+            except torch.OutOfMemoryError:  # no room on the device: recomputed, as without
+                pass
+            finally:
+                _Room.pending.room = None
+        del room
     out, _ = head_fwd(rows, weight, w_scale, labels, idx, count, *xf)
     return out
 

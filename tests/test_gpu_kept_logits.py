@@ -71,3 +71,18 @@ def test_some_rows_kept(n, scored, rows, ws, cap, monkeypatch):
 def test_one_gradient(need, monkeypatch):
     a, b = _both(300, 512, 3000, 0.7, 1.0, False, monkeypatch, need=need)
     assert all((x is None and y is None) or torch.equal(x, y) for x, y in zip(a, b))
+
+
+def test_out_of_memory_in_the_backward(monkeypatch):
+    """The backward lets the logits go and recomputes."""
+    want = _both(300, 512, 3000, 0.7, 1.0, False, monkeypatch)[1]
+    bwd = head_op.head_bwd
+
+    def full(*args):
+        if len(args) == 16 and args[15] is not None:
+            raise torch.OutOfMemoryError("full")
+        return bwd(*args)
+
+    monkeypatch.setattr(head_op, "head_bwd", full)
+    got = _both(300, 512, 3000, 0.7, 1.0, False, monkeypatch)[0]
+    assert all(torch.equal(x, y) for x, y in zip(got, want))

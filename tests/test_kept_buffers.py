@@ -62,3 +62,29 @@ def test_checkpointed_and_offloaded_calls_keep_no_logits():
             head(rows)
         head(rows)
         assert routes == [False, False, True]
+
+
+def test_live_logits_of_a_device_share_one_bound(monkeypatch):
+    with FakeTensorMode():
+        rows, weight, y = _operands()
+        monkeypatch.setattr(head_op, "_KEEP_BYTES", 512 * 33024 * 4)
+        first, second = (head_op.fused_head(rows, weight, y, 1.0) for _ in range(2))
+        assert _kept(first) and not _kept(second)
+        del first
+        again = head_op.fused_head(rows, weight, y, 1.0)
+        assert _kept(again)
+        del again
+        assert head_op._Room._taken[rows.device] == 0
+
+
+def test_out_of_memory_recomputes(monkeypatch):
+    def full(*_):
+        raise torch.OutOfMemoryError("full")
+
+    with FakeTensorMode():
+        operands = _operands()
+        with monkeypatch.context() as m:
+            m.setattr(head_op, "head_fwd_logits", full)
+            assert not _kept(head_op.fused_head(*operands, 1.0))
+        assert head_op._Room._taken[operands[0].device] == 0
+        assert _kept(head_op.fused_head(*operands, 1.0))
