@@ -535,6 +535,7 @@ def _logits_setup(ctx, inputs, output):
     rows, weight, labels, idx, count = inputs[:5]
     # the weight and the logits are held by reference, not saved: a pack hook never copies them to the host
     ctx.weight = weight
+    ctx.version = weight._version
     ctx.logits = output[2].detach()
     ctx.room = getattr(_Room.pending, "room", None)
     ctx.params = inputs[5:11]
@@ -552,7 +553,8 @@ def _logits_backward(ctx, gout, _glse, _glogits):
     args = (rows, ctx.weight, None, labels, idx, count, lse, g, inv_T, pre, post, use_tanh, labels_via_idx, need_rows,
             need_weight)
     got = None
-    if ctx.logits is not None:
+    # a weight changed in place since: the backward reads the one the module holds now (_head_setup), so does this one
+    if ctx.logits is not None and ctx.weight._version == ctx.version:
         try:
             got = head_bwd(*args, ctx.logits)
         except torch.OutOfMemoryError:  # recomputed below, without what is kept

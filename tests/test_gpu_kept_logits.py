@@ -86,3 +86,21 @@ def test_out_of_memory_in_the_backward(monkeypatch):
     monkeypatch.setattr(head_op, "head_bwd", full)
     got = _both(300, 512, 3000, 0.7, 1.0, False, monkeypatch)[0]
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_a_weight_changed_in_place(monkeypatch):
+    """The backward reads the weight as it is then, as the recomputing one does."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    W = (torch.randn(3000, 512, generator=g, device=DEV) * 0.05).bfloat16()
+    h = torch.randn(300, 512, generator=g, device=DEV).bfloat16()
+    y = torch.randint(0, 3000, (300,), generator=g, device=DEV)
+    got = []
+    for least in (0, 1 << 62):
+        monkeypatch.setattr(head_op, "_STAGE_WORK", least)
+        hd, Wd = h.clone().requires_grad_(True), W.clone().requires_grad_(True)
+        out = head_op.fused_head(hd, Wd, y, 1.0)
+        with torch.no_grad():
+            Wd.mul_(0.875)
+        out[:, 0].sum().backward()
+        got.append((hd.grad, Wd.grad))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
