@@ -841,13 +841,22 @@ template <int DT> __device__ __forceinline__ i32x4 pack_chunk(const float (&x)[1
 // logprob is not.
 struct ColStat {
   float m = -INFINITY, S = 0.f, U = 0.f;
+  // S and U relative to a maximum -d above m. Far below it they count for nothing, and what they hold may be no number: a
+  // thread that has only seen logits masked with a finite -1e38 or lower has m = x c rounded by up to 2^103, and its e are
+  // exp2 of that. (A NaN stays: it came from a NaN or infinite logit.)
+  __device__ __forceinline__ void shift(float d) {
+    if (d < -256.f) {
+      S = S == S ? 0.f : S;
+      U = U == U ? 0.f : U;
+    } else {
+      const float f = fexp2(d);
+      U = f * __builtin_fmaf(d, S, U);
+      S *= f;
+    }
+  }
   __device__ __forceinline__ void raise(float mx) {
     if (mx > m) {
-      if (m != -INFINITY) {
-        const float d = m - mx, f = fexp2(d);
-        U = f * __builtin_fmaf(d, S, U);
-        S *= f;
-      }
+      if (m != -INFINITY) shift(m - mx);
       m = mx;
     }
   }
@@ -905,8 +914,8 @@ __global__ __launch_bounds__(NT) void columns_fwd_kernel(const void *logits, int
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NW; ++k) m2 = fmaxf(m2, red[0][k]);
-  const float d = st.m == -INFINITY ? 0.f : st.m - m2, f = fexp2(d);  // m = -inf: S = 0, and U 0 or NaN
-  const float S = wave_sum(f * st.S), U = wave_sum(f * __builtin_fmaf(d, st.S, st.U));
+  if (st.m != -INFINITY) st.shift(st.m - m2);  // else S = 0, and U 0 or NaN
+  const float S = wave_sum(st.S), U = wave_sum(st.U);
   if (lane == 0) {
     red[1][w] = S;
     red[2][w] = U;
