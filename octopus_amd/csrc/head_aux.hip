@@ -802,7 +802,7 @@ __global__ __launch_bounds__(1024) void compact_kernel(const uint8_t *mask, int6
 // end), the backward reads it once more and writes its gradient. 16-byte loads, kColLoads of them in flight per thread;
 // a row that starts off a 16-byte boundary (an odd V) has up to 7 values before the first chunk and up to 7 after the
 // last, one per thread. [2048, 151,936] bf16, before (one value per load, the forward in two sweeps) and now: forward
-// 718 and 111 us, backward 746 and 220.
+// 718 and 105 us, backward 746 and 220.
 constexpr int kColLoads = 4;
 
 // The 16-byte chunks of a row of V values at p: `head` values before the first chunk, `chunks` of PER, then the rest.
@@ -868,10 +868,15 @@ struct ColStat {
   }
 };
 
-template <int DT, int NT>
-__global__ __launch_bounds__(NT) void columns_fwd_kernel(const void *logits, int64_t ld, const int64_t *labels, int V,
-                                                         float inv_T, float *out2, float *lse_out) {
-  constexpr int PER = 16 / Elem<DT>::bytes, NW = NT / 64;
+// One workgroup of 1,024 threads per row, at any number of rows: few rows are a chain of dependent steps (151,936 values
+// of bf16: 5 of 4 loads), and a row's sums keep their order, so its columns are the same to the bit beside any other
+// rows. [rows, 151,936] bf16 with 256 threads a row and with 1,024: 512 rows 33 and 31 us, 1,024 rows 57 and 55, 2,048
+// rows 109 and 105.
+constexpr int kColThreads = 1024;
+template <int DT>
+__global__ __launch_bounds__(kColThreads) void columns_fwd_kernel(const void *logits, int64_t ld, const int64_t *labels,
+                                                                  int V, float inv_T, float *out2, float *lse_out) {
+  constexpr int PER = 16 / Elem<DT>::bytes, NW = kColThreads / 64;
   typedef typename Elem<DT>::T T;
   __shared__ float red[3][NW];
   const int64_t r = blockIdx.x;
@@ -881,11 +886,11 @@ __global__ __launch_bounds__(NT) void columns_fwd_kernel(const void *logits, int
   const RowChunks rc = row_chunks<DT>(row, V);
   const i32x4 *vec = (const i32x4 *)(row + rc.head);
   ColStat st;
-  for (int k0 = threadIdx.x; k0 < rc.chunks; k0 += kColLoads * NT) {
+  for (int k0 = threadIdx.x; k0 < rc.chunks; k0 += kColLoads * kColThreads) {
     i32x4 v[kColLoads];
 #pragma unroll
     for (int u = 0; u < kColLoads; ++u)  // past the end: the last chunk again, left out below
-      v[u] = vec[min(k0 + u * NT, rc.chunks - 1)];
+      v[u] = vec[min(k0 + u * kColThreads, rc.chunks - 1)];
     float x[kColLoads][PER];
     float mx = -INFINITY;
 #pragma unroll
@@ -897,7 +902,7 @@ __global__ __launch_bounds__(NT) void columns_fwd_kernel(const void *logits, int
     st.raise(mx * c);
 #pragma unroll
     for (int u = 0; u < kColLoads; ++u)
-      if (k0 + u * NT < rc.chunks)
+      if (k0 + u * kColThreads < rc.chunks)
 #pragma unroll
         for (int e = 0; e < PER; ++e) st.add(x[u][e], c);
   }
@@ -955,7 +960,8 @@ __global__ __launch_bounds__(256) void columns_bwd_kernel(const void *logits, in
   T *drow = (T *)dl + r * ld_d;
   const float c = inv_T * OCTO_LOG2E, m2 = lse[2 * r], l2s = lse[2 * r + 1], gs = g[r] * inv_T;
   const int64_t y = labels[r];
-  // the forward's own t = fma(x, c, -m2), so the row's p keep the forward's rounding (row_state)
+  // t = fma(x, c, -m2) against the row's maximum, as the forward takes the label's logit (its sums add terms against
+  // each thread's own maximum, scaled): close to a probability of 1, 1 - p keeps the logprob's precision
   auto grad = [&](float x, int j) {
     const float p = fexp2(__builtin_fmaf(x, c, -m2) - l2s);
     return gs * ((y == j ? 1.f : 0.f) - p);
@@ -990,18 +996,11 @@ __global__ __launch_bounds__(256) void columns_bwd_kernel(const void *logits, in
   }
 }
 
-// Few rows: a workgroup of 1,024 threads shortens each row's chain of dependent steps (151,936 values of bf16: 5 of 4
-// loads, with 256 threads 19); from kColWide rows on, 2 per CU, the rows fill the chip and smaller workgroups end more
-// evenly.
-constexpr int64_t kColWide = 512;
 template <int DT>
 static void go_columns_fwd(const void *logits, int64_t ld, const int64_t *labels, int64_t n, int V, float inv_T,
                            float *out2, float *lse, hipStream_t st) {
-  const dim3 grid((unsigned)n);
-  if (n < kColWide)
-    hipLaunchKernelGGL((columns_fwd_kernel<DT, 1024>), grid, dim3(1024), 0, st, logits, ld, labels, V, inv_T, out2, lse);
-  else
-    hipLaunchKernelGGL((columns_fwd_kernel<DT, 256>), grid, dim3(256), 0, st, logits, ld, labels, V, inv_T, out2, lse);
+  hipLaunchKernelGGL(columns_fwd_kernel<DT>, dim3((unsigned)n), dim3(kColThreads), 0, st, logits, ld, labels, V, inv_T,
+                     out2, lse);
 }
 
 template <int DT>
