@@ -6,14 +6,16 @@
 // v_mfma_f32_32x32x2_f32) leave the sums no less exact, measured against 64 bits on [512, 32,000] logits of d 1024: the
 // columns 6.4e-7 off (relative) against 7.9e-7, the gradients 8e-7 against 3.2e-6. Time there: the logits and their
 // statistics 279 us with the fp32 instructions (120 TFLOP/s), 178 here (188 TFLOP/s in fp32 terms).
-// An infinite operand has no such parts: its products come out NaN (the sums of a row with one are NaN either way, as
-// inf - inf in the softmax).
+// An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: its remainder is not finite,
+// and so is every sum it enters. A tile with such a sum is made again by v_mfma_f32_16x16x4_f32 from the operands as they
+// are (mainloop_plain), infinities and NaN where those products have them; to look for one costs 0.6% of those logits'
+// time. Below 2^-110 the third part loses bits.
 //
 // One workgroup computes a 256 x 128 tile of C[m, n] = sum_k A[m, k] B[n, k] with 8 waves, two per SIMD, 2 x 4 of 128 x
 // 32 (AccX: the 16 x 16 block layout of the 16-bit kernels, 8 x 2 blocks). A stage is K = 32: 48 KB of fp32 go from
 // global memory to registers one stage ahead, are split there, and land in the LDS as three bf16 planes per operand
 // (72 KB a stage, two stages). Bound by the matrix cores: 96 MFMAs per wave and stage (1,536 cycles) against 24 values
-// per thread to split (5.5 instructions each, and two for infinities). One wave of each SIMD splits the next
+// per thread to split (5.5 instructions each). One wave of each SIMD splits the next
 // stage before its MFMAs and the other after them, so that one's vector instructions run beside the other's MFMAs. A
 // 256 x 256 tile would need 96 KB a stage: no room for the second.
 //
@@ -47,8 +49,7 @@ __device__ __forceinline__ int xslot(int row, int c) { return row * XROWB + ((c 
 // x = p0 + p1 + p2, 8 values at a time: p0 = x to the nearest bf16, p1 the (exact) remainder to the nearest, p2 what is
 // left, at most 7 bits, a bf16 as it stands. To the nearest and not towards zero, so that the remainders, and with them
 // the partial products left out, have either sign: cut off, they all lean one way, 2^-23 of every sum, and the logprobs
-// of [512, 32,000] logits were a quarter further from 64 bits than the fp32 instructions' (1.1e-6 against 8.8e-7). A
-// value whose p0 is not finite keeps p0 alone.
+// of [512, 32,000] logits were a quarter further from 64 bits than the fp32 instructions' (1.1e-6 against 8.8e-7).
 __device__ __forceinline__ void split8(const float (&x)[8], i32x4 (&p)[3]) {
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
@@ -63,10 +64,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], i32x4 (&p)[3]) {
       if (k == 2) break;
       const float f[2] = {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        r[e] -= f[e];
-        if (k == 0) r[e] = __builtin_fabsf(f[e]) < INFINITY ? r[e] : 0.f;
-      }
+      for (int e = 0; e < 2; ++e) r[e] -= f[e];
     }
   }
 }
@@ -240,6 +238,81 @@ __device__ __forceinline__ void mainloop_x(LA &a, LB &b, int nk, lds_char *smem,
   }
 }
 
+// An operand's value i (row, or column of a K-major one) at k, read by itself; 0 outside the matrix.
+struct XPlain {
+  const char *base;
+  const int64_t *map;
+  int64_t ld, rows, K;
+  bool down;  // K down the matrix rows
+  __device__ __forceinline__ XPlain(const Operand &op, int64_t row0, int64_t K_, bool down_)
+      : base(op.base), map(op.map ? op.map + row0 : nullptr), ld(op.ld), K(K_), down(down_) {
+    rows = down ? op.rows - row0 : dev_count(op.count, op.count_off + row0, op.rows - row0);
+    if (down) base += row0 * 4;
+    else if (!map) base += row0 * ld;
+  }
+  __device__ __forceinline__ float at(int i, int64_t k) const {
+    if (i >= rows || k >= K) return 0.f;
+    return *(const float *)(down ? base + k * ld + i * 4 : base + (map ? map[i] : i) * ld + k * 4);
+  }
+};
+
+// acc made again without the split, 4 K-values at a time from global memory. Rare and slow: it is not tuned.
+template <bool TR>
+__device__ __forceinline__ void mainloop_plain(const XPlain &a, const XPlain &b, XAcc &acc) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
+#pragma unroll
+  for (int i = 0; i < AccX::NI; ++i)
+#pragma unroll
+    for (int j = 0; j < AccX::NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int64_t k0 = 0; k0 < a.K; k0 += 4) {
+    const int64_t k = k0 + (lane >> 4);
+    float fb[AccX::NJ];
+#pragma unroll
+    for (int j = 0; j < AccX::NJ; ++j) fb[j] = b.at(wn * 32 + j * 16 + (lane & 15), k);
+#pragma unroll
+    for (int i = 0; i < AccX::NI; ++i) {
+      const float fa = a.at(wm * 128 + i * 16 + (lane & 15), k);
+#pragma unroll
+      for (int j = 0; j < AccX::NJ; ++j)
+        acc[i][j] = TR ? __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j], fa, acc[i][j], 0, 0, 0)
+                       : __builtin_amdgcn_mfma_f32_16x16x4f32(fa, fb[j], acc[i][j], 0, 0, 0);
+    }
+  }
+}
+
+// Whether an operand of the workgroup's tile had such a value (the same in every thread; a barrier): it leaves no finite
+// sum in its row or column of the tile, so one column of blocks, shared out among the waves of a row, and one row of blocks
+// tell.
+__device__ __forceinline__ bool xnonfinite(const XAcc &acc) {
+  const int wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+  float z = 0.f;
+#pragma unroll
+  for (int i = 0; i < AccX::NI; ++i)
+    if (i >> 1 == wn)
+#pragma unroll
+      for (int v = 0; v < AccX::NV; ++v) z = __builtin_fmaf(acc[i][0][v], 0.f, z);  // 0 x inf and 0 x NaN are NaN
+#pragma unroll
+  for (int j = 0; j < AccX::NJ; ++j)
+#pragma unroll
+    for (int v = 0; v < AccX::NV; ++v) z = __builtin_fmaf(acc[0][j][v], 0.f, z);
+  return __syncthreads_or(z != 0.f) != 0;
+}
+
+// The tile's sums over K of A's rows from m0 on and B's from n0 on; a K-major operand (KM_A, KM_B) as XCols.
+template <bool TR, int KM>
+__device__ __forceinline__ void xtile(const Operand &A, const Operand &B, int64_t m0, int64_t n0, int64_t K,
+                                      lds_char *smem, XAcc &acc) {
+  const int stages = __builtin_amdgcn_readfirstlane((int)cdiv(K, (int64_t)XK));
+  {
+    typename std::conditional<KM == KM_A, XCols<XM>, XRows<XM>>::type a;
+    typename std::conditional<KM == KM_B, XCols<XN>, XRows<XN>>::type b;
+    a.init(A, m0, K);
+    b.init(B, n0, K);
+    mainloop_x<TR>(a, b, stages, smem, acc);
+  }
+  if (xnonfinite(acc)) mainloop_plain<TR>(XPlain(A, m0, K, KM == KM_A), XPlain(B, n0, K, KM == KM_B), acc);
+}
+
 // Tiles of the 256 x 128 grid, shrunk by a device count that bounds M or N; the order is gemm_nt.h's.
 __device__ __forceinline__ void xtiles(const GemmShape &s, int64_t &mtiles, int64_t &ntiles) {
   mtiles = s.mtiles;
@@ -270,13 +343,7 @@ XKERNEL gemm_stats_x_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
   const int64_t m0 = (int64_t)mt * XM, n0 = (int64_t)nt * XN, nvalid = xtokens(s, n0);
   if (nvalid <= 0) return;
   XAcc acc;
-  {
-    XRows<XM> a;
-    XRows<XN> b;
-    a.init(A, m0, s.K);
-    b.init(B, n0, s.K);
-    mainloop_x<false>(a, b, (int)cdiv(s.K, (int64_t)XK), smem, acc);
-  }
+  xtile<false, KM_NONE>(A, B, m0, n0, s.K, smem, acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
   const int64_t ma = e.v0 + m0;                       // first vocabulary row of the tile
   const int valid = (int)min(e.V - ma, (int64_t)XM);  // its rows below V
@@ -329,13 +396,7 @@ XKERNEL gemm_dz_x_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
   const int64_t m0 = (int64_t)mt * XM, n0 = (int64_t)nt * XN, nvalid = xtokens(s, n0);
   if (nvalid <= 0) return;
   XAcc acc;
-  {
-    XRows<XM> a;
-    XRows<XN> b;
-    a.init(A, m0, s.K);
-    b.init(B, n0, s.K);
-    mainloop_x<false>(a, b, (int)cdiv(s.K, (int64_t)XK), (lds_char *)smem_, acc);
-  }
+  xtile<false, KM_NONE>(A, B, m0, n0, s.K, (lds_char *)smem_, acc);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
   const int64_t ma = e.v0 + m0;
   const int valid = (int)min(e.V - ma, (int64_t)XM);
@@ -452,21 +513,8 @@ XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
     B.base += k0 * B.ld;
     K = __builtin_amdgcn_readfirstlane(min(k1, (int)s.K) - k0);
   }
-  const int stages = __builtin_amdgcn_readfirstlane((int)cdiv(K, (int64_t)XK));
   XAcc acc;
-  if constexpr (KM == KM_A) {
-    XCols<XM> a;
-    XRows<XN> b;
-    a.init(A, m0, K);
-    b.init(B, n0, K);
-    mainloop_x<true>(a, b, stages, (lds_char *)smem_, acc);
-  } else {
-    XRows<XM> a;
-    XCols<XN> b;
-    a.init(A, m0, K);
-    b.init(B, n0, K);
-    mainloop_x<true>(a, b, stages, (lds_char *)smem_, acc);
-  }
+  xtile<true, KM>(A, B, m0, n0, K, (lds_char *)smem_, acc);
   if (S > 1) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     f32x4 *p = (f32x4 *)(e.split + (((int64_t)run * tiles + (int64_t)nt * mtiles + mt) * (XM * XN)) + w * (XM * XN / 8)) + lane;
