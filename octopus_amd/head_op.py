@@ -685,6 +685,22 @@ def _(kept, count, c, n_max, d, V, dtype, need_rows):
     return torch.empty(V, d, dtype=dtype, device=kept.device)
 
 
+def _later_w_setup(ctx, inputs, output):
+    kept, count, c, *sizes = inputs
+    ctx.held, ctx.sizes, ctx.like = (kept.detach(), count.detach()), sizes, (c.shape, c.dtype)
+
+
+def _later_w_backward(ctx, gout):
+    """Of c alone, the loss's gradient: the sum of gout times the weight gradient at c = 1."""
+    one = torch.ones((), dtype=torch.float32, device=gout.device)
+    unit = later_grad_w(*ctx.held, one, *ctx.sizes)
+    shape, dtype = ctx.like
+    return (None, None, (gout.float() * unit.float()).sum().reshape(shape).to(dtype)) + (None,) * len(ctx.sizes)
+
+
+torch.library.register_autograd("octohead::later_grad_w", _later_w_backward, setup_context=_later_w_setup)
+
+
 def _later_setup(ctx, inputs, output):
     rows, weight, idx = inputs[0], inputs[1], inputs[3]
     # held on ctx, not saved, as _step_setup's gradients

@@ -92,3 +92,22 @@ def test_later_weight_gradient_of_a_tree(monkeypatch):
     assert abs(a[0] - b[0]) <= 1e-6 * max(1.0, abs(b[0])) and torch.equal(a[1], b[1])
     _close(a[2], b[2], torch.bfloat16)
     _close(a[3], b[3], torch.bfloat16)
+
+
+def test_the_gradients_of_the_gradients(monkeypatch):
+    """Differentiated with respect to the loss's factor: what the step that holds its gradients gives."""
+    n, d, V = 300, 256, 2048
+    g = torch.Generator(device=DEV).manual_seed(4)
+    W = (torch.randn(V, d, generator=g, device=DEV) * 0.05).bfloat16().requires_grad_(True)
+    h = torch.randn(n, d, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    y = torch.randint(0, V, (n,), generator=g, device=DEV)
+    adv = torch.randn(n, generator=g, device=DEV)
+
+    def run():
+        loss, _ = head_op.fused_grpo_head(h, W, y, 0.7, adv, torch.ones(n, device=DEV))
+        s = torch.tensor(1.7, device=DEV, requires_grad=True)
+        gh, gw = torch.autograd.grad(s * loss, (h, W), create_graph=True)
+        return torch.autograd.grad(gw.float().square().sum() + gh.float().square().sum(), s)[0]
+
+    a, b = _both(run, monkeypatch)
+    assert abs(a - b) <= 2.0 ** -8 * abs(b)  # gradients rounded to bf16 once or twice
