@@ -360,18 +360,18 @@ int octo_head_step_grpo_pairs(const void *h, int64_t h_rows, int64_t ldh, int h_
                               void *ws, size_t ws_bytes, void *stream);
 
 /* octo_head_step_grpo (flat_pair NULL) or octo_head_step_grpo_pairs (flat_pair given, out2 its out_flat) in two calls:
- * the first leaves out grad_w, and octo_head_later_grad_w makes grad_W times c = *c (read on the device) of the buffer
- * the first one worked in, which the caller keeps, and of nothing else; the buffer is left as it was. One row pass of
- * BF16 or F16 weights; octo_head_later_bytes gives the buffer's size (need_gh: with a grad_h), 0 for a call that takes
- * more (OCTO_EUNSUPPORTED from the others). No counterpart in the reference: the gradient of a loss that is scaled
- * afterwards need not be written, read and written again. */
-int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *bytes);
+ * the first leaves out grad_w and leaves its operands, dz and h^T, in `kept`, and octo_head_later_grad_w makes grad_W times
+ * c = *c (read on the device) of that buffer and of nothing else; the buffer is left as it was. One row pass of BF16 or
+ * F16 weights; octo_head_later_bytes gives the sizes of the buffer and of the first call's workspace (need_gh: with a
+ * grad_h), 0 for a call that takes more (OCTO_EUNSUPPORTED from the others). No counterpart in the reference: the
+ * gradient of a loss that is scaled afterwards need not be written, read and written again. */
+int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *kept_bytes, size_t *ws_bytes);
 int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
                          int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
                          int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
                          const int64_t *flat_pair, int64_t n_flat, float *out2, int64_t ld_out2,
                          const octo_grpo_tail *grpo, void *grad_h, int64_t ld_gh, int gh_dtype, void *kept,
-                         size_t kept_bytes, void *stream);
+                         size_t kept_bytes, void *ws, size_t ws_bytes, void *stream);
 int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype, int need_gh,
                            const float *c, void *grad_w, int gw_dtype, void *stream);
 

@@ -60,9 +60,10 @@ SIGNATURES = {
     "octo_head_step_grpo_pairs": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _p, _i64, _i32, _i32, _i32,
                                   _f32, _f32, _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail),
                                   _p, _i64, _i32, _p, _i32, _p, _sz, _p],
-    "octo_head_later_bytes": [_i64, _i32, _i32, _i32, _i32, ctypes.POINTER(_sz)],
+    "octo_head_later_bytes": [_i64, _i32, _i32, _i32, _i32, ctypes.POINTER(_sz), ctypes.POINTER(_sz)],
     "octo_head_step_later": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
-                             _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail), _p, _i64, _i32, _p, _sz, _p],
+                             _f32, _i32, _p, _p, _i64, _p, _i64, ctypes.POINTER(GrpoTail), _p, _i64, _i32, _p, _sz, _p,
+                             _sz, _p],
     "octo_head_later_grad_w": [_p, _p, _i64, _i32, _i32, _i32, _i32, _p, _p, _i32, _p],
     "octo_head_fwd_logits": [_p, _i64, _i64, _i32, _p, _i64, _i32, _p, _p, _p, _i64, _i32, _i32, _i32, _f32, _f32,
                              _f32, _i32, _p, _p, _i64, _p, _i64, _i64, _p, _sz, _p],
@@ -144,10 +145,19 @@ def bwd_plan(n_max: int, d: int, V: int, w_dtype: int, flags: int, ws_bytes: int
 
 
 def later_bytes(n_max: int, d: int, V: int, w_dtype: int, need_gh: bool) -> int:
-    """The buffer octo_head_step_later works in and its caller keeps; 0 for a call it does not take."""
-    out = _sz(0)
-    call("octo_head_later_bytes", n_max, d, V, w_dtype, int(need_gh), ctypes.byref(out))
-    return out.value
+    """The buffer octo_head_step_later leaves to its caller; 0 for a call it does not take."""
+    return _later_sizes(n_max, d, V, w_dtype, need_gh)[0]
+
+
+def later_workspace_bytes(n_max: int, d: int, V: int, w_dtype: int, need_gh: bool) -> int:
+    """octo_head_step_later's own workspace."""
+    return _later_sizes(n_max, d, V, w_dtype, need_gh)[1]
+
+
+def _later_sizes(n_max: int, d: int, V: int, w_dtype: int, need_gh: bool) -> tuple[int, int]:
+    kept, ws = _sz(0), _sz(0)
+    call("octo_head_later_bytes", n_max, d, V, w_dtype, int(need_gh), ctypes.byref(kept), ctypes.byref(ws))
+    return kept.value, ws.value
 
 
 def timing_read(kernel: str) -> tuple[int, float]:

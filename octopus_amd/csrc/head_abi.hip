@@ -401,13 +401,13 @@ struct StepPairs {
   int64_t ld_out;
 };
 
-// later: without grad_W (grad_w NULL), its operands left in the workspace (later_plan).
+// later: without grad_W (grad_w NULL), its operands left there (later_plan).
 int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw, int w_dtype,
               const float *w_scale, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
               int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *logp, float *ent,
               float *lse, float *out2, int64_t ld_out2, const octo_grpo_tail *gt, void *grad_h, int64_t ld_gh,
               int gh_dtype, void *grad_w, int gw_dtype, void *ws, size_t ws_bytes, void *stream,
-              const StepPairs *pm = nullptr, bool later = false) {
+              const StepPairs *pm = nullptr, void *later = nullptr) {
   Common cm;
   int rc = check_common(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, n_max, d, V, flags, inv_T,
                         pre, post, use_tanh, cm);
@@ -449,10 +449,12 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
   }
   StepLayout L;
   if (later) {
-    if (cm.gather || !later_plan(n_max, d, V, w_dtype, need_gh, L))
+    LaterLayout K;
+    if (cm.gather || !later_plan(n_max, d, V, w_dtype, need_gh, K))
       return octo_fail(OCTO_EUNSUPPORTED, "head_step_later: not for this call");
+    L = K.step;
     if (!ws || ws_bytes < L.total)
-      return octo_fail(OCTO_EWORKSPACE, "head_step_later: buffer %zu < %zu bytes", ws ? ws_bytes : (size_t)0, L.total);
+      return octo_fail(OCTO_EWORKSPACE, "head_step_later: workspace %zu < %zu bytes", ws ? ws_bytes : (size_t)0, L.total);
   } else if (!ws || !step_plan_for(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, ws_bytes, L)) {
     StepLayout Lmin;
     size_t least = 0;
@@ -464,10 +466,10 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
                      cm.gather ? " (hidden of 2 GiB or more through idx: query with OCTO_WS_GATHER)" : "");
   }
   hipStream_t st = (hipStream_t)stream;
-  char *wsb = (char *)ws;
+  char *wsb = (char *)ws, *keep = later ? (char *)later : wsb;
   f32x4 *part = (f32x4 *)(wsb + L.part);
   float *z = (float *)(wsb + L.z), *hit = (float *)(wsb + L.hit), *gacc = (float *)(wsb + L.gacc);
-  void *ht = wsb + L.ht, *dz = wsb + L.dz, *wt = wsb + L.wt;
+  void *ht = keep + L.ht, *dz = keep + L.dz, *wt = wsb + L.wt;
   const int esz = L.esz;
 
   rc = launch_grpo_count(gt->mask, gt->n_tokens, z, gt->loss, st);  // Z, and the loss zeroed
@@ -913,10 +915,12 @@ int octo_head_step_grpo_pairs(const void *h, int64_t h_rows, int64_t ldh, int h_
                    gh_dtype, grad_w, gw_dtype, ws, ws_bytes, stream, &pm);
 }
 
-int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *bytes) {
-  OCTO_CHECK_ARG(bytes && n_max >= 0 && d > 0 && V > 0, "head_later_bytes: bad arguments");
-  StepLayout L;
-  *bytes = later_plan(n_max, d, V, w_dtype, need_gh != 0, L) ? L.total : 0;
+int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *kept_bytes, size_t *ws_bytes) {
+  OCTO_CHECK_ARG(kept_bytes && ws_bytes && n_max >= 0 && d > 0 && V > 0, "head_later_bytes: bad arguments");
+  LaterLayout K;
+  const bool ok = later_plan(n_max, d, V, w_dtype, need_gh != 0, K);
+  *kept_bytes = ok ? K.kept : 0;
+  *ws_bytes = ok ? K.step.total : 0;
   return OCTO_OK;
 }
 
@@ -925,19 +929,26 @@ int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype
                          int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
                          const int64_t *flat_pair, int64_t n_flat, float *out2, int64_t ld_out2,
                          const octo_grpo_tail *grpo, void *grad_h, int64_t ld_gh, int gh_dtype, void *kept,
-                         size_t kept_bytes, void *stream) {
+                         size_t kept_bytes, void *ws, size_t ws_bytes, void *stream) {
   OCTO_CHECK_ARG(!flat_pair || idx, "head_step_later: pair rows without idx");
   OCTO_CHECK_ARG(n_max > 0, "head_step_later: no rows");
+  LaterLayout K;
+  if (d <= 0 || V <= 0 || !later_plan(n_max, d, V, w_dtype, grad_h != nullptr, K))
+    return octo_fail(OCTO_EUNSUPPORTED, "head_step_later: not for this call");
+  OCTO_CHECK_ARG(kept && (uintptr_t)kept % 16 == 0, "head_step_later: null or misaligned buffer");
+  if (kept_bytes < K.kept)
+    return octo_fail(OCTO_EWORKSPACE, "head_step_later: buffer %zu < %zu bytes", kept_bytes, K.kept);
   const StepPairs pm{flat_pair, n_flat, out2, ld_out2};
   return head_step(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T,
                    pre, post, use_tanh, nullptr, nullptr, lse, flat_pair ? nullptr : out2, flat_pair ? 2 : ld_out2, grpo,
-                   grad_h, ld_gh, gh_dtype, nullptr, OCTO_F32, kept, kept_bytes, stream, flat_pair ? &pm : nullptr, true);
+                   grad_h, ld_gh, gh_dtype, nullptr, OCTO_F32, ws, ws_bytes, stream, flat_pair ? &pm : nullptr, kept);
 }
 
 int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype, int need_gh,
                            const float *c, void *grad_w, int gw_dtype, void *stream) {
-  StepLayout L;
-  if (d <= 0 || d % 8 || V <= 0 || !later_plan(n_max, d, V, w_dtype, need_gh != 0, L))
+  LaterLayout K;
+  const StepLayout &L = K.step;
+  if (d <= 0 || d % 8 || V <= 0 || !later_plan(n_max, d, V, w_dtype, need_gh != 0, K))
     return octo_fail(OCTO_EUNSUPPORTED, "head_later_grad_w: not for this call");
   OCTO_CHECK_ARG(kept && c && grad_w, "head_later_grad_w: null pointer");
   OCTO_CHECK_ARG(gw_dtype == OCTO_BF16 || gw_dtype == OCTO_F16 || gw_dtype == OCTO_F32, "head_later_grad_w: dtype");

@@ -371,15 +371,26 @@ inline bool step_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh
   return false;
 }
 
-// The step without grad_W, whose operands (dz and the pass's h^T) stay in the workspace for octo_head_later_grad_w: one
-// pass of 16-bit weights within the staging budget. grad_h's partial tiles, one round of the CUs at most, lie behind.
-inline bool later_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, StepLayout &L) {
+// The step without grad_W, whose operands stay in a buffer of the caller's for octo_head_later_grad_w: one pass of 16-bit
+// weights within the staging budget. Kept: dz [P, V_pad] and h^T [d, P], nothing else. What only the step itself needs
+// (statistics, W^T, grad_h's partial tiles, one round of the CUs at most) is a workspace that ends with the call.
+struct LaterLayout {
+  StepLayout step;  // its dz and ht lie in the kept buffer, its total is the workspace
+  size_t kept;
+};
+inline bool later_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, LaterLayout &K) {
+  StepLayout &L = K.step;
   if ((w_dtype != OCTO_BF16 && w_dtype != OCTO_F16) || n_max <= 0) return false;
-  if (!step_plan(n_max, d, V, w_dtype, need_gh, true, false, kStagingBudget, L, false, false) || L.passes != 1) return false;
+  if (!step_plan(n_max, d, V, w_dtype, need_gh, false, false, kStagingBudget, L, false, false) || L.passes != 1) return false;
+  const size_t dz = align_up((size_t)L.P * L.V_pad * L.esz);
+  L.wt -= dz;  // behind dz in the step's own workspace
+  L.split = L.total - dz;
   L.split_items = need_gh ? gradh_split(L.P, d, V, true) : 0;
   if (L.split_items > octo_tiles::kCus) L.split_items = octo_tiles::kCus;
-  L.split = L.total;
-  L.total += L.split_items * kSplitTile;
+  L.total = L.split + L.split_items * kSplitTile;
+  L.dz = 0;
+  L.ht = dz;
+  K.kept = dz + align_up((size_t)d * L.P * L.esz);
   return true;
 }
 

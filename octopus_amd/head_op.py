@@ -600,11 +600,11 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
 # V 151,936 1,005 and 772; 1,351 at d 2304, V 64,000 (f16) 1,238 and 1,199; 3,000 at d 2560, V 151,936 6,434 and 6,850.
 _LATER_WEIGHTS = 1 << 25
 _LATER_ROWS = 1536
+_LATER_SHARE = 1  # what is kept takes at most this many times the bytes of the weight gradient held otherwise
 
 
 def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows: bool, need_weight: bool) -> int:
-    """The buffer of a step whose weight gradient is left to the backward, 0 where it is not. At most twice as many rows as
-    the hidden width: what is kept, dz, then takes at most twice the bytes of the weight gradient that would be."""
+    """The bytes of the buffer (dz and h^T) of a step whose weight gradient is left to the backward, 0 where it is not."""
     if not need_weight or STEP_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not rows.is_cuda:
         return 0
     if rows.dim() != 2 or weight.dim() != 2 or weight.numel() < _LATER_WEIGHTS or rows.dtype != weight.dtype:
@@ -613,9 +613,11 @@ def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows:
         return 0
     V, d = weight.shape
     n = idx.numel() if idx is not None else rows.shape[0]
-    if not 0 < n <= min(_LATER_ROWS, 2 * d) or (idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff):
+    if not 0 < n <= _LATER_ROWS or (
+            idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff):
         return 0
-    return _lib.later_bytes(n, d, V, _dtype_code(weight), need_rows)
+    nbytes = _lib.later_bytes(n, d, V, _dtype_code(weight), need_rows)
+    return nbytes if nbytes <= _LATER_SHARE * weight.numel() * 2 else 0
 
 
 @torch.library.custom_op("octohead::head_step_later", mutates_args=(), device_types="cuda")
@@ -646,13 +648,14 @@ def head_step_later(rows: Tensor, weight: Tensor, labels: Tensor, idx: Optional[
                          _p(g), _p(loss))
     code = _dtype_code(weight2)
     kept = _workspace(nbytes, rows2)
+    ws = _workspace(_lib.later_workspace_bytes(n_max, d, V, code, need_rows), rows2)
     gh = None
     if need_rows:  # compact-order rows; scattered into grad_rows below
         gh = grad_rows if idx is None else torch.empty(n_max, d, dtype=rows2.dtype, device=dev)
     _lib.call("octo_head_step_later", _p(rows2), rows2.shape[0], rows2.stride(0), code, _p(weight2), weight2.stride(0),
               code, _p(labels), _p(idx), _p(count), n_max, d, V, flags, inv_T, pre, post, int(use_tanh), _p(lse),
-              _p(flat_pair), n_out, _p(out), 2, ctypes.byref(tail), _p(gh), d, code, _p(kept), kept.numel(),
-              _stream(rows2))
+              _p(flat_pair), n_out, _p(out), 2, ctypes.byref(tail), _p(gh), d, code, _p(kept), kept.numel(), _p(ws),
+              ws.numel(), _stream(rows2))
     if need_rows and idx is not None:
         _lib.call("octo_rows_scatter", _p(gh), d, code, _p(idx), _p(count), n_max, d, _p(grad_rows),
                   grad_rows.stride(0), code, 0, _stream(rows2))

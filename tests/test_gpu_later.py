@@ -11,10 +11,14 @@ DEV = "cuda"
 
 
 def _both(run, monkeypatch):
-    got = []
+    got, routes = [], []
+    later_bytes = head_op._later_bytes
+    monkeypatch.setattr(head_op, "_LATER_SHARE", 1 << 20)
+    monkeypatch.setattr(head_op, "_later_bytes", lambda *a: routes.append(later_bytes(*a)) or routes[-1])
     for least in (0, 1 << 62):
         monkeypatch.setattr(head_op, "_LATER_WEIGHTS", least)
         got.append(run())
+    assert len(routes) == 2 and routes[0] > 0 and routes[1] == 0
     return got
 
 

@@ -88,3 +88,15 @@ def test_out_of_memory_recomputes(monkeypatch):
             assert not _kept(head_op.fused_head(*operands, 1.0))
         assert head_op._Room._taken[operands[0].device] == 0
         assert _kept(head_op.fused_head(*operands, 1.0))
+
+
+@pytest.mark.parametrize("n,d,V", [(64, 1024, 50257), (300, 4096, 50257), (1536, 1024, 50257), (1536, 1024, 32768),
+                                   (768, 1024, 32768), (1351, 2304, 64000), (225, 2560, 151936), (1536, 2560, 151936)])
+def test_a_step_keeps_no_more_than_the_gradient_it_would_hold(n, d, V):
+    """dz and h^T alone, whatever else the step works in (W^T where V % 64 or d % 256)."""
+    P, Vp = -(-n // 256) * 256, -(-V // 256) * 256
+    with FakeTensorMode():
+        rows, weight, _ = _operands(n, d, V)
+        kept = head_op._later_bytes(rows, weight, None, True, True)
+    assert kept <= V * d * 2
+    assert kept == (P * Vp * 2 + d * P * 2 if P * (Vp + d) <= V * d else 0)
