@@ -594,11 +594,15 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
 
 # ---- the GRPO step with its weight gradient made in the backward (octo_head_step_later) ------------------------------
 
-# From this many weights on, and up to this many rows. Scaling a held weight gradient costs a read and a write of it, 264 us
-# at 2^28.5 weights whatever the rows; leaving it to the backward costs a few launches of 5 us and, in proportion to the
-# rows, the tiles of grad_W that ran beside grad_h's in one launch. us a pass, held and left for later: 225 rows at d 2560,
-# V 151,936 1,005 and 772; 1,351 at d 2304, V 64,000 (f16) 1,238 and 1,199; 3,000 at d 2560, V 151,936 6,434 and 6,850.
-_LATER_WEIGHTS = 1 << 25
+# From this many weights on, or this many multiply-adds (n d V), and up to this many rows. Scaling a held weight gradient
+# costs a read and a write of it; leaving it to the backward costs a few launches, 12 us of host time where a call is so
+# short that the host sets the pace, and, in proportion to the rows, the tiles of grad_W that ran beside grad_h's in one
+# launch. us a forward and backward, held and left for later, bf16: d 2560, V 151,936 (2^28.5) 57 rows 861 and 569, 225
+# rows 999 and 741, 1,024 rows 2,235 and 2,019, 1,536 rows 3,106 and 2,865, 2,048 rows 3,991 and 3,784; d 2304, V 64,000
+# (2^27.1) 512 rows 562 and 472; d 1024, V 65,536 (2^26) 57 rows 319 and 334, 256 rows (2^34) 323 and 329, 768 rows
+# (2^35.6) 379 and 340; d 1024, V 32,768 (2^25) 57 rows 330 and 343, 1,024 rows (2^35) 322 and 334.
+_LATER_WEIGHTS = 1 << 27
+_LATER_WORK = 3 << 34
 _LATER_ROWS = 1536
 _LATER_SHARE = 1  # what is kept takes at most this many times the bytes of the weight gradient held otherwise
 
@@ -607,7 +611,7 @@ def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows:
     """The bytes of the buffer (dz and h^T) of a step whose weight gradient is left to the backward, 0 where it is not."""
     if not need_weight or STEP_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not rows.is_cuda:
         return 0
-    if rows.dim() != 2 or weight.dim() != 2 or weight.numel() < _LATER_WEIGHTS or rows.dtype != weight.dtype:
+    if rows.dim() != 2 or weight.dim() != 2 or rows.dtype != weight.dtype:
         return 0
     if weight.dtype not in (torch.bfloat16, torch.float16):
         return 0
@@ -615,6 +619,8 @@ def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows:
     n = idx.numel() if idx is not None else rows.shape[0]
     if not 0 < n <= _LATER_ROWS or (
             idx is not None and rows.shape[0] * max(rows.stride(0), rows.shape[1]) * 2 >= 0x7fffffff):
+        return 0
+    if weight.numel() < _LATER_WEIGHTS and n * weight.numel() < _LATER_WORK:
         return 0
     nbytes = _lib.later_bytes(n, d, V, _dtype_code(weight), need_rows)
     return nbytes if nbytes <= _LATER_SHARE * weight.numel() * 2 else 0

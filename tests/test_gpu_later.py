@@ -14,6 +14,7 @@ def _both(run, monkeypatch):
     got, routes = [], []
     later_bytes = head_op._later_bytes
     monkeypatch.setattr(head_op, "_LATER_SHARE", 1 << 20)
+    monkeypatch.setattr(head_op, "_LATER_WORK", 1 << 62)
     monkeypatch.setattr(head_op, "_later_bytes", lambda *a: routes.append(later_bytes(*a)) or routes[-1])
     for least in (0, 1 << 62):
         monkeypatch.setattr(head_op, "_LATER_WEIGHTS", least)
