@@ -439,6 +439,12 @@ def _head_backward(ctx, gout, _glse):
 torch.library.register_autograd("octohead::head_fwd", _head_backward, setup_context=_head_setup)
 
 
+def _sized(*tensors: Optional[Tensor]) -> bool:
+    """Whether the sizes are plain numbers: a traced call's symbols take the route that reads none of them, which serves
+    every size the trace is run at."""
+    return all(type(n) is int for t in tensors if t is not None for n in t.shape)
+
+
 # ---- the head with logits kept between forward and backward (octo_head_fwd_logits) ------------------------------------
 
 # Bytes of fp32 logits one call keeps, and all live ones on a device together; the rows past them are recomputed, as all
@@ -493,7 +499,7 @@ def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
     # a frozen weight has no gradient for the kept bytes to stand beside
     if not weight.requires_grad or not rows.is_cuda or rows.dim() != 2 or weight.dim() != 2:
         return 0
-    if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+    if rows.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or not _sized(rows, weight, idx):
         return 0
     n = idx.numel() if idx is not None else rows.shape[0]
     V, d = weight.shape
@@ -613,7 +619,7 @@ def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows:
         return 0
     if rows.dim() != 2 or weight.dim() != 2 or rows.dtype != weight.dtype:
         return 0
-    if weight.dtype not in (torch.bfloat16, torch.float16):
+    if weight.dtype not in (torch.bfloat16, torch.float16) or not _sized(rows, weight, idx):
         return 0
     V, d = weight.shape
     n = idx.numel() if idx is not None else rows.shape[0]

@@ -2,6 +2,7 @@
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.symbolic_shapes import DimDynamic, ShapeEnv, StatelessSymbolicContext
 from torch.utils.checkpoint import checkpoint
 
 from octopus_amd import _lib, head_op
@@ -103,3 +104,20 @@ def test_a_step_keeps_no_more_than_the_gradient_it_would_hold(n, d, V, least):
         kept = head_op._later_bytes(rows, weight, None, True, True)
     assert kept <= V * d * 2
     assert kept == (P * Vp * 2 + d * P * 2 if P * (Vp + d) <= V * d and n >= least else 0)
+
+
+def test_symbolic_sizes_take_the_routes_that_serve_any():
+    """A call traced with symbols for its sizes (make_fx, export) neither fixes them nor picks a route by them."""
+    env = ShapeEnv()
+    mode = FakeTensorMode(shape_env=env)
+    dynamic = StatelessSymbolicContext(dynamic_sizes=[DimDynamic.DYNAMIC, DimDynamic.STATIC])
+    with FakeTensorMode() as plain:
+        rows, weight, y = _operands(V=151936)
+    assert head_op._keeps(rows, weight, None) and head_op._later_bytes(rows, weight, None, True, True)
+    rows, weight = (mode.from_tensor(torch.empty(t.shape, dtype=t.dtype, device="meta"), symbolic_context=dynamic)
+                    for t in (rows, weight))
+    with mode:
+        rows, weight = (torch.empty(t.shape, dtype=t.dtype, device="cuda", requires_grad=True) for t in (rows, weight))
+        assert not isinstance(rows.shape[0], int)
+        assert head_op._keeps(rows, weight, None) == head_op._later_bytes(rows, weight, None, True, True) == 0
+    assert not env.guards
