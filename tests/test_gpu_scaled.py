@@ -1,6 +1,6 @@
 """octohead::scaled, the fused step's backward: c x in fp32 rounded once, against the same arithmetic in torch, bit for
-bit, over vector lengths around the kernel's 16-byte chunks and its grid's stride; and a retained graph's second
-backward, which finds the held gradients as the first did."""
+bit, over vector lengths around the kernel's 16-byte chunks and its workgroups' 1,024; the in-place form, which walks the
+vector; and a retained graph's second backward, which finds the held gradients as the first did."""
 
 import pytest
 import torch
@@ -18,6 +18,34 @@ def test_scaled_rounds_the_fp32_product_once(n, dtype):
     for c in (1.0, -2.0, 1 / 3):
         c = torch.tensor(c, device="cuda")
         assert torch.equal(head_op.scaled(x, c), (x.float() * c).to(dtype))
+
+
+# the in-place form walks the vector with 2,048 workgroups of 256 threads and 4 loads in flight: lengths around one load of
+# every thread, around all four, and past them
+_WALK = 2048 * 256
+
+
+@pytest.mark.parametrize("dtype,per", [(torch.bfloat16, 8), (torch.float16, 8), (torch.float32, 4)])
+@pytest.mark.parametrize("chunks,over", [(0, 3), (1, 0), (_WALK, -1), (_WALK, 5), (4 * _WALK, 5), (5 * _WALK, 1)])
+def test_scale_add_in_place(chunks, over, dtype, per):
+    """y = c y + x, formed in fp32 and rounded once; x left out while skip is set, or not given at all."""
+    n = chunks * per + over
+    g = torch.Generator(device="cuda").manual_seed(n)
+    y, x = (torch.randn(n, generator=g, device="cuda").to(dtype) for _ in range(2))
+    on, off = (torch.tensor([k], dtype=torch.int32, device="cuda") for k in (0, 1))
+    for c in (1.0, -1.7):
+        c = torch.tensor([c], device="cuda")
+        for rest, skip in ((None, None), (x, None), (x, on), (x, off)):
+            got = head_op._scale_add(y.clone(), rest, c, skip)
+            want = c.double() * y.double()
+            if rest is not None and skip is not off:
+                want += x.double()
+            # 64-bit sums rounded to fp32, and then to 16 bits: a sum next to a tie of the two roundings may fall either way
+            want = want.float()
+            if dtype == torch.float32:
+                assert ((got - want).abs() <= want.abs() * 2.0 ** -23).all()
+            else:
+                assert torch.equal(got, want.to(dtype))
 
 
 def test_a_retained_graph_gives_its_gradients_twice():
