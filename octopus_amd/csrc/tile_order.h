@@ -65,8 +65,9 @@ constexpr bool tile_at(int group_m, int x, int k, int mtiles, int ntiles, int &m
 // kSplitCost stages of time to write and sum: 256 KB each way at 5 TB/s over 256 CUs, against 1.25 us a stage), and
 // tiles x S stays within cap, the partial tiles the workspace holds.
 //   beside grad_W (alone = false): the short tiles fill any CU the long ones leave, so a run need only be no longer
-//     than a CU's share of both products, tiles x nk / 128 stages: S = ceil(144 / tiles), none from 112 tiles on (at
-//     120 tiles three runs per tile took 0.13 ms of 5.7 longer: their partial tiles' traffic, nothing evened out).
+//     than a CU's share of both products, tiles x nk / 128 stages: S = ceil(144 / tiles), none from 144 tiles on. us a
+//     step and its backward, unsplit and in two runs, at d 2560, V 151,936: 120 tiles 6,044 and 6,019, 130 tiles 6,720
+//     and 6,518, 140 tiles 7,076 and 6,951; 112 tiles at d 4096, V 128,256 5,001 and 4,905.
 //   alone: whole rounds of the 256 CUs count, r of them with S = floor(256 r / tiles) runs, each run nk / S stages and
 //     its partial tile: the cheapest of r = 1 .. 4 and of no split (120 tiles: r = 1, S = 2, half of the time; 200
 //     tiles: r = 4, S = 5, 0.83 of it; 250 tiles: none).
@@ -79,7 +80,7 @@ constexpr int k_splits(int tiles, int nk, bool alone, int cap) {
   if (most > cap / tiles) most = cap / tiles;
   if (most < 2) return 1;
   if (!alone) {
-    const int s = tiles >= 112 ? 1 : (144 + tiles - 1) / tiles;
+    const int s = (144 + tiles - 1) / tiles;
     return s < most ? s : most;
   }
   int best = 1, cost = ((tiles + kCus - 1) / kCus) * nk;

@@ -27,6 +27,7 @@ def _rel(a, b):
 @pytest.mark.parametrize("n,d,V,dtype", [
     (1, 64, 8192, torch.bfloat16), (255, 264, 5120, torch.bfloat16), (257, 256, 6400, torch.float16),
     (513, 520, 5001, torch.bfloat16), (300, 512, 12800, torch.bfloat16),
+    (2945, 2560, 2048, torch.bfloat16),  # 120 tiles: two runs beside grad_W too
 ], ids=str)
 def test_runs_sum_to_the_unsplit_product(route, n, d, V, dtype):
     gen = torch.Generator().manual_seed(n + V)
