@@ -88,6 +88,31 @@ static void check_step(const StepLayout &L, int64_t n_max, int d, int V, int w_d
     CHECK(round_to(V, 64) == V && d % kTile == 0, "step W K-major: V %d d %d", V, d);
 }
 
+// The step without grad_W: its workspace, and the buffer that is kept.
+static void check_later(int64_t n, int d, int V, int w_dtype, bool need_gh) {
+  LaterLayout K;
+  if (!later_plan(n, d, V, w_dtype, need_gh, K)) return;
+  const StepLayout &L = K.step;
+  const size_t dz = (size_t)L.P * L.V_pad * 2, ht = (size_t)d * L.P * 2;
+  check_regions({{"part", L.part, (size_t)L.P * L.mtiles * kStat4},
+                 {"z", L.z, 4},
+                 {"hit", L.hit, (size_t)L.P * 4},
+                 {"rowout", L.rowout, (size_t)n * 8},
+                 {"g64", L.g64, (size_t)L.P * 8},
+                 {"xoff", L.xoff, (size_t)n * 4},
+                 {"tdot", L.tdot, (size_t)n * 4},
+                 {"xuse", L.xuse, (size_t)L.P * 4},
+                 {"scale", L.scale, (size_t)L.P * 4},
+                 {"flags", L.flags, (size_t)(1 + L.P) * 4},
+                 {"wt", L.wt, need_gh && !gh_reads_w(d, V, w_dtype) ? (size_t)d * L.V_pad * 2 : 0},
+                 {"split", L.split, (size_t)L.split_items << 18}},
+                L.total, "later workspace", n, d, V);
+  check_regions({{"dz", L.dz, dz}, {"ht", L.ht, ht}}, K.kept, "later buffer", n, d, V);
+  CHECK(K.kept <= align_up(dz) + align_up(ht), "later buffer %zu", K.kept);
+  CHECK(L.passes == 1 && L.P >= n, "later rows: P %lld n %lld", (long long)L.P, (long long)n);
+  if (need_gh && !L.wt_on) CHECK(round_to(V, 64) == V && d % kTile == 0, "later W K-major: V %d d %d", V, d);
+}
+
 static void check_bwd(const BwdLayout &L, int64_t n_max, int d, int V, int w_dtype, bool need_gh, bool need_gw,
                       bool gather) {
   const size_t esz = L.esz, hesz = w_dtype == OCTO_FP8E4M3 ? 2 : elem_bytes(w_dtype);
@@ -236,6 +261,7 @@ int main() {
                   }
                 }
               }
+              if (gw && !gather && n > 0) check_later(n, d, V, dt, gh);
               StepLayout S0;
               if (n <= 32768 && step_plan(n, d, V, dt, gh, gw, gather, kStagingBudget, S0)) {
                 for (size_t ws : {S0.total, S0.total / 3, (size_t)(64 << 20)}) {
