@@ -100,15 +100,15 @@ int octo_timing_enable(int on);
 int octo_timing_read(const char *kernel, int *launches, double *total_ms);
 
 /* Workspace bytes for octo_head_fwd (flags without OCTO_WS_BACKWARD) or octo_head_bwd
- * (OCTO_WS_BACKWARD [| OCTO_WS_NO_GRADW | OCTO_WS_NO_GRADH]) at n_max rows, width d, vocabulary V. With idx, a hidden matrix of
- * 2 GiB or more (h_rows * ldh * element bytes >= 2^31) is first gathered into the workspace (the GEMMs address
- * mapped rows with 32-bit offsets): add OCTO_WS_GATHER for those calls.
+ * (OCTO_WS_BACKWARD [| OCTO_WS_NO_GRADW | OCTO_WS_NO_GRADH]) at n_max rows, width d, vocabulary V. With idx, a hidden
+ * matrix of 2 GiB or more (h_rows * ldh * element bytes >= 2^31) is first gathered into the workspace (the GEMMs
+ * address mapped rows with 32-bit offsets): add OCTO_WS_GATHER for those calls.
  * Backward: the size of its plan at a 2 GiB staging budget (see octo_head_bwd); a smaller workspace is accepted
  * down to the plan at a 1 MiB budget, a larger one may run fewer chunks. Both gradient sizes hold room for fp32
- * partial tiles of grad_h where few rows make it worth splitting its contraction over V (it runs unsplit without). OCTO_WS_STEP [| OCTO_WS_NO_GRADW |
- * OCTO_WS_NO_GRADH]: for octo_head_step_grpo and octo_head_step_grpo_pairs (n_max = the pair rows), whose plan has
- * row passes only, each pass's [rows, V] exponentials within the 2 GiB staging budget (a larger workspace runs larger
- * passes); for fp32 operands the larger of the forward's and the backward's. */
+ * partial tiles of grad_h where few rows make it worth splitting its contraction over V (it runs unsplit without).
+ * OCTO_WS_STEP [| OCTO_WS_NO_GRADW | OCTO_WS_NO_GRADH]: for octo_head_step_grpo and octo_head_step_grpo_pairs (n_max =
+ * the pair rows), whose plan has row passes only, each pass's [rows, V] exponentials within the 2 GiB staging budget
+ * (a larger workspace runs larger passes); for fp32 operands the larger of the forward's and the backward's. */
 int octo_head_workspace_bytes(int64_t n_max, int d, int V, int w_dtype, int flags, size_t *bytes);
 
 /* The chunking octo_head_bwd runs in ws_bytes of workspace (a planning aid; no counterpart in the reference):
@@ -177,12 +177,12 @@ int octo_head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype,
                   void *grad_h, int64_t ld_gh, int gh_dtype, void *grad_w, int gw_dtype,
                   void *ws, size_t ws_bytes, void *stream);
 
-/* octo_head_fwd and octo_head_bwd without the logits' recompute for the first logit_rows compact rows (a multiple of 256,
- * padding included): the forward leaves their fp32 logits (tanh(pre z) with the soft-cap) in logits [logit_rows,
- * ld_logits], ld_logits >= V rounded up to 256, a multiple of 4, 16-byte aligned; the backward reads dz off them and leaves
- * them as they were, for another backward. Arguments, workspaces and results (to the bit) as theirs; bf16 operands. The
- * logits are those of the forward's weights: a caller that changes the weights in between calls octo_head_bwd.
- * No counterpart in the reference, which keeps or recomputes the logits. */
+/* octo_head_fwd and octo_head_bwd without the logits' recompute for the first logit_rows compact rows (a multiple of
+ * 256, padding included): the forward leaves their fp32 logits (tanh(pre z) with the soft-cap) in logits [logit_rows,
+ * ld_logits], ld_logits >= V rounded up to 256, a multiple of 4, 16-byte aligned; the backward reads dz off them and
+ * leaves them as they were, for another backward. Arguments, workspaces and results (to the bit) as theirs; bf16
+ * operands. The logits are those of the forward's weights: a caller that changes the weights in between calls
+ * octo_head_bwd. No counterpart in the reference, which keeps or recomputes the logits. */
 int octo_head_fwd_logits(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
                          int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
                          int d, int V, int flags, float inv_T, float pre, float post, int use_tanh, float *lse,
@@ -242,9 +242,9 @@ int octo_rows_scatter(const void *src, int64_t ld_src, int src_dtype, const int6
 
 /* y[i] = c y[i] + x[i] for i < n, with c = *c read on the device, formed in fp32 and rounded once to dtype (BF16, F16
  * or F32); while skip_x is given and *skip_x != 0, or x is NULL, x counts as zero and is not read (c = 1 then leaves y
- * as it is at once). y and x 16-byte aligned. No counterpart in the reference, whose autograd sums the chunks' gradients: the
- * backward of the bound GRPO step (octopus_amd/head_op.py) uses it to scale the gradients its forward computed by the
- * incoming gradient's multiple of the head's own GRPO weight and add the backward of the rest. */
+ * as it is at once). y and x 16-byte aligned. No counterpart in the reference, whose autograd sums the chunks'
+ * gradients: the backward of the bound GRPO step (octopus_amd/head_op.py) uses it to scale the gradients its forward
+ * computed by the incoming gradient's multiple of the head's own GRPO weight and add the backward of the rest. */
 int octo_scale_add(void *y, const void *x, int dtype, int64_t n, const float *c, const int32_t *skip_x,
                    void *stream);
 
@@ -360,11 +360,11 @@ int octo_head_step_grpo_pairs(const void *h, int64_t h_rows, int64_t ldh, int h_
                               void *ws, size_t ws_bytes, void *stream);
 
 /* octo_head_step_grpo (flat_pair NULL) or octo_head_step_grpo_pairs (flat_pair given, out2 its out_flat) in two calls:
- * the first leaves out grad_w and leaves its operands, dz and h^T, in `kept`, and octo_head_later_grad_w makes grad_W times
- * c = *c (read on the device) of that buffer and of nothing else; the buffer is left as it was. One row pass of BF16 or
- * F16 weights; octo_head_later_bytes gives the sizes of the buffer and of the first call's workspace (need_gh: with a
- * grad_h), 0 for a call that takes more (OCTO_EUNSUPPORTED from the others). No counterpart in the reference: the
- * gradient of a loss that is scaled afterwards need not be written, read and written again. */
+ * the first leaves out grad_w and leaves its operands, dz and h^T, in `kept`, and octo_head_later_grad_w makes grad_W
+ * times c = *c (read on the device) of that buffer and of nothing else; the buffer is left as it was. One row pass of
+ * BF16 or F16 weights; octo_head_later_bytes gives the sizes of the buffer and of the first call's workspace (need_gh:
+ * with a grad_h), 0 for a call that takes more (OCTO_EUNSUPPORTED from the others). No counterpart in the reference:
+ * the gradient of a loss that is scaled afterwards need not be written, read and written again. */
 int octo_head_later_bytes(int64_t n_max, int d, int V, int w_dtype, int need_gh, size_t *kept_bytes, size_t *ws_bytes);
 int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const void *w, int64_t ldw,
                          int w_dtype, const int64_t *labels, const int64_t *idx, const int32_t *count, int64_t n_max,
@@ -372,8 +372,8 @@ int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype
                          const int64_t *flat_pair, int64_t n_flat, float *out2, int64_t ld_out2,
                          const octo_grpo_tail *grpo, void *grad_h, int64_t ld_gh, int gh_dtype, void *kept,
                          size_t kept_bytes, void *ws, size_t ws_bytes, void *stream);
-int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype, int need_gh,
-                           const float *c, void *grad_w, int gw_dtype, void *stream);
+int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype,
+                           int need_gh, const float *c, void *grad_w, int gw_dtype, void *stream);
 
 /* GRPO/PPO policy-gradient weight per token (AReaL grpo_loss_fn semantics):
  *   ratio r = exp(logp - prox)          (prox == NULL: prox = logp, i.e. reuse_train_logp)

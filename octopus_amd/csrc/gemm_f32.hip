@@ -6,10 +6,10 @@
 // v_mfma_f32_32x32x2_f32) leave the sums no less exact, measured against 64 bits on [512, 32,000] logits of d 1024: the
 // columns 6.4e-7 off (relative) against 7.9e-7, the gradients 8e-7 against 3.2e-6. Time there: the logits and their
 // statistics 279 us with the fp32 instructions (120 TFLOP/s), 178 here (188 TFLOP/s in fp32 terms).
-// An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: its remainder is not finite,
-// and so is every sum it enters. A tile with such a sum is made again by v_mfma_f32_16x16x4_f32 from the operands as they
-// are (mainloop_plain), infinities and NaN where those products have them; to look for one costs 0.6% of those logits'
-// time. Below 2^-110 the third part loses bits.
+// An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: its remainder is not
+// finite, and so is every sum it enters. A tile with such a sum is made again by v_mfma_f32_16x16x4_f32 from the
+// operands as they are (mainloop_plain), infinities and NaN where those products have them; to look for one costs 0.6%
+// of those logits' time. Below 2^-110 the third part loses bits.
 //
 // One workgroup computes a 256 x 128 tile of C[m, n] = sum_k A[m, k] B[n, k] with 8 waves, two per SIMD, 2 x 4 of 128 x
 // 32 (AccX: the 16 x 16 block layout of the 16-bit kernels, 8 x 2 blocks). A stage is K = 32: 48 KB of fp32 go from
@@ -37,7 +37,9 @@ static_assert(2 * XSTAGE <= 160 * 1024, "LDS budget");
 struct AccX {
   static constexpr int NI = 8, NJ = 2, NV = 4, NWN = 4;
   typedef f32x4 V;
-  static __device__ __forceinline__ int row(int wm, int i, int v, int lane) { return wm * 128 + i * 16 + 4 * (lane >> 4) + v; }
+  static __device__ __forceinline__ int row(int wm, int i, int v, int lane) {
+    return wm * 128 + i * 16 + 4 * (lane >> 4) + v;
+  }
   static __device__ __forceinline__ int col(int wn, int j, int lane) { return wn * 32 + j * 16 + (lane & 15); }
 };
 typedef f32x4 XAcc[AccX::NI][AccX::NJ];
@@ -69,8 +71,8 @@ __device__ __forceinline__ void split8(const float (&x)[8], i32x4 (&p)[3]) {
   }
 }
 
-// K-contiguous rows: R rows of the tile, 4 chunks of 8 values each per stage; item q of thread t is row (512 q + t) / 4,
-// chunk t % 4, so that 4 neighbouring lanes read a row's 128 bytes.
+// K-contiguous rows: R rows of the tile, 4 chunks of 8 values each per stage; item q of thread t is row (512 q + t) /
+// 4, chunk t % 4, so that 4 neighbouring lanes read a row's 128 bytes.
 template <int R> struct XRows {
   static constexpr int Q = R * 4 / XTHREADS;
   __amdgpu_buffer_rsrc_t rs;
@@ -140,7 +142,8 @@ template <int C> struct XCols {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const bool in = col_ok[q] && k0 + e < K;
-        x[q][e] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, in ? (int)(lo[q] + e * ld) : (int)0x80000000u, 0, 0));
+        const int off = in ? (int)(lo[q] + e * ld) : (int)0x80000000u;
+        x[q][e] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
       }
     }
   }
@@ -280,9 +283,9 @@ __device__ __forceinline__ void mainloop_plain(const XPlain &a, const XPlain &b,
   }
 }
 
-// Whether an operand of the workgroup's tile had such a value (the same in every thread; a barrier): it leaves no finite
-// sum in its row or column of the tile, so one column of blocks, shared out among the waves of a row, and one row of blocks
-// tell.
+// Whether an operand of the workgroup's tile had such a value (the same in every thread; a barrier): it leaves no
+// finite sum in its row or column of the tile, so one column of blocks, shared out among the waves of a row, and one
+// row of blocks tell.
 __device__ __forceinline__ bool xnonfinite(const XAcc &acc) {
   const int wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
   float z = 0.f;
@@ -331,7 +334,7 @@ __device__ __forceinline__ int64_t xtokens(const GemmShape &s, int64_t n0) {  //
 
 #define XKERNEL __global__ __launch_bounds__(XTHREADS, 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 
-// ---- logits: softmax statistics ---------------------------------------------------------------------------------------
+// ---- logits: softmax statistics -------------------------------------------------------------------------------------
 // As gemm_stats8_kernel (head_gemm.hip) without exponentials: part[row][vocab tile] = (m_a, S, U, m_b).
 template <bool TANH>
 XKERNEL gemm_stats_x_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
@@ -386,7 +389,7 @@ XKERNEL gemm_stats_x_kernel(Operand A, Operand B, GemmShape s, StatsArgs e) {
   }
 }
 
-// ---- logits: dz -------------------------------------------------------------------------------------------------------
+// ---- logits: dz -----------------------------------------------------------------------------------------------------
 // dz = g (onehot - p) / T x post'(z), token-major [token][chunk column] fp32, zero past V.
 template <bool TANH>
 XKERNEL gemm_dz_x_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
@@ -429,7 +432,7 @@ XKERNEL gemm_dz_x_kernel(Operand A, Operand B, GemmShape s, DzArgs e) {
   }
 }
 
-// ---- gradients --------------------------------------------------------------------------------------------------------
+// ---- gradients ------------------------------------------------------------------------------------------------------
 // C = rs[row] x acc (+ addend) (+ C when accumulate), one loop with the run-time choices inside. A lane's 4 values of a
 // block are neighbours in C's row (TR). An fp32 C += acc is one no-return atomic per element (one tile adds to it per
 // launch, so the sums keep launch order).
@@ -479,8 +482,8 @@ __device__ __forceinline__ void store_x(const XAcc &acc, const StoreArgs &e, int
   }
 }
 
-// KM_B: grad_h = dz . W, its K in runs where StoreArgs::split has room (tile_order.h; partial tiles of 256 x 128, summed
-// by split_sum). KM_A: grad_W = dz^T . h from h^T.
+// KM_B: grad_h = dz . W, its K in runs where StoreArgs::split has room (tile_order.h; partial tiles of 256 x 128,
+// summed by split_sum). KM_A: grad_W = dz^T . h from h^T.
 template <int OT, int KM>
 XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
   __shared__ __attribute__((aligned(16))) char smem_[2 * XSTAGE];
@@ -491,7 +494,8 @@ XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
   if (KM == KM_B && e.split)
     S = __builtin_amdgcn_readfirstlane(octo_tiles::k_splits(tiles, nk, true, e.split_cap));
   if (S > 1) {
-    const bool in = octo_tiles::split_item_at((int)(blockIdx.x & 7), (int)(blockIdx.x >> 3), S, (int)mtiles, (int)ntiles, run, mt, nt);
+    const bool in = octo_tiles::split_item_at((int)(blockIdx.x & 7), (int)(blockIdx.x >> 3), S, (int)mtiles,
+                                              (int)ntiles, run, mt, nt);
     if (!__builtin_amdgcn_readfirstlane(in)) return;
     run = __builtin_amdgcn_readfirstlane(run);
     mt = __builtin_amdgcn_readfirstlane(mt);
@@ -517,7 +521,8 @@ XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
   xtile<true, KM>(A, B, m0, n0, K, (lds_char *)smem_, acc);
   if (S > 1) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    f32x4 *p = (f32x4 *)(e.split + (((int64_t)run * tiles + (int64_t)nt * mtiles + mt) * (XM * XN)) + w * (XM * XN / 8)) + lane;
+    const int64_t at = (int64_t)run * tiles + (int64_t)nt * mtiles + mt;
+    f32x4 *p = (f32x4 *)(e.split + at * (XM * XN) + w * (XM * XN / 8)) + lane;
 #pragma unroll
     for (int i = 0; i < AccX::NI; ++i)
 #pragma unroll
@@ -527,7 +532,7 @@ XKERNEL gemm_store_x_kernel(Operand A, Operand B, GemmShape s, StoreArgs e) {
   store_x<typename Elem<OT>::T>(acc, e, m0, n0, mvalid, nvalid);
 }
 
-// ---- host launchers ---------------------------------------------------------------------------------------------------
+// ---- host launchers -------------------------------------------------------------------------------------------------
 
 // The shape over 256 x 128 tiles.
 static GemmShape xshape(GemmShape s) {
@@ -570,7 +575,8 @@ int launch_gemm_store_f32(const Operand &A, const Operand &B, const GemmShape &s
   if (e.part || e.part_blocked || kmajor == KM_NONE || (e.split && kmajor != KM_B))
     return octo_fail(OCTO_EUNSUPPORTED, "gemm_store: this product of fp32 operands");
   const Operand &c = kmajor == KM_A ? A : B;  // the K-major operand's stage: 32 rows within 32-bit offsets
-  if (c.map || c.ld > 0x7fffffffLL / XK || c.ld % 4) return octo_fail(OCTO_EINVAL, "gemm_store: K-major operand layout");
+  if (c.map || c.ld > 0x7fffffffLL / XK || c.ld % 4)
+    return octo_fail(OCTO_EINVAL, "gemm_store: K-major operand layout");
   const GemmShape s = xshape(s0);
   switch (e.dtype) {
     case OCTO_BF16: go_store_x<OCTO_BF16>(A, B, s, e, st, kmajor); break;

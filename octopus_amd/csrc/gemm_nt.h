@@ -4,10 +4,10 @@
 //
 // One workgroup computes a 256 x 256 tile of C. The 16-bit loop runs 512 threads = 8 wave64s, two per SIMD, sat
 // 2 x 4, each owning a 128 x 64 sub-tile as 8 x 4 blocks of v_mfma_f32_16x16x32_{bf16,f16} (Acc16N<4>, 128
-// accumulation registers): while one wave of a SIMD waits on a stage the other issues MFMAs. fp32 operands have a loop of
-// their own (gemm_f32.hip). Under the part's power limit the
-// 16x16x32 form sustains 12% more bf16 FLOP/s than the 32x32x16 one on random operands (2.10 against 1.88 PFLOP/s,
-// a register-only loop on every SIMD), and each MFMA streams fewer accumulator bytes per FLOP.
+// accumulation registers): while one wave of a SIMD waits on a stage the other issues MFMAs. fp32 operands have a loop
+// of their own (gemm_f32.hip). Under the part's power limit the 16x16x32 form sustains 12% more bf16 FLOP/s than the
+// 32x32x16 one on random operands (2.10 against 1.88 PFLOP/s, a register-only loop on every SIMD), and each MFMA
+// streams fewer accumulator bytes per FLOP.
 //
 // The mainloop feeds the MFMAs from LDS: the A and B K-slices go straight from global memory into a ring of
 // LDS stages by buffer_load_dwordx4 ... lds (no register hop), with the instruction order fixed in the source:
@@ -473,8 +473,8 @@ struct Acc16N {
   }
   static __device__ __forceinline__ bool col_lane(int lane) { return lane < 16; }
 };
-// The 8-wave gradient kernels' blocks, with the MFMA operands in each other's place (ring5_stage TR): row l & 15, columns
-// 4 (l >> 4) + v, so a lane's 4 values are neighbours in a row-major C.
+// The 8-wave gradient kernels' blocks, with the MFMA operands in each other's place (ring5_stage TR): row l & 15,
+// columns 4 (l >> 4) + v, so a lane's 4 values are neighbours in a row-major C.
 struct Acc16T {
   static constexpr int NI = 8, NJ = 4, NV = 4;
   typedef f32x4 V;

@@ -162,7 +162,6 @@ Operand gemm_weight(const void *w, int64_t ldw, const Common &cm, int64_t v0, in
   return A;
 }
 
-// Hidden rows [r0, r0 + rows) of the compact order.
 // Hidden rows [r0, r0 + rows) of the compact order: through idx, or (gathered != NULL) from the contiguous copy
 // [n_max, d] of them that launch_rows_gather wrote.
 Operand hidden_operand(const void *h, int64_t ldh, const int64_t *idx, const int32_t *count, int64_t r0,
@@ -433,7 +432,8 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
     if (cm.dt == OCTO_F32) return octo_fail(OCTO_EUNSUPPORTED, "head_step_grpo_pairs: fp32 operands");
   }
   if (n_max == 0 && !pm) return OCTO_OK;
-  if (!need_gh && !need_gw && !pm && !later)  // no gradient asked for: the forward with its GRPO tail (its own workspace size)
+  // no gradient asked for: the forward with its GRPO tail (its own workspace size)
+  if (!need_gh && !need_gw && !pm && !later)
     return head_fwd(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, w_scale, labels, idx, count, n_max, d, V, flags, inv_T,
                     pre, post, use_tanh, logp, ent, lse, out2, ld_out2, gt, ws, ws_bytes, stream);
   if (cm.dt == OCTO_F32) {  // fp32: the forward, then the backward
@@ -454,7 +454,8 @@ int head_step(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, const voi
       return octo_fail(OCTO_EUNSUPPORTED, "head_step_later: not for this call");
     L = K.step;
     if (!ws || ws_bytes < L.total)
-      return octo_fail(OCTO_EWORKSPACE, "head_step_later: workspace %zu < %zu bytes", ws ? ws_bytes : (size_t)0, L.total);
+      return octo_fail(OCTO_EWORKSPACE, "head_step_later: workspace %zu < %zu bytes", ws ? ws_bytes : (size_t)0,
+                       L.total);
   } else if (!ws || !step_plan_for(n_max, d, V, w_dtype, need_gh, need_gw, cm.gather, ws_bytes, L)) {
     StepLayout Lmin;
     size_t least = 0;
@@ -940,12 +941,13 @@ int octo_head_step_later(const void *h, int64_t h_rows, int64_t ldh, int h_dtype
     return octo_fail(OCTO_EWORKSPACE, "head_step_later: buffer %zu < %zu bytes", kept_bytes, K.kept);
   const StepPairs pm{flat_pair, n_flat, out2, ld_out2};
   return head_step(h, h_rows, ldh, h_dtype, w, ldw, w_dtype, nullptr, labels, idx, count, n_max, d, V, flags, inv_T,
-                   pre, post, use_tanh, nullptr, nullptr, lse, flat_pair ? nullptr : out2, flat_pair ? 2 : ld_out2, grpo,
-                   grad_h, ld_gh, gh_dtype, nullptr, OCTO_F32, ws, ws_bytes, stream, flat_pair ? &pm : nullptr, kept);
+                   pre, post, use_tanh, nullptr, nullptr, lse, flat_pair ? nullptr : out2, flat_pair ? 2 : ld_out2,
+                   grpo, grad_h, ld_gh, gh_dtype, nullptr, OCTO_F32, ws, ws_bytes, stream, flat_pair ? &pm : nullptr,
+                   kept);
 }
 
-int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype, int need_gh,
-                           const float *c, void *grad_w, int gw_dtype, void *stream) {
+int octo_head_later_grad_w(const void *kept, const int32_t *count, int64_t n_max, int d, int V, int w_dtype,
+                           int need_gh, const float *c, void *grad_w, int gw_dtype, void *stream) {
   LaterLayout K;
   const StepLayout &L = K.step;
   if (d <= 0 || d % 8 || V <= 0 || !later_plan(n_max, d, V, w_dtype, need_gh != 0, K))
@@ -1075,7 +1077,8 @@ static int head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, con
       const Operand Aw = gemm_weight(w, ldw, cm, v0, vc, d, wsb + L.wide, st, rc);
       if (rc) return rc;
       e.v0 = v0;
-      const int64_t kr = kept.rows <= r0 ? 0 : (kept.rows - r0 < L.P ? kept.rows - r0 : L.P);  // of the pass, with logits
+      // rows of the pass whose logits are kept
+      const int64_t kr = kept.rows <= r0 ? 0 : (kept.rows - r0 < L.P ? kept.rows - r0 : L.P);
       if (kr) {
         DzLogitsArgs za{};
         za.dz = dza;
@@ -1109,7 +1112,8 @@ static int head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, con
         if (e.hit) er.hit = e.hit + kr;
         const Operand Br = kr ? hidden_operand(h, ldh, idx, count, r0 + kr, rows - kr, cm, gathered, d) : Bh;
         TimedLaunch t("gemm_dz", st);
-        rc = launch_gemm_dz(cm.dt, cm.fp8, use_tanh != 0, Aw, Br, shape(vc, rows - kr, d, kGroupM, 2, count, r0 + kr), er, st);
+        rc = launch_gemm_dz(cm.dt, cm.fp8, use_tanh != 0, Aw, Br, shape(vc, rows - kr, d, kGroupM, 2, count, r0 + kr),
+                            er, st);
       }
       if (rc) return rc;
 

@@ -37,9 +37,9 @@ __device__ __forceinline__ i32x4 pack8(const float (&x)[8], bool f16) {
   return v;
 }
 
-// 16-byte loads a lane of the merge keeps in flight per operand: a row of d 2560 at once, 320 vocabulary tiles. With few
-// rows the merge is a chain of loads (57 rows, d 2560, V 151,936: 14.9 us one at a time, 11.0 now; the sums keep their
-// order).
+// 16-byte loads a lane of the merge keeps in flight per operand: a row of d 2560 at once, 320 vocabulary tiles. With
+// few rows the merge is a chain of loads (57 rows, d 2560, V 151,936: 14.9 us one at a time, 11.0 now; the sums keep
+// their order).
 constexpr int kRowLoads = 5;
 
 // This lane's part of the fp32 dot product of hidden row hrow and weight row y (the target logit before any scale):
@@ -443,9 +443,9 @@ int launch_ex_fix(const ExFixArgs &a, hipStream_t st) {
   return OCTO_OK;
 }
 
-// ---- dz from kept logits (octo_head_bwd_logits) ----------------------------------------------------------------------
-// One workgroup per (row, 4,096 chunk columns): 2 chunks of 8 columns per thread, 32 bytes read and 16 written each. Bound
-// by memory, 6 bytes an element: [3,584, 128,256] 478 us (5.8 TB/s), in place of 2.7 ms of recompute.
+// ---- dz from kept logits (octo_head_bwd_logits) ---------------------------------------------------------------------
+// One workgroup per (row, 4,096 chunk columns): 2 chunks of 8 columns per thread, 32 bytes read and 16 written each.
+// Bound by memory, 6 bytes an element: [3,584, 128,256] 478 us (5.8 TB/s), in place of 2.7 ms of recompute.
 constexpr int kDzChunks = 2;
 template <bool TANH> __global__ __launch_bounds__(256) void dz_logits_kernel(DzLogitsArgs a) {
   const int64_t i = blockIdx.y;  // row of the pass
@@ -505,13 +505,13 @@ int launch_dz_logits(const DzLogitsArgs &a, hipStream_t st) {
   return OCTO_OK;
 }
 
-// ---- y = c s + x over a vector (the held gradients' scaling in the GRPO routes' backward) ----------------------------
+// ---- y = c s + x over a vector (the held gradients' scaling in the GRPO routes' backward) ---------------------------
 // c is read from device memory, and so is `skip_x` (when given): while it is non-zero x counts as zero and is not read.
 // x = NULL: y = c s. The product and the sum are formed in fp32 and rounded once to the vector's type. In place (s =
 // y) with c = 1 and no x to add, y is already the result and every workgroup ends at once. Bound by memory: 16 bytes
-// per load, kScaleLoads of them in flight per thread. Out of place one workgroup takes 1,024 chunks: [151,936, 2560] bf16
-// 267 us, against 1,350 us for the same arithmetic as three elementwise kernels (widen, multiply, narrow). In place, where
-// mostly there is nothing to do, 8 workgroups per CU walk the vector: 355 us, with x 545.
+// per load, kScaleLoads of them in flight per thread. Out of place one workgroup takes 1,024 chunks: [151,936, 2560]
+// bf16 267 us, against 1,350 us for the same arithmetic as three elementwise kernels (widen, multiply, narrow). In
+// place, where mostly there is nothing to do, 8 workgroups per CU walk the vector: 355 us, with x 545.
 constexpr int kScaleLoads = 4;
 __global__ __launch_bounds__(256) void scale_add_kernel(void *y, const void *src, const void *x, int dtype, int64_t n,
                                                         const float *c, const int32_t *skip_x) {
@@ -841,9 +841,9 @@ template <int DT> __device__ __forceinline__ i32x4 pack_chunk(const float (&x)[1
 // logprob is not.
 struct ColStat {
   float m = -INFINITY, S = 0.f, U = 0.f;
-  // S and U relative to a maximum -d above m. Far below it they count for nothing, and what they hold may be no number: a
-  // thread that has only seen logits masked with a finite -1e38 or lower has m = x c rounded by up to 2^103, and its e are
-  // exp2 of that. (A NaN stays: it came from a NaN or infinite logit.)
+  // S and U relative to a maximum -d above m. Far below it they count for nothing, and what they hold may be no number:
+  // a thread that has only seen logits masked with a finite -1e38 or lower has m = x c rounded by up to 2^103, and its
+  // e are exp2 of that. (A NaN stays: it came from a NaN or infinite logit.)
   __device__ __forceinline__ void shift(float d) {
     if (d < -256.f) {
       S = S == S ? 0.f : S;
@@ -868,10 +868,10 @@ struct ColStat {
   }
 };
 
-// One workgroup of 1,024 threads per row, at any number of rows: few rows are a chain of dependent steps (151,936 values
-// of bf16: 5 of 4 loads), and a row's sums keep their order, so its columns are the same to the bit beside any other
-// rows. [rows, 151,936] bf16 with 256 threads a row and with 1,024: 512 rows 33 and 31 us, 1,024 rows 57 and 55, 2,048
-// rows 109 and 105.
+// One workgroup of 1,024 threads per row, at any number of rows: few rows are a chain of dependent steps (151,936
+// values of bf16: 5 of 4 loads), and a row's sums keep their order, so its columns are the same to the bit beside any
+// other rows. [rows, 151,936] bf16 with 256 threads a row and with 1,024: 512 rows 33 and 31 us, 1,024 rows 57 and 55,
+// 2,048 rows 109 and 105.
 constexpr int kColThreads = 1024;
 template <int DT>
 __global__ __launch_bounds__(kColThreads) void columns_fwd_kernel(const void *logits, int64_t ld, const int64_t *labels,
@@ -935,8 +935,8 @@ __global__ __launch_bounds__(kColThreads) void columns_fwd_kernel(const void *lo
     }
     const float l2S = flog2(s);
     const int64_t y = labels[r];
-    // the label's logit as the sums have it, base 2 and relative to the maximum: close to a probability of 1 the logprob
-    // is far smaller than the logits, and lse's own rounding (1e-6 at 18) would be a part of it
+    // the label's logit as the sums have it, base 2 and relative to the maximum: close to a probability of 1 the
+    // logprob is far smaller than the logits, and lse's own rounding (1e-6 at 18) would be a part of it
     const float ty = (y >= 0 && y < V) ? __builtin_fmaf((float)row[y], c, -m2) : __builtin_nanf("");
     out2[2 * r] = (ty - l2S) * OCTO_LN2;
     out2[2 * r + 1] = (l2S - u / s) * OCTO_LN2;
@@ -968,7 +968,8 @@ __global__ __launch_bounds__(256) void columns_bwd_kernel(const void *logits, in
   };
   if constexpr (!VEC) {
     const int j0 = blockIdx.x * (256 * kColLoads * PER);
-    for (int j = j0 + threadIdx.x; j < min(V, j0 + 256 * kColLoads * PER); j += 256) drow[j] = (T)grad((float)row[j], j);
+    for (int j = j0 + threadIdx.x; j < min(V, j0 + 256 * kColLoads * PER); j += 256)
+      drow[j] = (T)grad((float)row[j], j);
     return;
   }
   const RowChunks rc = row_chunks<DT>(row, V);
@@ -1009,9 +1010,11 @@ static void go_columns_bwd(const void *logits, int64_t ld, const int64_t *labels
   constexpr int B = Elem<DT>::bytes;
   const dim3 grid((unsigned)cdiv(V, 256 * kColLoads * (16 / B)), (unsigned)n);
   if (((uintptr_t)logits - (uintptr_t)dl) % 16 == 0 && ((ld - ld_d) * B) % 16 == 0)
-    hipLaunchKernelGGL((columns_bwd_kernel<DT, true>), grid, dim3(256), 0, st, logits, ld, labels, V, inv_T, lse, g, dl, ld_d);
+    hipLaunchKernelGGL((columns_bwd_kernel<DT, true>), grid, dim3(256), 0, st, logits, ld, labels, V, inv_T, lse, g,
+                       dl, ld_d);
   else
-    hipLaunchKernelGGL((columns_bwd_kernel<DT, false>), grid, dim3(256), 0, st, logits, ld, labels, V, inv_T, lse, g, dl, ld_d);
+    hipLaunchKernelGGL((columns_bwd_kernel<DT, false>), grid, dim3(256), 0, st, logits, ld, labels, V, inv_T, lse, g,
+                       dl, ld_d);
 }
 
 // ---- pairs / rows plumbing -----------------------------------------------------------------------

@@ -52,10 +52,10 @@ template <int NJ> struct DzSwz<Acc16N<NJ>> {
 
 // ---- epilogue: online softmax statistics ----------------------------------------------------
 
-// The softcap's tanh of every accumulator in place, acc = tanh(pre z), with z = acc times its vocabulary row's scale for
-// fp8 weights (the tile's scales staged in LDS at wsl, 0 past V). Without the softcap nothing is done here: stats_cols
-// applies an fp8 row scale as it reads each accumulator (the same fp32 product; an in-place multiply here made the
-// compiler spill accumulators: 112-136 bytes per lane against 24).
+// The softcap's tanh of every accumulator in place, acc = tanh(pre z), with z = acc times its vocabulary row's scale
+// for fp8 weights (the tile's scales staged in LDS at wsl, 0 past V). Without the softcap nothing is done here:
+// stats_cols applies an fp8 row scale as it reads each accumulator (the same fp32 product; an in-place multiply here
+// made the compiler spill accumulators: 112-136 bytes per lane against 24).
 template <class L, bool A_FP8, bool TANH>
 __device__ __forceinline__ void pre_transform(typename L::V (&acc)[L::NI][L::NJ], int wm, int lane, float pre,
                                               const __attribute__((address_space(3))) f32x4 *wsl = nullptr) {
@@ -204,7 +204,8 @@ typedef __attribute__((address_space(3))) short lds_short;
 // fp8 weights: the accumulators are raw e4m3 products; z = acc x the row's scale (the forward's pre_transform, the same
 // fp32 multiply, so the row state still matches), and d/d(raw product) = dz x that scale. A lane's 4 consecutive rows'
 // scales are loaded once per (i, g4) and serve all its token columns (loaded per column, and once more to scale the
-// accumulators: same box, 65,536-row passes of 114,688 rows, d 2560, V 151,936, gemm_dz 35.5-35.8 against 35.1-35.5 ms).
+// accumulators: same box, 65,536-row passes of 114,688 rows, d 2560, V 151,936, gemm_dz 35.5-35.8 against 35.1-35.5
+// ms).
 template <class L, typename P2, bool TANH, bool EDGE>
 __device__ __forceinline__ void dz_stage_fp8(const typename L::V (&acc)[L::NI][L::NJ], const DzArgs &e, int64_t m0,
                                              int64_t n0, int64_t nvalid, int wm, int wn, int lane, lds_char *tile) {
@@ -327,12 +328,12 @@ __device__ __forceinline__ void dz_write(const DzArgs &e, int64_t ma, int64_t m0
 
 // ---- epilogue: plain store -------------------------------------------------------------------
 
-// C = rs[row] x acc (rs NULL: acc; x alpha) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to OT, value
-// by value: ragged and unaligned tiles, fp32 output, sums. The accumulators go through the LDS (the ring, free after the
-// mainloop) in two halves of 128 rows, so that a wave stores, adds to or reads 64 neighbours of a row; from the
-// registers it would cover 16 bytes of each of 16 rows (Acc16T), and the fp32 partials of several passes, read and
-// added to at every pass, made the step's gradients slower: 20,110 rows without a row count, d 2048, V 128,256, 26.3 ms
-// a step so, 25.3 with 64-byte pieces (Acc16N).
+// C = rs[row] x acc (rs NULL: acc; x alpha) (+ addend, fp32, row stride ld_add) (+ C when accumulate), rounded once to
+// OT, value by value: ragged and unaligned tiles, fp32 output, sums. The accumulators go through the LDS (the ring,
+// free after the mainloop) in two halves of 128 rows, so that a wave stores, adds to or reads 64 neighbours of a row;
+// from the registers it would cover 16 bytes of each of 16 rows (Acc16T), and the fp32 partials of several passes, read
+// and added to at every pass, made the step's gradients slower: 20,110 rows without a row count, d 2048, V 128,256,
+// 26.3 ms a step so, 25.3 with 64-byte pieces (Acc16N).
 // An fp32 C += acc is one no-return atomic add per element, performed in the L2, so the tile's epilogue does
 // not wait for C to be read (grad_W's fp32 partials of the fused step at 24,576 rows, d 2560, V 151,936: the gradient
 // launches 28.35 against 28.65 ms per step, same box). A launch adds to each element once (one tile), so the sums keep
@@ -381,11 +382,11 @@ __device__ __forceinline__ void store_tile(const typename L::V (&acc)[L::NI][L::
 
 // A whole-width 16-bit tile with nothing to add: through the LDS (the ring, free after the mainloop) and out in rows of
 // 512 bytes, 16 bytes per lane. Stored from the registers, as four 2-byte stores (the MFMA's own layout) or one of 8
-// bytes per block, a wave's store covers 32-byte pieces of 4 or 16 lines, and tiles of few K-stages, grad_W's of a short
-// call, spend longer storing than multiplying: at d 2560, V 151,936 and 64 rows (one stage) grad_W takes 195 us this
-// way, 264 with 2-byte and 294 with 8-byte stores; at 225 rows 298, 376 and 401; at 3,000 1,765, 1,783 and 1,811. Its
-// floor is the write of 0.78 GB, 114 us at this card's fill rate. With the operands exchanged (Acc16T) a lane's 4 values
-// go into the LDS in one write.
+// bytes per block, a wave's store covers 32-byte pieces of 4 or 16 lines, and tiles of few K-stages, grad_W's of a
+// short call, spend longer storing than multiplying: at d 2560, V 151,936 and 64 rows (one stage) grad_W takes 195 us
+// this way, 264 with 2-byte and 294 with 8-byte stores; at 225 rows 298, 376 and 401; at 3,000 1,765, 1,783 and 1,811.
+// Its floor is the write of 0.78 GB, 114 us at this card's fill rate. With the operands exchanged (Acc16T) a lane's 4
+// values go into the LDS in one write.
 template <class L, typename OT>
 __device__ __forceinline__ void store_staged(const typename L::V (&acc)[L::NI][L::NJ], const StoreArgs &e, int64_t m0,
                                              int64_t n0, int64_t mvalid, lds_char *smem) {
@@ -512,9 +513,12 @@ __device__ __forceinline__ void store8_tile(const Operand &A, const Operand &B, 
   if (mvalid <= 0 || nvalid <= 0 || adds_nothing(e, which, K_eff)) return;
   typedef Acc16T L;
   f32x4 acc[8][4];
-  if constexpr (KM == KM_A) mainloop_ring5<DT, OpColsN<8, 128>, OpRowsN<8, 64>, false, true>(A, B, m0, n0, K_eff, smem, acc);
-  else if constexpr (KM == KM_B) mainloop_ring5<DT, OpRowsN<8, 128>, OpColsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
-  else mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
+  if constexpr (KM == KM_A)
+    mainloop_ring5<DT, OpColsN<8, 128>, OpRowsN<8, 64>, false, true>(A, B, m0, n0, K_eff, smem, acc);
+  else if constexpr (KM == KM_B)
+    mainloop_ring5<DT, OpRowsN<8, 128>, OpColsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
+  else
+    mainloop_ring5<DT, OpRowsN<8, 128>, OpRowsN<8, 64>, true, true>(A, B, m0, n0, K_eff, smem, acc);
   if (KM != KM_A && part) {
     store_split<L>(acc, part);
     return;

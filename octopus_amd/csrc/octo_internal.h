@@ -41,8 +41,8 @@ struct StatsArgs {
   void *ex = nullptr;
   int64_t ldx = 0;
   const float *xoff = nullptr;  // per-token base-2 offsets of the stored exponentials (tokens of this GEMM), or NULL
-  // z != NULL (bf16 operands, no ex): the accumulators themselves (tanh(pre z) with the soft-cap) of tokens below z_rows,
-  // a multiple of 256, [z_rows, ldx] fp32, V_pad columns of each row written; launch_dz_logits reads them.
+  // z != NULL (bf16 operands, no ex): the accumulators themselves (tanh(pre z) with the soft-cap) of tokens below
+  // z_rows, a multiple of 256, [z_rows, ldx] fp32, V_pad columns of each row written; launch_dz_logits reads them.
   float *z = nullptr;
   int64_t z_rows = 0;
 };
@@ -313,9 +313,10 @@ struct DzScaleArgs {
 };
 int launch_dz_scale(const DzScaleArgs &a, hipStream_t st);
 
-// dz of a row pass over a vocabulary chunk from kept logits (StatsArgs::z), with gemm_dz's own formula and rounding: dz[i]
-// [k] for local rows i < rows (compact rows r0 + i) and chunk columns k < cols (vocabulary v0 + k; 0 from V on), the label
-// entry hit[i] (launch_hit's). Rows from the count to the next multiple of 64, which a count-bounded grad_W reads, get 0.
+// dz of a row pass over a vocabulary chunk from kept logits (StatsArgs::z), with gemm_dz's own formula and rounding:
+// dz[i][k] for local rows i < rows (compact rows r0 + i) and chunk columns k < cols (vocabulary v0 + k; 0 from V on),
+// the label entry hit[i] (launch_hit's). Rows from the count to the next multiple of 64, which a count-bounded grad_W
+// reads, get 0.
 struct DzLogitsArgs {
   void *dz;  // bf16
   int64_t ld;
@@ -338,10 +339,11 @@ int launch_dz_logits(const DzLogitsArgs &a, hipStream_t st);
 // The GRPO tail of the fused step over prefix-tree pair rows: flat token t reads its pair row p = flat_pair[t]; for
 // the pass's rows (r0 <= p < r0 + rows, below the row count) it takes the row's (logprob, entropy) from rowout (2
 // floats per compact row) into out2[t] and, when mask[t] != 0, adds its GRPO weight to its pair's sum and its loss term
-// to the loss (atomics: the last bits of the loss may vary). The pairs' sums are kept in 64 bits, g64[p - r0], zeroed by
-// the pass's merge, and rounded once to g[p]: in 32 bits the order of the additions showed in g's last bit, and where
-// a gradient lies near a tie of its 16-bit rounding, in the gradient. Tokens with no pair (p < 0 or past the count) get out2 = 0
-// in the first pass and, when masked, their loss term at logprob 0 (as the objective over the expanded columns).
+// to the loss (atomics: the last bits of the loss may vary). The pairs' sums are kept in 64 bits, g64[p - r0], zeroed
+// by the pass's merge, and rounded once to g[p]: in 32 bits the order of the additions showed in g's last bit, and
+// where a gradient lies near a tie of its 16-bit rounding, in the gradient. Tokens with no pair (p < 0 or past the
+// count) get out2 = 0 in the first pass and, when masked, their loss term at logprob 0 (as the objective over the
+// expanded columns).
 struct PairsGrpoArgs {
   const int64_t *flat_pair;
   int64_t n_flat;

@@ -198,12 +198,13 @@ inline bool bwd_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, boo
   if (L.hacc_on) off += align_up((size_t)L.P * d * sizeof(float));
   L.gacc = off;  // fp32 grad_W partial sums across passes, for a 16-bit grad_W
   if (L.gacc_on) off += align_up((size_t)V * d * sizeof(float));
-  // grad_h's split-K partial tiles, part of the staging: with one chunk, where the budget has room for them (more chunks
-  // mean rows in plenty; the default budget bounds them where the staging itself is unbounded)
+  // grad_h's split-K partial tiles, part of the staging: with one chunk, where the budget has room for them (more
+  // chunks mean rows in plenty; the default budget bounds them where the staging itself is unbounded)
   L.split = off;
   L.split_items = split && need_gh && L.esz == 2 && L.chunks == 1 ? gradh_split(L.P, d, L.Vc, true) : 0;
   if (L.split_items) {
-    const size_t staged = (size_t)L.P * L.Vc * L.esz + (wt ? (size_t)d * L.Vc * L.esz : 0) + (wide ? (size_t)L.Vc * d * 2 : 0);
+    const size_t staged = (size_t)L.P * L.Vc * L.esz + (wt ? (size_t)d * L.Vc * L.esz : 0) +
+                          (wide ? (size_t)L.Vc * d * 2 : 0);
     if (staged + L.split_items * kSplitTile > (budget ? budget : kStagingBudget)) L.split_items = 0;
   }
   off += L.split_items * kSplitTile;
@@ -371,9 +372,9 @@ inline bool step_plan_for(int64_t n_max, int d, int V, int w_dtype, bool need_gh
   return false;
 }
 
-// The step without grad_W, whose operands stay in a buffer of the caller's for octo_head_later_grad_w: one pass of 16-bit
-// weights within the staging budget. Kept: dz [P, V_pad] and h^T [d, P], nothing else. What only the step itself needs
-// (statistics, W^T, grad_h's partial tiles, one round of the CUs at most) is a workspace that ends with the call.
+// The step without grad_W, whose operands stay in a buffer of the caller's for octo_head_later_grad_w: one pass of
+// 16-bit weights within the staging budget. Kept: dz [P, V_pad] and h^T [d, P], nothing else. What only the step itself
+// needs (statistics, W^T, grad_h's partial tiles, one round of the CUs at most) is a workspace that ends with the call.
 struct LaterLayout {
   StepLayout step;  // its dz and ht lie in the kept buffer, its total is the workspace
   size_t kept;
@@ -381,7 +382,8 @@ struct LaterLayout {
 inline bool later_plan(int64_t n_max, int d, int V, int w_dtype, bool need_gh, LaterLayout &K) {
   StepLayout &L = K.step;
   if ((w_dtype != OCTO_BF16 && w_dtype != OCTO_F16) || n_max <= 0) return false;
-  if (!step_plan(n_max, d, V, w_dtype, need_gh, false, false, kStagingBudget, L, false, false) || L.passes != 1) return false;
+  if (!step_plan(n_max, d, V, w_dtype, need_gh, false, false, kStagingBudget, L, false, false) || L.passes != 1)
+    return false;
   const size_t dz = align_up((size_t)L.P * L.V_pad * L.esz);
   L.wt -= dz;  // behind dz in the step's own workspace
   L.split = L.total - dz;

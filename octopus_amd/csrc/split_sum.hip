@@ -3,7 +3,8 @@
 //
 // Bound by memory: S partial tiles of 256 KB read per tile of C. One workgroup per 16 rows of a tile, 256 threads: each
 // wave reads its accumulator blocks in the order the GEMM's wave left them (1 KB per load, the runs in order, so the
-// sum is the same every time), and the 16 x 256 result goes through the LDS to be stored in whole rows. 225 rows at d 2560, V 151,936 (26 runs of 10 tiles, 68 MB): 16 us.
+// sum is the same every time), and the 16 x 256 result goes through the LDS to be stored in whole rows. 225 rows at d
+// 2560, V 151,936 (26 runs of 10 tiles, 68 MB): 16 us.
 #include "gemm_nt.h"
 #include "octo_internal.h"
 

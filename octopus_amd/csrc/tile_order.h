@@ -45,7 +45,8 @@ constexpr bool tile_at(int group_m, int x, int k, int mtiles, int ntiles, int &m
     nt = (int)q;
     return true;
   }
-  const unsigned r = (unsigned)(mtiles - 8 * mfull), T = r * (unsigned)ntiles;  // the last r M-tiles, M fastest, cut in 8
+  // the last r M-tiles, M fastest, cut in 8
+  const unsigned r = (unsigned)(mtiles - 8 * mfull), T = r * (unsigned)ntiles;
   const unsigned L = (unsigned)x * T / 8 + (unsigned)(k - main);
   if (L >= (unsigned)(x + 1) * T / 8) return false;
   const unsigned q = L / r;
@@ -56,10 +57,11 @@ constexpr bool tile_at(int group_m, int x, int k, int mtiles, int ntiles, int &m
 
 // ---- split K (grad_h) ----------------------------------------------------------------------------------------
 //
-// grad_h = dz . W contracts over the vocabulary: few tiles (rows / 256 x d / 256), each long (V / 64 stages). With fewer
-// tiles than CUs the long tiles set the time: 225 scored rows at d 2560, V 151,936 are 10 tiles of 2,374 stages, 3.0 ms
-// on 10 CUs while grad_W's 5,940 tiles of 4 stages keep the others busy for 0.3. So a tile's K is cut into S runs of
-// whole stages, each a workgroup of its own that leaves an fp32 partial tile, which a small kernel sums in run order.
+// grad_h = dz . W contracts over the vocabulary: few tiles (rows / 256 x d / 256), each long (V / 64 stages). With
+// fewer tiles than CUs the long tiles set the time: 225 scored rows at d 2560, V 151,936 are 10 tiles of 2,374 stages,
+// 3.0 ms on 10 CUs while grad_W's 5,940 tiles of 4 stages keep the others busy for 0.3. So a tile's K is cut into S
+// runs of whole stages, each a workgroup of its own that leaves an fp32 partial tile, which a small kernel sums in run
+// order.
 //
 // k_splits: S for `tiles` tiles of nk stages. A run keeps at least kSplitStages stages (a partial tile costs about
 // kSplitCost stages of time to write and sum: 256 KB each way at 5 TB/s over 256 CUs, against 1.25 us a stage), and

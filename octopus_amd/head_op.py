@@ -445,16 +445,17 @@ def _sized(*tensors: Optional[Tensor]) -> bool:
     return all(type(n) is int for t in tensors if t is not None for n in t.shape)
 
 
-# ---- the head with logits kept between forward and backward (octo_head_fwd_logits) ------------------------------------
+# ---- the head with logits kept between forward and backward (octo_head_fwd_logits) -----------------------------------
 
 # Bytes of fp32 logits one call keeps, and all live ones on a device together; the rows past them are recomputed, as all
-# are without. In fp32, so that dz is rounded once, to bf16, and the gradients are the recomputing backward's to the bit.
+# are without. In fp32, so that dz is rounded once, to bf16, and the gradients are the recomputing backward's to the
+# bit.
 _KEEP_BYTES = 2 << 30
-# fused_head keeps logits from this many multiply-adds on (n d V), and for at most twice as many rows as the width (beyond,
-# fewer than half of the rows would be kept). us a forward and backward, kept and recomputed: 64 rows at d 1024, V 32,000
-# (2^31) 462 and 460, 256 rows 463 and 463, 1,024 rows 466 and 467; 32 rows at d 2560, V 151,936 (2^33.5) 623 and 787,
-# 3,000 rows, three quarters of them scored, 4,795 and 5,602; 8,192 rows at d 4096, V 128,256 (4,096 kept) 22,200 and
-# 24,250, 3,584 of them scored 9,196 and 11,149.
+# fused_head keeps logits from this many multiply-adds on (n d V), and for at most twice as many rows as the width
+# (beyond, fewer than half of the rows would be kept). us a forward and backward, kept and recomputed: 64 rows at d
+# 1024, V 32,000 (2^31) 462 and 460, 256 rows 463 and 463, 1,024 rows 466 and 467; 32 rows at d 2560, V 151,936 (2^33.5)
+# 623 and 787, 3,000 rows, three quarters of them scored, 4,795 and 5,602; 8,192 rows at d 4096, V 128,256 (4,096 kept)
+# 22,200 and 24,250, 3,584 of them scored 9,196 and 11,149.
 _STAGE_WORK = 1 << 33
 
 
@@ -470,8 +471,8 @@ def _kept_rows(n: int, d: int, V: int) -> int:
 
 class _Room:
     """A share of the _KEEP_BYTES that the kept logits of a device take together, given back when this object goes. A
-    caller that holds several losses before their backwards keeps one call's logits, or two smaller ones'; the other calls
-    recompute, to the same bits."""
+    caller that holds several losses before their backwards keeps one call's logits, or two smaller ones'; the other
+    calls recompute, to the same bits."""
 
     _lock = threading.RLock()  # a collection inside the lock may free another share
     _taken: dict = {}
@@ -493,7 +494,8 @@ def _keeps(rows: Tensor, weight: Tensor, idx: Optional[Tensor]) -> int:
     """The rows whose logits fused_head keeps, 0 where the backward recomputes them all."""
     if not torch.is_grad_enabled() or BWD_WORKSPACE_BYTES is not None or torch.compiler.is_compiling():
         return 0
-    # inside checkpoint or an offload's hooks the caller has said that little is to stay on the device until the backward
+    # inside checkpoint or an offload's hooks the caller has said that little is to stay on the device until the
+    # backward
     if torch._C._autograd._top_saved_tensors_default_hooks(False) is not None:
         return 0
     # a frozen weight has no gradient for the kept bytes to stand beside
@@ -600,13 +602,13 @@ def fused_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: float,
 
 # ---- the GRPO step with its weight gradient made in the backward (octo_head_step_later) ------------------------------
 
-# From this many weights on, or this many multiply-adds (n d V), and up to this many rows. Scaling a held weight gradient
-# costs a read and a write of it; leaving it to the backward costs a few launches, 12 us of host time where a call is so
-# short that the host sets the pace, and, in proportion to the rows, the tiles of grad_W that ran beside grad_h's in one
-# launch. us a forward and backward, held and left for later, bf16: d 2560, V 151,936 (2^28.5) 57 rows 861 and 569, 225
-# rows 999 and 741, 1,024 rows 2,235 and 2,019, 1,536 rows 3,106 and 2,865, 2,048 rows 3,991 and 3,784; d 2304, V 64,000
-# (2^27.1) 512 rows 562 and 472; d 1024, V 65,536 (2^26) 57 rows 319 and 334, 256 rows (2^34) 323 and 329, 768 rows
-# (2^35.6) 379 and 340; d 1024, V 32,768 (2^25) 57 rows 330 and 343, 1,024 rows (2^35) 322 and 334.
+# From this many weights on, or this many multiply-adds (n d V), and up to this many rows. Scaling a held weight
+# gradient costs a read and a write of it; leaving it to the backward costs a few launches, 12 us of host time where a
+# call is so short that the host sets the pace, and, in proportion to the rows, the tiles of grad_W that ran beside
+# grad_h's in one launch. us a forward and backward, held and left for later, bf16: d 2560, V 151,936 (2^28.5) 57 rows
+# 861 and 569, 225 rows 999 and 741, 1,024 rows 2,235 and 2,019, 1,536 rows 3,106 and 2,865, 2,048 rows 3,991 and 3,784;
+# d 2304, V 64,000 (2^27.1) 512 rows 562 and 472; d 1024, V 65,536 (2^26) 57 rows 319 and 334, 256 rows (2^34) 323 and
+# 329, 768 rows (2^35.6) 379 and 340; d 1024, V 32,768 (2^25) 57 rows 330 and 343, 1,024 rows (2^35) 322 and 334.
 _LATER_WEIGHTS = 1 << 27
 _LATER_WORK = 3 << 34
 _LATER_ROWS = 1536
@@ -614,7 +616,7 @@ _LATER_SHARE = 1  # what is kept takes at most this many times the bytes of the 
 
 
 def _later_bytes(rows: Tensor, weight: Tensor, idx: Optional[Tensor], need_rows: bool, need_weight: bool) -> int:
-    """The bytes of the buffer (dz and h^T) of a step whose weight gradient is left to the backward, 0 where it is not."""
+    """The bytes of the buffer (dz and h^T) of a step whose weight gradient is left to the backward, else 0."""
     if not need_weight or STEP_WORKSPACE_BYTES is not None or torch.compiler.is_compiling() or not rows.is_cuda:
         return 0
     if rows.dim() != 2 or weight.dim() != 2 or rows.dtype != weight.dtype:
@@ -751,7 +753,8 @@ def fused_grpo_head(rows: Tensor, weight: Tensor, labels: Tensor, temperature: f
     and weight (each when it requires grad and grad mode is on); loss.backward() then only scales them, or, for a short
     call, makes the weight's from the operands kept (head_step_later). The columns
     carry no gradient: for losses other than this objective, use fused_head. prox, old, adv, mask are per flat
-    token (row of `rows`), as grpo_loss takes them. The gradients or operands are held from this call to the backward."""
+    token (row of `rows`), as grpo_loss takes them. The gradients or operands are held from this call until the graph
+    goes."""
     if temperature <= 0:
         raise ValueError("temperature must be positive")
     grad_on = torch.is_grad_enabled()

@@ -60,6 +60,6 @@ def test_columns_close_to_zero(dtype):
     zl = torch.randn(n, V, generator=g, device=DEV).scatter_(1, y[:, None], torch.linspace(14, 18, n, device=DEV)[:, None]).to(dtype)
     want = zl.double().gather(1, y[:, None])[:, 0] - torch.logsumexp(zl.double(), 1)
     got = head_op.head_columns(zl, 1.0, y)[:, 0].double()
-    # the label's own logit among the sums: what is left is the sum's rounding, 1.05 in 24 merges (wave and workgroup) of
-    # at most 2^-24 each, and the label's thread, whose 125 terms are each rounded against 1
+    # the label's own logit among the sums: what is left is the sum's rounding, 1.05 in 24 merges (wave and workgroup)
+    # of at most 2^-24 each, and the label's thread, whose 125 terms are each rounded against 1
     assert (got - want).abs().max() <= (24 + math.sqrt(125)) * 2.0 ** -24

@@ -1,6 +1,6 @@
 """octohead::scaled, the fused step's backward: c x in fp32 rounded once, against the same arithmetic in torch, bit for
-bit, over vector lengths around the kernel's 16-byte chunks and its workgroups' 1,024; the in-place form, which walks the
-vector; and a retained graph's second backward, which finds the held gradients as the first did."""
+bit, over vector lengths around the kernel's 16-byte chunks and its workgroups' 1,024; the in-place form, which walks
+the vector; and a retained graph's second backward, which finds the held gradients as the first did."""
 
 import pytest
 import torch
@@ -20,8 +20,8 @@ def test_scaled_rounds_the_fp32_product_once(n, dtype):
         assert torch.equal(head_op.scaled(x, c), (x.float() * c).to(dtype))
 
 
-# the in-place form walks the vector with 2,048 workgroups of 256 threads and 4 loads in flight: lengths around one load of
-# every thread, around all four, and past them
+# the in-place form walks the vector with 2,048 workgroups of 256 threads and 4 loads in flight: lengths around one load
+# of every thread, around all four, and past them
 _WALK = 2048 * 256
 
 
@@ -40,7 +40,8 @@ def test_scale_add_in_place(chunks, over, dtype, per):
             want = c.double() * y.double()
             if rest is not None and skip is not off:
                 want += x.double()
-            # 64-bit sums rounded to fp32, and then to 16 bits: a sum next to a tie of the two roundings may fall either way
+            # 64-bit sums rounded to fp32, and then to 16 bits: a sum next to a tie of the two roundings may fall either
+            # way
             want = want.float()
             if dtype == torch.float32:
                 assert ((got - want).abs() <= want.abs() * 2.0 ** -23).all()
