@@ -7,9 +7,10 @@
 // columns 6.4e-7 off (relative) against 7.9e-7, the gradients 8e-7 against 3.2e-6. Time there: the logits and their
 // statistics 279 us with the fp32 instructions (120 TFLOP/s), 178 here (188 TFLOP/s in fp32 terms).
 // An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: its remainder is not
-// finite, and so is every sum it enters. A tile with such a sum is made again by v_mfma_f32_16x16x4_f32 from the
-// operands as they are (mainloop_plain), infinities and NaN where those products have them; to look for one costs 0.6%
-// of those logits' time. Below 2^-110 the third part loses bits.
+// finite, and so is every sum it enters. A wave that finds such a sum makes its part of the tile again by
+// v_mfma_f32_16x16x4_f32 from the operands as they are (mainloop_plain), infinities and NaN where those products have
+// them; to look for one takes no time that shows (those logits 178.6 us, 178.9 without). Below 2^-110 the third part
+// loses bits.
 //
 // One workgroup computes a 256 x 128 tile of C[m, n] = sum_k A[m, k] B[n, k] with 8 waves, two per SIMD, 2 x 4 of 128 x
 // 32 (AccX: the 16 x 16 block layout of the 16-bit kernels, 8 x 2 blocks). A stage is K = 32: 48 KB of fp32 go from
@@ -259,7 +260,7 @@ struct XPlain {
   }
 };
 
-// acc made again without the split, 4 K-values at a time from global memory. Rare and slow: it is not tuned.
+// This wave's acc made again without the split, 4 K-values at a time from global memory. Rare and slow: not tuned.
 template <bool TR>
 __device__ __forceinline__ void mainloop_plain(const XPlain &a, const XPlain &b, XAcc &acc) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wm = w >> 2, wn = w & 3;
@@ -283,22 +284,19 @@ __device__ __forceinline__ void mainloop_plain(const XPlain &a, const XPlain &b,
   }
 }
 
-// Whether an operand of the workgroup's tile had such a value (the same in every thread; a barrier): it leaves no
-// finite sum in its row or column of the tile, so one column of blocks, shared out among the waves of a row, and one
-// row of blocks tell.
-__device__ __forceinline__ bool xnonfinite(const XAcc &acc) {
-  const int wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
+// Whether an operand of this wave's part of the tile had such a value: it leaves no finite sum in its row or column, so
+// one row and one column of blocks tell.
+template <bool TR> __device__ __forceinline__ bool xnonfinite(const XAcc &acc) {
   float z = 0.f;
 #pragma unroll
   for (int i = 0; i < AccX::NI; ++i)
-    if (i >> 1 == wn)
 #pragma unroll
-      for (int v = 0; v < AccX::NV; ++v) z = __builtin_fmaf(acc[i][0][v], 0.f, z);  // 0 x inf and 0 x NaN are NaN
+    for (int v = 0; v < (TR ? 1 : AccX::NV); ++v) z = __builtin_fmaf(acc[i][0][v], 0.f, z);  // 0 x inf and 0 x NaN: NaN
 #pragma unroll
   for (int j = 0; j < AccX::NJ; ++j)
 #pragma unroll
-    for (int v = 0; v < AccX::NV; ++v) z = __builtin_fmaf(acc[0][j][v], 0.f, z);
-  return __syncthreads_or(z != 0.f) != 0;
+    for (int v = 0; v < (TR ? AccX::NV : 1); ++v) z = __builtin_fmaf(acc[0][j][v], 0.f, z);
+  return __any(z != 0.f);
 }
 
 // The tile's sums over K of A's rows from m0 on and B's from n0 on; a K-major operand (KM_A, KM_B) as XCols.
@@ -313,7 +311,7 @@ __device__ __forceinline__ void xtile(const Operand &A, const Operand &B, int64_
     b.init(B, n0, K);
     mainloop_x<TR>(a, b, stages, smem, acc);
   }
-  if (xnonfinite(acc)) mainloop_plain<TR>(XPlain(A, m0, K, KM == KM_A), XPlain(B, n0, K, KM == KM_B), acc);
+  if (xnonfinite<TR>(acc)) mainloop_plain<TR>(XPlain(A, m0, K, KM == KM_A), XPlain(B, n0, K, KM == KM_B), acc);
 }
 
 // Tiles of the 256 x 128 grid, shrunk by a device count that bounds M or N; the order is gemm_nt.h's.
