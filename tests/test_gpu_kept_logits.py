@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from octopus_amd import head_op
+from tests.test_gpu_poisoned import poisoned
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -104,3 +105,12 @@ def test_a_weight_changed_in_place(monkeypatch):
         out[:, 0].sum().backward()
         got.append((hd.grad, Wd.grad))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n,d,V,scored,rows", [(300, 512, 5003, 0.7, None), (900, 512, 2500, 0.9, 256),
+                                               (900, 512, 2500, 0.2, 256), (300, 136, 1000, 0.0, None)])
+def test_reads_only_what_it_wrote(n, d, V, scored, rows, monkeypatch):
+    want = _both(n, d, V, scored, 0.7, False, monkeypatch, rows=rows)[1]
+    with poisoned():
+        got = _both(n, d, V, scored, 0.7, False, monkeypatch, rows=rows)[0]
+    assert all(torch.equal(x, y) for x, y in zip(got, want))

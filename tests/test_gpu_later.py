@@ -5,6 +5,7 @@ import torch
 
 from octopus_amd import head_op
 from octopus_amd.rl.prefix_tree import TreeMeta
+from tests.test_gpu_poisoned import poisoned
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -116,3 +117,28 @@ def test_the_gradients_of_the_gradients(monkeypatch):
 
     a, b = _both(run, monkeypatch)
     assert abs(a - b) <= 2.0 ** -8 * abs(b)  # gradients rounded to bf16 once or twice
+
+
+@pytest.mark.parametrize("d,V,dtype", [(512, 5003, torch.bfloat16), (136, 1000, torch.float16),
+                                       (512, 2048, torch.bfloat16)])
+def test_reads_only_what_it_wrote(d, V, dtype, monkeypatch):
+    n = 300
+    g = torch.Generator(device=DEV).manual_seed(V)
+    W = (torch.randn(V, d, generator=g, device=DEV) * 0.05).to(dtype)
+    h = torch.randn(n, d, generator=g, device=DEV).to(dtype)
+    y = torch.randint(0, V, (n,), generator=g, device=DEV)
+    adv, mask = torch.randn(n, generator=g, device=DEV), (torch.rand(n, generator=g, device=DEV) < 0.7).float()
+    idx, count = head_op.compact_rows(mask.bool())
+
+    def run():
+        hd, Wd = h.clone().requires_grad_(True), W.clone().requires_grad_(True)
+        loss, out = head_op.fused_grpo_head(hd, Wd, y, 0.7, adv, mask, idx=idx, count=count, labels_via_idx=True,
+                                            scatter=True)
+        loss.backward()
+        return out, hd.grad, Wd.grad
+
+    want = _both(run, monkeypatch)[0]
+    with poisoned(), monkeypatch.context() as m:
+        m.setattr(head_op, "_LATER_WEIGHTS", 0)
+        got = run()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
