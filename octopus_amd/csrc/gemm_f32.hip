@@ -1,5 +1,7 @@
 // The fp32 GEMMs of the LM-head path on the bf16 matrix cores: each fp32 operand is the exact sum of three bf16 values
-// (its 24 significand bits, 8 at a time), and a product is the six partial products that reach fp32's last bit,
+// (its 24 significand bits, 8 at a time; the method of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", ARITH 2019), and a product is the six partial products that
+// reach fp32's last bit,
 //     a b = a0 b0 + a0 b1 + a1 b0 + a1 b1 + a0 b2 + a2 b0   (+ a1 b2 + a2 b1 + a2 b2, below 2^-23 |a b|),
 // summed by v_mfma_f32_16x16x32_bf16 in fp32. The matrix cores' fp32 rate is 1/16 of their bf16 rate, so six bf16
 // products are 2.6 times as fast. What is left out and one rounding per 32 products (against one per 2 with
