@@ -1,5 +1,7 @@
 """fused_head with logits kept for the backward (octo_head_fwd_logits, octo_head_bwd_logits): to the bit what the
 recomputing backward gives, over what both take."""
+import threading
+
 import pytest
 import torch
 
@@ -114,3 +116,63 @@ def test_reads_only_what_it_wrote(n, d, V, scored, rows, monkeypatch):
     with poisoned():
         got = _both(n, d, V, scored, 0.7, False, monkeypatch, rows=rows)[0]
     assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
+def _inputs(seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    W = (torch.randn(5003, 512, generator=g, device=DEV) * 0.05).bfloat16().requires_grad_(True)
+    h = torch.randn(300, 512, generator=g, device=DEV).bfloat16().requires_grad_(True)
+    y = torch.randint(0, 5003, (300,), generator=g, device=DEV)
+    gout = torch.randn(300, 2, generator=g, device=DEV)
+    return h, W, y, gout
+
+
+def _step(h, W, y, gout):
+    return torch.autograd.grad(head_op.fused_head(h, W, y, 0.7), (h, W), gout)
+
+
+def test_captured(monkeypatch):
+    """Forward and backward in one graph, replayed on new values between the program's own calls."""
+    monkeypatch.setattr(head_op, "_STAGE_WORK", 0)
+    static = _inputs(0)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _step(*static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = _step(*static)
+    for seed in (1, 2, 3):
+        new = _inputs(seed)
+        with torch.no_grad():
+            for a, b in zip(static, new):
+                a.copy_(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, _step(*new)))
+
+
+def test_threads_and_streams(monkeypatch):
+    """Threads with a stream of their own, more of them than the bound on live logits serves."""
+    monkeypatch.setattr(head_op, "_STAGE_WORK", 0)
+    monkeypatch.setattr(head_op, "_KEEP_BYTES", 2 * 512 * 5120 * 4)
+    inputs = [_inputs(k) for k in range(4)]
+    want = [_step(*x) for x in inputs]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                got = _step(*inputs[k])
+                torch.cuda.current_stream().synchronize()
+                if not all(torch.equal(a, b) for a, b in zip(got, want[k])):
+                    wrong.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong and head_op._Room._taken[inputs[0][0].device] == 0

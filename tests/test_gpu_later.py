@@ -142,3 +142,40 @@ def test_reads_only_what_it_wrote(d, V, dtype, monkeypatch):
         m.setattr(head_op, "_LATER_WEIGHTS", 0)
         got = run()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_captured(monkeypatch):
+    """The step and its backward in one graph, replayed on new values between the program's own calls."""
+    monkeypatch.setattr(head_op, "_LATER_WEIGHTS", 0)
+    monkeypatch.setattr(head_op, "_LATER_SHARE", 1 << 20)
+
+    def inputs(seed):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        W = (torch.randn(5003, 512, generator=g, device=DEV) * 0.05).bfloat16().requires_grad_(True)
+        h = torch.randn(300, 512, generator=g, device=DEV).bfloat16().requires_grad_(True)
+        y = torch.randint(0, 5003, (300,), generator=g, device=DEV)
+        return h, W, y, torch.randn(300, generator=g, device=DEV), torch.randn((), generator=g, device=DEV)
+
+    mask = torch.ones(300, device=DEV)
+
+    def step(h, W, y, adv, c):
+        loss, out = head_op.fused_grpo_head(h, W, y, 0.7, adv, mask)
+        return (out, *torch.autograd.grad(loss, (h, W), c))
+
+    static = inputs(0)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(*static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(*static)
+    for seed in (1, 2, 3):
+        new = inputs(seed)
+        with torch.no_grad():
+            for a, b in zip(static, new):
+                a.copy_(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, step(*new)))
