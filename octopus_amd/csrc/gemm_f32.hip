@@ -8,17 +8,16 @@
 // v_mfma_f32_32x32x2_f32) leave the sums no less exact, measured against 64 bits on [512, 32,000] logits of d 1024: the
 // columns 6.4e-7 off (relative) against 7.9e-7, the gradients 8e-7 against 3.2e-6. Time there: the logits and their
 // statistics 279 us with the fp32 instructions (120 TFLOP/s), 178 here (188 TFLOP/s in fp32 terms).
-// An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: its remainder is not
-// finite, and so is every sum it enters. A wave that finds such a sum makes its part of the tile again by
-// v_mfma_f32_16x16x4_f32 from the operands as they are (mainloop_plain), infinities and NaN where those products have
-// them; to look for one takes no time that shows (those logits 178.6 us, 178.9 without). Below 2^-110 the third part
-// loses bits.
+// An infinite operand, or one that bf16 rounds to infinity (from 3.39e38 on), has no such parts: no sum that it enters
+// is finite. A wave that finds such a sum makes its part of the tile again by v_mfma_f32_16x16x4_f32 from the operands
+// as they are (mainloop_plain), infinities and NaN where those products have them; to look for one takes no time that
+// shows (those logits 182.2 us, 183.0 without). Below 2^-110 the third part loses bits.
 //
 // One workgroup computes a 256 x 128 tile of C[m, n] = sum_k A[m, k] B[n, k] with 8 waves, two per SIMD, 2 x 4 of 128 x
 // 32 (AccX: the 16 x 16 block layout of the 16-bit kernels, 8 x 2 blocks). A stage is K = 32: 48 KB of fp32 go from
 // global memory to registers one stage ahead, are split there, and land in the LDS as three bf16 planes per operand
 // (72 KB a stage, two stages). Bound by the matrix cores: 96 MFMAs per wave and stage (1,536 cycles) against 24 values
-// per thread to split (5.5 instructions each). One wave of each SIMD splits the next
+// per thread to split (5.5 instructions each, and two for infinities). One wave of each SIMD splits the next
 // stage before its MFMAs and the other after them, so that one's vector instructions run beside the other's MFMAs. A
 // 256 x 256 tile would need 96 KB a stage: no room for the second.
 //
@@ -54,7 +53,9 @@ __device__ __forceinline__ int xslot(int row, int c) { return row * XROWB + ((c 
 // x = p0 + p1 + p2, 8 values at a time: p0 = x to the nearest bf16, p1 the (exact) remainder to the nearest, p2 what is
 // left, at most 7 bits, a bf16 as it stands. To the nearest and not towards zero, so that the remainders, and with them
 // the partial products left out, have either sign: cut off, they all lean one way, 2^-23 of every sum, and the logprobs
-// of [512, 32,000] logits were a quarter further from 64 bits than the fp32 instructions' (1.1e-6 against 8.8e-7).
+// of [512, 32,000] logits were a quarter further from 64 bits than the fp32 instructions' (1.1e-6 against 8.8e-7). A
+// value whose p0 is not finite keeps p0 alone: nothing needs it to (mainloop_plain), but the loop is 1-2% slower
+// without the select (those logits 182 and 186 us).
 __device__ __forceinline__ void split8(const float (&x)[8], i32x4 (&p)[3]) {
 #pragma unroll
   for (int h = 0; h < 4; ++h) {
@@ -69,7 +70,10 @@ __device__ __forceinline__ void split8(const float (&x)[8], i32x4 (&p)[3]) {
       if (k == 2) break;
       const float f[2] = {__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
 #pragma unroll
-      for (int e = 0; e < 2; ++e) r[e] -= f[e];
+      for (int e = 0; e < 2; ++e) {
+        r[e] -= f[e];
+        if (k == 0) r[e] = __builtin_fabsf(f[e]) < INFINITY ? r[e] : 0.f;
+      }
     }
   }
 }
