@@ -1117,6 +1117,12 @@ static int head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, con
       }
       if (rc) return rc;
 
+      const Operand A3 = plain_operand(dza, L.Vc * esz, L.Vc, nullptr, 0);  // dz token-major, read K-major
+      const Operand B3 = plain_operand(ht, L.P * esz, d, nullptr, 0);
+      // With logits kept and one chunk, both gradients in one launch: grad_W's short tiles fill the CUs that grad_h's
+      // long ones leave (3,584 rows at d 4096, V 128,256: 5,516 against 5,712 us). Chunks have tiles of about one
+      // length, and take longer so (24,576 rows at d 2560 in six chunks 27.7 against 27.4 ms).
+      const bool both = kept.rows && need_gh && need_gw && L.chunks == 1;
       if (need_gh) {  // grad_h[rows] (+)= dz . W[v0 .. v0 + vc)   (K = vc, or vc_pad through the staged W^T)
         if (!wk) {  // W^T [d, Vc] of the chunk's rows in the staged type (fp8: from the widened rows), zero past vc
           rc = launch_transpose(Aw.base, Aw.ld / esz, cm.dt, nullptr, nullptr, nullptr, 0, vc, L.Vc, d, wt, L.Vc,
@@ -1146,16 +1152,18 @@ static int head_bwd(const void *h, int64_t h_rows, int64_t ldh, int h_dtype, con
           o.split_cap = (int)L.split_items;
           o.split_alone = 1;
         }
-        {
+        if (both) {
+          const StoreArgs ow = grad_w_store(d, r0, rows, p, L.passes, L.gacc_on, gacc, grad_w, gw_dtype, flags, count);
+          TimedLaunch t("gemm_grads", st);
+          rc = launch_gemm_grads(cm.dt, A2, B2, s2, o, wk, A3, B3, shape(vc, d, rows, kGroupM, 3, count, r0), ow, st);
+        } else {
           TimedLaunch t("gemm_store_grad_h", st);
           rc = launch_gemm_store(cm.dt, A2, B2, s2, o, st, wk ? KM_B : KM_NONE);
         }
         if (!rc) rc = launch_split_sum(s2, o, esz == 4, st);
         if (rc) return rc;
       }
-      if (need_gw) {  // grad_W[v0 .. v0 + vc) (+)= dz^T . h   (K = this pass's rows)
-        const Operand A3 = plain_operand(dza, L.Vc * esz, L.Vc, nullptr, 0);  // dz token-major, read K-major
-        const Operand B3 = plain_operand(ht, L.P * esz, d, nullptr, 0);
+      if (need_gw && !both) {  // grad_W[v0 .. v0 + vc) (+)= dz^T . h   (K = this pass's rows)
         rc = grad_w_pass(cm.dt, A3, KM_A, B3, vc, d, r0, rows, p, L.passes, L.gacc_on, gacc + v0 * d,
                          (char *)grad_w + v0 * d * elem_bytes(gw_dtype), gw_dtype, flags, count, st);
         if (rc) return rc;

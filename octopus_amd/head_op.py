@@ -455,7 +455,7 @@ _KEEP_BYTES = 2 << 30
 # (beyond, fewer than half of the rows would be kept). us a forward and backward, kept and recomputed: 64 rows at d
 # 1024, V 32,000 (2^31) 462 and 460, 256 rows 463 and 463, 1,024 rows 466 and 467; 32 rows at d 2560, V 151,936 (2^33.5)
 # 623 and 787, 3,000 rows, three quarters of them scored, 4,795 and 5,602; 8,192 rows at d 4096, V 128,256 (4,096 kept)
-# 22,200 and 24,250, 3,584 of them scored 9,196 and 11,149.
+# 22,200 and 24,250, 3,584 of them scored 9,051 and 11,133.
 _STAGE_WORK = 1 << 33
 
 
