@@ -5,8 +5,8 @@ import threading
 import pytest
 import torch
 
-from octopus_amd import head_op
-from tests.test_gpu_poisoned import poisoned
+from octopus_amd import _lib, head_op
+from tests.test_gpu_poisoned import _bwd_ws, poisoned
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -67,6 +67,15 @@ def test_as_recomputed(n, d, V, scored, T, cap, bad, monkeypatch):
 @pytest.mark.parametrize("cap", [False, True])
 def test_some_rows_kept(n, scored, rows, ws, cap, monkeypatch):
     a, b = _both(n, 512, 2500, scored, 0.7, cap, monkeypatch, rows=rows, ws=ws)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("scored", [1.0, 0.6, 0.1])
+def test_several_passes_of_one_chunk(scored, monkeypatch):
+    """Both gradients in one launch per pass, grad_W's sum over the passes in fp32, the last one the count decides; the
+    kept rows end within the second pass."""
+    ws = _bwd_ws(4000, 2048, 192, _lib.BF16, 0, lambda plan: plan[1] == 2 and plan[3] == 1)
+    a, b = _both(4000, 2048, 192, scored, 0.7, False, monkeypatch, rows=2560, ws=ws)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
 
 
